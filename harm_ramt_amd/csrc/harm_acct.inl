@@ -174,12 +174,12 @@ __global__ void k_acct_srcterm(KParams P, AcctRegions R, const double* __restric
   if (i >= P.n1 || j >= P.n2) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR], dU[NPR], ft[NPR], fd[NPR];
   load8(pb, z, pr);
-  source_conn_sym(P, pr, g, gConn + z, dU, (size_t)(P.n1 + 2 * NG) * P.N2M);
+  source_conn_at(P, pr, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, dU);
   const double Dt = ds->dt;
 #pragma unroll
   for (int k = 0; k < NPR; k++) ft[k] = Dt * R.dVF * (0.0 + dU[k]);  // dUcomp[GEOMSOURCE] = 0 e + e dUconn
@@ -256,7 +256,7 @@ __global__ void k_acct_faceterm(KParams P, AcctRegions R, const int* __restrict_
   {
     double f[NPR], ft[NPR], fd[NPR];
     final_flux(P, x1 ? F1 : F2, q1, q2, gC, fluxdir, i, j, f);
-    const double fg = gF[((x1 ? 0 : nz) + z) * GF + 15];
+    const double fg = face_gdet(P, gF + (x1 ? 0 : nz * GF), z);
 #pragma unroll
     for (int k = 0; k < NPR; k++) ft[k] = f[k] * surface;
     evolve_to_diag(P, fg, ft, fd);
@@ -264,7 +264,7 @@ __global__ void k_acct_faceterm(KParams P, AcctRegions R, const int* __restrict_
     for (int k = 0; k < NPR; k++) o[k] = fd[k];
   }
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR];
@@ -360,7 +360,7 @@ __global__ void k_acct_frterm(KParams P, AcctRegions R, const double* __restrict
   const double surface = P.dx2 * R.dx3;
 #pragma unroll
   for (int k = 0; k < NPR; k++) ft[k] = f[k] * surface;
-  evolve_to_diag(P, gF[(size_t)zidx(P, i, j) * GF + 15], ft, fd);
+  evolve_to_diag(P, face_gdet(P, gF, zidx(P, i, j)), ft, fd);
   store8(out, i * P.n2 + j, fd);
 }
 
@@ -389,8 +389,8 @@ __device__ double corner_divb(const KParams& P, const double* __restrict__ p, co
   if ((j != 0) && (j != P.n2)) {
     const double dx1 = P.dx1, dx2 = P.dx2;
     const int z00 = zidx(P, i, j), z0m = zidx(P, i, j - 1), zm0 = zidx(P, i - 1, j), zmm = zidx(P, i - 1, j - 1);
-    const double g00 = gC[(size_t)z00 * GCN + GC_GDET], g0m = gC[(size_t)z0m * GCN + GC_GDET];
-    const double gm0 = gC[(size_t)zm0 * GCN + GC_GDET], gmm = gC[(size_t)zmm * GCN + GC_GDET];
+    const double g00 = geo_entry(P, gC, GC_GDET, z00), g0m = geo_entry(P, gC, GC_GDET, z0m);
+    const double gm0 = geo_entry(P, gC, GC_GDET, zm0), gmm = geo_entry(P, gC, GC_GDET, zmm);
     const double b100 = p[(size_t)z00 * 8 + B1], b10m = p[(size_t)z0m * 8 + B1];
     const double b1m0 = p[(size_t)zm0 * 8 + B1], b1mm = p[(size_t)zmm * 8 + B1];
     const double b200 = p[(size_t)z00 * 8 + B2], b20m = p[(size_t)z0m * 8 + B2];
@@ -400,7 +400,7 @@ __device__ double corner_divb(const KParams& P, const double* __restrict__ p, co
                         0.5 * (b200 * g00 + b2m0 * gm0 - b20m * g0m - b2mm * gmm) / dx2);
     const double sum = b100 * g00 + b10m * g0m + b1m0 * gm0 + b1mm * gmm + b200 * g00 + b2m0 * gm0 + b20m * g0m +
                        b2mm * gmm;
-    divb = fabs(num / (gC[(size_t)z00 * GCN + GC_GDETC] * 0.125 * fabs(fabs(sum) + 1.e-20)));
+    divb = fabs(num / (geo_entry(P, gC, GC_GDETC, z00) * 0.125 * fabs(fabs(sum) + 1.e-20)));
   }
   return divb;
 }
@@ -457,7 +457,7 @@ __global__ void k_cons_term(KParams P, AcctRegions R, const double* __restrict__
   if (i >= P.n1 || j >= P.n2) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR], U[NPR], ft[NPR];
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256) void k_acct_faceg(KParams P, const double* __r
   p[1][kb] = bavg;
   const size_t nz = (size_t)(P.n1 + 2 * NG) * P.N2M;
   GeoU g;
-  load_geo_face(gF + (dir == 2 ? nz * GF : 0), zidx(P, i, j), g);
+  load_geo_face(P, gF + (dir == 2 ? nz * GF : 0), zidx(P, i, j), g);
   const int slot = (dir == 1) ? acct_base(P.n1, P.n2, 0) + (i * (P.n2 + 2) + (j + 1)) * 2
                               : acct_base(P.n1, P.n2, 1) + ((i + 1) * (P.n2 + 1) + j) * 2;
   for (int side = 0; side < 2; side++) {
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(256) void k_acct_zoneg(KParams P, const double* __r
   if (i >= P.n1 || j >= P.n2) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double p0[NPR], p1[NPR], p2[NPR];
@@ -680,7 +680,7 @@ __global__ __launch_bounds__(256) void k_acct_fixg(KParams P, const double* __re
   if (f >= 0) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pavg[NPR], pfin[NPR], pr0[NPR];

@@ -108,7 +108,7 @@ __global__ void k_adj_seed_bsq(KParams P, const double* p, const double* gC, dou
   double l[NPR] = {0., 0., 0., 0., 0., 0., 0., 0.};
   if (i >= 0 && i < P.n1 && j >= 0 && j < P.n2) {
     double gc[36];
-    load_cent(gC, z, gc);
+    load_cent(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     double pr[NPR];
@@ -121,7 +121,7 @@ __global__ void k_adj_seed_bsq(KParams P, const double* p, const double* gC, dou
     for (int jj = 0; jj < P.n2; jj++) {
       const int zz = zidx(P, i, jj);
       double gc[36];
-      load_cent(gC, zz, gc);
+      load_cent(P, gC, zz, gc);
       GeoU g;
       geo_from_cent(gc, g);
       double pr[NPR];
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void k_adj_zone(KParams P0, AdjRK R, const dou
   R.dt = dts[ctr[0]];
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double p[NPR], lpf[NPR];
@@ -216,10 +216,10 @@ __device__ __forceinline__ void adj_face(const KParams& P, const double* __restr
     Fob[k] = (DIR == 1) ? (adj_ld(P, ldU, i, j, k) - adj_ld(P, ldU, i - 1, j, k)) * idx
                         : (adj_ld(P, ldU, i, j, k) - adj_ld(P, ldU, i, j - 1, k)) * idx;
   GeoU g;
-  load_geo_face(gF, z0, g);
+  load_geo_face(P, gF, z0, g);
   if (P.fluxb == HARM_FLUXCTTOTH) {
     auto le = [&](int a, int b) {
-      return (a >= 0 && a <= P.n1 && b >= 0 && b <= P.n2) ? gC[(size_t)zidx(P, a, b) * GCN + GC_GDETC] * lemf[zidx(P, a, b)]
+      return (a >= 0 && a <= P.n1 && b >= 0 && b <= P.n2) ? geo_entry(P, gC, GC_GDETC, zidx(P, a, b)) * lemf[zidx(P, a, b)]
                                                            : 0.;
     };
     if (DIR == 1) {
@@ -336,16 +336,13 @@ __global__ __launch_bounds__(256) void k_adj_gather(KParams P0, const double* co
   }
   if (i >= 0 && i < P.n1 && j >= 0 && j < P.n2) {
     double gc[36];
-    load_cent(gC, z, gc);
+    load_cent(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     double pr[NPR], ldu[NPR];
     load8(pb, z, pr);
     load8(ldU, z, ldu);
-    {
-      const size_t cs = (size_t)(P.n1 + 2 * NG) * P.N2M;
-      source_rev_at(P, pr, g, [&](int e) { return gConn[(size_t)conn_sym(e) * cs + z]; }, ldu, l);
-    }
+    source_rev_at(P, pr, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, ldu, l);
   }
   store8(lp, z, l);
 }
@@ -361,7 +358,7 @@ __global__ __launch_bounds__(256) void k_adj_ui(KParams P, const double* const* 
   const double* __restrict__ pn = slot[0];
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR], lui[NPR], l[NPR];

@@ -27,7 +27,7 @@ constexpr double NUMEPSILON = 2.2204460492503131e-16;
 
 // kernel-side parameter block (by value in kernel arguments)
 struct KParams {
-  int n1, n2, N2M;
+  int n1, n2, N2M, nz;  // nz = (n1 + 6) N2M zones, ghosts included
   int eomtype, lim, fluxmethod, fluxb;
   int bc[4];
   int fixupflux, poledeath, checksolution, eno;
@@ -314,12 +314,6 @@ HARM_HD constexpr int conn_sym(int e) {
   const int k = e >> 4, l = (e >> 2) & 3, j = e & 3;
   const int a = (l < j) ? l : j, b = (l < j) ? j : l;
   return k * 10 + a * 4 - (a * (a - 1)) / 2 + (b - a);
-}
-
-// source_conn from the symmetric component-major table (cs = the number of zones)
-template <class T>
-HARM_HD void source_conn_sym(const KParams& P, const T* pr, const GeoT<T>& g, const T* cn, T* dU, size_t cs) {
-  source_conn_at(P, pr, g, [&](int e) { return cn[(size_t)conn_sym(e) * cs]; }, dU);
 }
 
 // ---------------- reconstruction (interp.c) ----------------

@@ -28,7 +28,7 @@ __global__ void k_cur_pre(KParams P, const double* __restrict__ p, const double*
   if (ii >= P.n1 + 2 * NG || jj >= P.N2M) return;
   const int z = ii * P.N2M + jj;
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR];
@@ -74,7 +74,7 @@ __global__ void k_cur_calc(KParams P, const double* __restrict__ cf, const doubl
   const bool full = st[0] >= 2.0;
   const double dtl = st[1], dtr = ds->dt_step;
   const double idx1 = 1.0 / (2.0 * P.dx1), idx2 = 1.0 / (2.0 * P.dx2);
-  auto GD = [&](int a, int b) { return gC[(size_t)zidx(P, a, b) * GCN + GC_GDET]; };
+  auto GD = [&](int a, int b) { return geo_entry(P, gC, GC_GDET, zidx(P, a, b)); };
   auto CF = [&](int a, int b, int s, int m) { return cf[(size_t)zidx(P, a, b) * 15 + s * 3 + m]; };
   const double gt = GD(i, j), gr = GD(i, j), grp1 = GD(i + 1, j), ghp1 = GD(i, j + 1), grm1 = GD(i - 1, j),
                ghm1 = GD(i, j - 1);
@@ -135,7 +135,7 @@ __global__ void k_dump(KParams P, const double* __restrict__ p, const double* __
   if (i >= P.n1 || j >= P.n2) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR];

@@ -19,11 +19,12 @@
 //
 // Device layout (HBM):
 //   primitive-shaped arrays: the reference's AoS p[N1M][N2M][8] (64 B/zone);
-//   gF[2][nz][16]  FACE1/FACE2: gcov upper 10, gcon^{00..03}, gcon^{dd}, gdet
-//   gC[nz][30]     CENT: gcov upper 10 (gcov is symmetric to the bit), gcon 16
+//   gF[2][16][nz]  FACE1/FACE2: gcov upper 10, gcon^{00..03}, gcon^{dd}, gdet
+//   gC[30][nz]     CENT: gcov upper 10 (gcov is symmetric to the bit), gcon 16
 //                  (whose row 0 can hold -0 where its column holds +0), gdet,
 //                  floor rho, floor u, gdet(CORN)
-//   gConn[40][nz]  CENT connection Gamma^k_{lj}, l <= j (conn_sym), component-major
+//   gConn[40][nz]  CENT connection Gamma^k_{lj}, l <= j (conn_sym)
+//   (component-major: see geo_entry)
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 #include <string.h>
@@ -146,12 +147,26 @@ __device__ __forceinline__ void store8(double* __restrict__ a, int z, const doub
   for (int m = 0; m < 4; m++) a2[m] = make_double2(v[2 * m], v[2 * m + 1]);
 }
 
-__device__ __forceinline__ void load_geo_face(const double* __restrict__ gF, int z, GeoU& g) {
-  const double2* a = reinterpret_cast<const double2*>(gF + (size_t)z * GF);
-  double2 t0 = a[0], t1 = a[1], t2 = a[2], t3 = a[3], t4 = a[4], t5 = a[5], t6 = a[6], t7 = a[7];
-  g.g00 = t0.x; g.g01 = t0.y; g.g02 = t1.x; g.g03 = t1.y; g.g11 = t2.x; g.g12 = t2.y;
-  g.g13 = t3.x; g.g22 = t3.y; g.g23 = t4.x; g.g33 = t4.y;
-  g.n00 = t5.x; g.n01 = t5.y; g.n02 = t6.x; g.n03 = t6.y; g.ndd = t7.x; g.gdet = t7.y;
+// Entry m of zone z in a component-major table t[m][nz].  The geometry is kept
+// so because a wavefront's lanes are neighbouring zones: an entry is then 512
+// adjacent bytes (4-5 cache lines), where records of 128 and 240 bytes a zone
+// put every lane of every load on a line of its own.  The byte offset is 32
+// bits (nz <= 2^28, checked at harm_create), so a load is a scalar base plus
+// one shared lane offset.
+__device__ __forceinline__ double geo_entry(const KParams& P, const double* __restrict__ t, int m, int z) {
+  const char* b = reinterpret_cast<const char*>(t + (size_t)m * (unsigned)P.nz);
+  return *reinterpret_cast<const double*>(b + (unsigned)z * 8u);
+}
+
+// entries GF of the face records: gcov upper 10, gcon^{00..03}, gcon^{dd}, gdet
+__device__ __forceinline__ double face_gdet(const KParams& P, const double* __restrict__ gF, int z) {
+  return geo_entry(P, gF, 15, z);
+}
+__device__ __forceinline__ void load_geo_face(const KParams& P, const double* __restrict__ gF, int z, GeoU& g) {
+  auto a = [&](int m) { return geo_entry(P, gF, m, z); };
+  g.g00 = a(0); g.g01 = a(1); g.g02 = a(2); g.g03 = a(3); g.g11 = a(4); g.g12 = a(5);
+  g.g13 = a(6); g.g22 = a(7); g.g23 = a(8); g.g33 = a(9);
+  g.n00 = a(10); g.n01 = a(11); g.n02 = a(12); g.n03 = a(13); g.ndd = a(14); g.gdet = a(15);
 }
 
 // upper-triangle view of a full CENT record
@@ -224,7 +239,7 @@ __device__ __forceinline__ void flux_face(const KParams& P, const double* __rest
         p[k] = side ? (s[2][k] - 0.5 * dq) : (s[2][k] + 0.5 * dq);
       }
     }
-    load_geo_face(gF, z0, g);
+    load_geo_face(P, gF, z0, g);
   } else {
 #pragma unroll
     for (int k = 0; k < NPR; k++) p[k] = 0.0;
@@ -292,12 +307,12 @@ __device__ __forceinline__ void flux_face(const KParams& P, const double* __rest
         if (j == 0 && P.bc[HARM_X2DN] == HARM_POLARAXIS) {
           int zg = zidx(P, i, -1);
           F[(size_t)zg * 8 + B2] = -Fh[B2 - 4];
-          q[zg] = (-Fh[B2 - 4]) / gF[(size_t)zg * GF + 15];
+          q[zg] = (-Fh[B2 - 4]) / face_gdet(P, gF, zg);
         }
         if (j == P.n2 - 1 && P.bc[HARM_X2UP] == HARM_POLARAXIS) {
           int zg = zidx(P, i, P.n2);
           F[(size_t)zg * 8 + B2] = -Fh[B2 - 4];
-          q[zg] = (-Fh[B2 - 4]) / gF[(size_t)zg * GF + 15];
+          q[zg] = (-Fh[B2 - 4]) / face_gdet(P, gF, zg);
         }
         skip_b2 = (j == -1 && P.bc[HARM_X2DN] == HARM_POLARAXIS) || (j == P.n2 && P.bc[HARM_X2UP] == HARM_POLARAXIS);
       }
@@ -418,7 +433,7 @@ __device__ __forceinline__ void face_finish(const KParams& P, double* p_l, doubl
                                             double& dtij, int& fail) {
   const int z0 = zidx(P, i, j);
   GeoU g;
-  load_geo_face(gF, z0, g);
+  load_geo_face(P, gF, z0, g);
   double Fo[NPR];
   face_flux<DIR>(P, p_l, p_r, g, Fo, dtij, fail);
   bool skip_b2 = false;
@@ -430,12 +445,12 @@ __device__ __forceinline__ void face_finish(const KParams& P, double* p_l, doubl
         if (j == 0 && P.bc[HARM_X2DN] == HARM_POLARAXIS) {
           int zg = zidx(P, i, -1);
           F[(size_t)zg * 8 + B2] = -Fo[B2];
-          q[zg] = (-Fo[B2]) / gF[(size_t)zg * GF + 15];
+          q[zg] = (-Fo[B2]) / face_gdet(P, gF, zg);
         }
         if (j == P.n2 - 1 && P.bc[HARM_X2UP] == HARM_POLARAXIS) {
           int zg = zidx(P, i, P.n2);
           F[(size_t)zg * 8 + B2] = -Fo[B2];
-          q[zg] = (-Fo[B2]) / gF[(size_t)zg * GF + 15];
+          q[zg] = (-Fo[B2]) / face_gdet(P, gF, zg);
         }
         skip_b2 = (j == -1 && P.bc[HARM_X2DN] == HARM_POLARAXIS) || (j == P.n2 && P.bc[HARM_X2UP] == HARM_POLARAXIS);
       }
@@ -613,7 +628,7 @@ __global__ __launch_bounds__(64 * FSH_ROWS) void k_flux_shared(KParams P, const 
 __device__ __forceinline__ double emf_at(const KParams& P, const double* __restrict__ q1,
                                          const double* __restrict__ q2, const double* __restrict__ gC, int i, int j) {
   const int z = zidx(P, i, j);
-  return 0.25 * (gC[(size_t)z * GCN + GC_GDETC]) *
+  return 0.25 * (geo_entry(P, gC, GC_GDETC, z)) *
          (q1[z] + q1[zidx(P, i, j - 1)] - q2[z] - q2[zidx(P, i - 1, j)]);
 }
 
@@ -661,7 +676,7 @@ __global__ void k_fixflux(KParams P, double* __restrict__ F1, double* __restrict
     const int zs = zidx(P, i, j == -1 ? 0 : P.n2 - 1);
     const double v = -F1[(size_t)zs * 8 + B2];
     F1[(size_t)z * 8 + B2] = v;
-    q1[z] = v / gF[(size_t)z * GF + 15];
+    q1[z] = v / face_gdet(P, gF, z);
   }
   // F2 at the polar faces (i in [-1,N1)) and the equator (i in [0,N1)):
   // every component but U2 zeroed
@@ -673,7 +688,7 @@ __global__ void k_fixflux(KParams P, double* __restrict__ F1, double* __restrict
 #pragma unroll
     for (int k = 0; k < NPR; k++)
       if (k != U2) f[k] = 0.;
-    q2[z] = f[B1] / gF[(nz + z) * GF + 15];
+    q2[z] = f[B1] / face_gdet(P, gF + nz * GF, z);
   }
   // no mass flux into the grid through an outflow x1 face, j in [-1,N2)
   if (j < P.n2) {
@@ -693,8 +708,8 @@ __global__ void k_qfromF(KParams P, const double* __restrict__ F1, const double*
   if (i > P.n1 || j > P.n2) return;
   const size_t nz = (size_t)(P.n1 + 2 * NG) * P.N2M;
   const int z = zidx(P, i, j);
-  if (i >= 0) q1[z] = F1[(size_t)z * 8 + B2] / gF[(size_t)z * GF + 15];
-  if (j >= 0) q2[z] = F2[(size_t)z * 8 + B1] / gF[(nz + z) * GF + 15];
+  if (i >= 0) q1[z] = F1[(size_t)z * 8 + B2] / face_gdet(P, gF, z);
+  if (j >= 0) q2[z] = F2[(size_t)z * 8 + B1] / face_gdet(P, gF + nz * GF, z);
 }
 
 struct RKCoef {
@@ -939,15 +954,10 @@ __device__ __forceinline__ void cent_expand(const R& r, T* gc) {
 }
 
 // full CENT geometry record of zone z
-__device__ __forceinline__ void load_cent(const double* __restrict__ gC, int z, double* gc) {
-  const double2* a = reinterpret_cast<const double2*>(gC + (size_t)z * GCN);
+__device__ __forceinline__ void load_cent(const KParams& P, const double* __restrict__ gC, int z, double* gc) {
   double v[GCN];
 #pragma unroll
-  for (int m = 0; m < GCN / 2; m++) {
-    const double2 t = a[m];
-    v[2 * m] = t.x;
-    v[2 * m + 1] = t.y;
-  }
+  for (int m = 0; m < GCN; m++) v[m] = geo_entry(P, gC, m, z);
   cent_expand(
       [&](int m) { return v[m]; }, gc);
 }
@@ -1159,7 +1169,7 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
     const int z = zidx(P, i, j);
     const double dt = ds->dt;
     double gc[36];
-    load_cent(gC, z, gc);
+    load_cent(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     double pin[NPR], pbz[NPR];
@@ -1175,7 +1185,7 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
     }
     // source(pb): T^j_k Gamma^k_{lj} contraction (phys.c:475-619)
     double dUg[NPR];
-    source_conn_sym(P, pbz, g, gConn + z, dUg, (size_t)(P.n1 + 2 * NG) * P.N2M);
+    source_conn_at(P, pbz, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, dUg);
     double d1[NPR], d2[NPR];
     if constexpr (ENO == 2) {
       eno_cvt_zone<ENO_A2C, 1>(P, eA, i, j, d1);
@@ -1289,7 +1299,7 @@ __global__ __launch_bounds__(256) void k_eno_ucenter(KParams P, const double* __
   if (i >= P.n1 || j >= P.n2) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pin[NPR], U[NPR];
@@ -1340,7 +1350,7 @@ __global__ __launch_bounds__(256) void k_eno_invert(KParams P, const double* __r
   if (i < P.n1 && j < P.n2) {
     const int z = zidx(P, i, j);
     double gc[36];
-    load_cent(gC, z, gc);
+    load_cent(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     double pin[NPR], U[NPR];
@@ -1400,7 +1410,7 @@ __device__ __forceinline__ void x1_value(const KParams& P, const double* __restr
   const int bc = (i < 0) ? P.bc[HARM_X1DN] : P.bc[HARM_X1UP];
   if (bc != HARM_OUTFLOW) return;  // periodic: the copy itself
   double gc[36];
-  load_cent(gC, zidx(P, i, j), gc);
+  load_cent(P, gC, zidx(P, i, j), gc);
   GeoU g;
   geo_from_cent(gc, g);
   if (inflow_check_x1(P, i, v, gc, g) >= 1) fail = 1;
@@ -1600,7 +1610,7 @@ __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, cons
       }
   }
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pz[NPR];
@@ -2077,7 +2087,7 @@ __device__ __forceinline__ void outflow_value(const KParams& P, const double* __
     for (int k = 0; k < NPR; k++) v[k] = (src[k] / sr[k]) * si[k];
     return;
   }
-  const double gr = gC[(size_t)zidx(P, ri, j) * GCN + GC_GDET], gi = gC[(size_t)zidx(P, i, j) * GCN + GC_GDET];
+  const double gr = geo_entry(P, gC, GC_GDET, zidx(P, ri, j)), gi = geo_entry(P, gC, GC_GDET, zidx(P, i, j));
   const bool up = ri > 0;
   const double dx1 = P.dx1;
   for (int k = RHO; k <= UU; k++) v[k] = src[k] * gr / gi;
@@ -2210,7 +2220,7 @@ __global__ void k_bg_disk(KParams P, double* __restrict__ pv, const double* __re
     p[B3] = (1.0 - fun) * an[B3] + fun * rp[B3];
     p[B2] = an[B2];
     double gc[36];
-    load_cent(gC, zidx(P, i, j), gc);
+    load_cent(P, gC, zidx(P, i, j), gc);
     GeoU g;
     geo_from_cent(gc, g);
     double Bcon[4], Bcov[4], Bsq;
@@ -2258,7 +2268,7 @@ __global__ __launch_bounds__(128) void k_utoprim_batch(KParams P, int n, const i
   if (t >= n) return;
   int z = zidx(P, zone[2 * t], zone[2 * t + 1]);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   double u[NPR], p[NPR];
 #pragma unroll
   for (int k = 0; k < NPR; k++) {
@@ -2307,7 +2317,7 @@ __global__ void k_bsqflags(KParams P, const double* __restrict__ pv, const doubl
   int f0 = 0, f3 = 0;
   if (P.eomtype == HARM_EOMGRMHD) {
     double gc[36];
-    load_cent(gC, z, gc);
+    load_cent(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     double pr[NPR];
@@ -2336,7 +2346,7 @@ __global__ void k_gammacheck(KParams P, const double* __restrict__ pv, const dou
   if (bsqf[zm] == 0 || pflag[zm] != 0) return;
   const int z = zidx(P, i, j);
   double gc[36];
-  load_cent(gC, z, gc);
+  load_cent(P, gC, z, gc);
   GeoU g;
   geo_from_cent(gc, g);
   double pr[NPR];
@@ -2660,7 +2670,7 @@ extern "C" int harm_create(const harm_params* prm, harm_ctx** out) {
   c->N2M = prm->n2 + 2 * NG;
   c->nz = c->N1M * c->N2M;
   KParams& k = c->kp;
-  k.n1 = prm->n1; k.n2 = prm->n2; k.N2M = c->N2M;
+  k.n1 = prm->n1; k.n2 = prm->n2; k.N2M = c->N2M; k.nz = c->nz;
   k.eomtype = prm->eomtype; k.lim = prm->lim; k.fluxmethod = prm->fluxmethod; k.fluxb = prm->fluxb;
   for (int b = 0; b < 4; b++) k.bc[b] = prm->bc[b];
   // advance_eno_u calls fix_flux whatever FIXUPFLUX says (advance.c:355)
@@ -2828,8 +2838,8 @@ extern "C" int harm_set_stream(harm_ctx* c, void* s) {
 }
 
 // the reference's set_grid() tables packed into the device records: face
-// records hF [2][nz][GF], CENT records hC [nz][GCN], the connection
-// component-major hT [NCONN][nz] (floors may be null: zero).  The records keep
+// tables, component-major: faces hF [2][GF][nz], CENT hC [GCN][nz], the
+// connection hT [NCONN][nz] (floors may be null: zero).  The records keep
 // one triangle of gcov and of the connection's lower index pair, so those
 // must be symmetric to the bit (set_grid()'s are); returns false if not.
 static bool pack_geometry(size_t nz, const double* gcov, const double* gcon, const double* gdet, const double* conn,
@@ -2854,26 +2864,22 @@ static bool pack_geometry(size_t nz, const double* gcov, const double* gcon, con
     for (int pos = 0; pos < 2; pos++) {
       const double* gc = gcov + (z * 4 + pos) * 16;
       const double* gn = gcon + (z * 4 + pos) * 16;
-      double* o = &hF[((size_t)pos * nz + z) * GF];
-      o[0] = gc[0]; o[1] = gc[1]; o[2] = gc[2]; o[3] = gc[3];
-      o[4] = gc[5]; o[5] = gc[6]; o[6] = gc[7];
-      o[7] = gc[10]; o[8] = gc[11]; o[9] = gc[15];
-      o[10] = gn[0]; o[11] = gn[1]; o[12] = gn[2]; o[13] = gn[3];
-      o[14] = (pos == 0) ? gn[5] : gn[10];
-      o[15] = gdet[z * 4 + pos];
+      double* o = &hF[(size_t)pos * GF * nz + z];
+      for (int u = 0; u < 10; u++) o[u * nz] = gc[ua[u] * 4 + ub[u]];
+      for (int m = 0; m < 4; m++) o[(10 + m) * nz] = gn[m];
+      o[14 * nz] = (pos == 0) ? gn[5] : gn[10];
+      o[15 * nz] = gdet[z * 4 + pos];
     }
-    double* o = &hC[z * GCN];
+    double* o = &hC[z];
     const double* gc = gcov + (z * 4 + 3) * 16;
     const double* gn = gcon + (z * 4 + 3) * 16;
-    for (int u = 0; u < 10; u++) o[u] = gc[ua[u] * 4 + ub[u]];
-    for (int m = 0; m < 16; m++) o[10 + m] = gn[m];
-    o[GC_GDET] = gdet[z * 4 + 3];
-    o[GC_GDET + 1] = floors ? floors[z * 2 + 0] : 0.0;
-    o[GC_GDET + 2] = floors ? floors[z * 2 + 1] : 0.0;
-    o[GC_GDETC] = gdet[z * 4 + 2];
+    for (int u = 0; u < 10; u++) o[u * nz] = gc[ua[u] * 4 + ub[u]];
+    for (int m = 0; m < 16; m++) o[(10 + m) * nz] = gn[m];
+    o[GC_GDET * nz] = gdet[z * 4 + 3];
+    o[(GC_GDET + 1) * nz] = floors ? floors[z * 2 + 0] : 0.0;
+    o[(GC_GDET + 2) * nz] = floors ? floors[z * 2 + 1] : 0.0;
+    o[GC_GDETC * nz] = gdet[z * 4 + 2];
   }
-  // the connection component-major ([NCONN][zones]): the update's lanes
-  // (adjacent zones) then read adjacent words of each component
   for (size_t z = 0; z < nz; z++)
     for (int k = 0; k < 4; k++)
       for (int u = 0; u < 10; u++) hT[(size_t)(k * 10 + u) * nz + z] = conn[z * 64 + (k * 4 + ua[u]) * 4 + ub[u]];

@@ -37,11 +37,11 @@ __device__ __forceinline__ void store8t(double* __restrict__ a, double* __restri
   store8(da, z, dx);
 }
 
-__device__ __forceinline__ void load_geo_face_t(const double* __restrict__ gF, const double* __restrict__ dgF, int z,
+__device__ __forceinline__ void load_geo_face_t(const KParams& P, const double* __restrict__ gF, const double* __restrict__ dgF, int z,
                                                 GeoT<Dual>& g) {
   GeoU a, b;
-  load_geo_face(gF, z, a);
-  load_geo_face(dgF, z, b);
+  load_geo_face(P, gF, z, a);
+  load_geo_face(P, dgF, z, b);
   g.g00 = Dual(a.g00, b.g00); g.g01 = Dual(a.g01, b.g01); g.g02 = Dual(a.g02, b.g02); g.g03 = Dual(a.g03, b.g03);
   g.g11 = Dual(a.g11, b.g11); g.g12 = Dual(a.g12, b.g12); g.g13 = Dual(a.g13, b.g13);
   g.g22 = Dual(a.g22, b.g22); g.g23 = Dual(a.g23, b.g23); g.g33 = Dual(a.g33, b.g33);
@@ -50,9 +50,9 @@ __device__ __forceinline__ void load_geo_face_t(const double* __restrict__ gF, c
   g.gdet = Dual(a.gdet, b.gdet);
 }
 
-__device__ __forceinline__ void load_cent_t(const double* __restrict__ gC, const double* __restrict__ dgC, int z,
+__device__ __forceinline__ void load_cent_t(const KParams& P, const double* __restrict__ gC, const double* __restrict__ dgC, int z,
                                             Dual* gc) {
-  cent_expand([&](int m) { return Dual(gC[(size_t)z * GCN + m], dgC[(size_t)z * GCN + m]); }, gc);
+  cent_expand([&](int m) { return Dual(geo_entry(P, gC, m, z), geo_entry(P, dgC, m, z)); }, gc);
 }
 
 // ---- fluxcalc: one thread per face (flux_face_single / face_finish) ----
@@ -82,7 +82,7 @@ __device__ __forceinline__ void tl_face(const KParams& P, const double* __restri
     }
   }
   GeoT<Dual> g;
-  load_geo_face_t(gF, dgF, z0, g);
+  load_geo_face_t(P, gF, dgF, z0, g);
   Dual Fo[NPR], dt;
   face_flux<DIR>(P, p_l, p_r, g, Fo, dt, fail);
   dtij = dt.v;
@@ -96,7 +96,7 @@ __device__ __forceinline__ void tl_face(const KParams& P, const double* __restri
         if ((j == 0 && P.bc[HARM_X2DN] == HARM_POLARAXIS) || (j == P.n2 - 1 && P.bc[HARM_X2UP] == HARM_POLARAXIS)) {
           const int zg = zidx(P, i, j == 0 ? -1 : P.n2);
           const Dual v = -Fo[B2];
-          const Dual qg = v / Dual(gF[(size_t)zg * GF + 15], dgF[(size_t)zg * GF + 15]);
+          const Dual qg = v / Dual(face_gdet(P, gF, zg), face_gdet(P, dgF, zg));
           F[(size_t)zg * 8 + B2] = v.v;
           dF[(size_t)zg * 8 + B2] = v.d;
           q[zg] = qg.v;
@@ -160,7 +160,7 @@ __device__ __forceinline__ Dual tl_emf(const KParams& P, const double* __restric
                                        const double* __restrict__ q2, const double* __restrict__ dq2,
                                        const double* __restrict__ gC, const double* __restrict__ dgC, int i, int j) {
   const int z = zidx(P, i, j), zj = zidx(P, i, j - 1), zi = zidx(P, i - 1, j);
-  const Dual gc(gC[(size_t)z * GCN + GC_GDETC], dgC[(size_t)z * GCN + GC_GDETC]);
+  const Dual gc(geo_entry(P, gC, GC_GDETC, z), geo_entry(P, dgC, GC_GDETC, z));
   return 0.25 * gc * (Dual(q1[z], dq1[z]) + Dual(q1[zj], dq1[zj]) - Dual(q2[z], dq2[z]) - Dual(q2[zi], dq2[zi]));
 }
 
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void k_tl_update(KParams P, RKCoef C, TLArrays
     const int z = zidx(P, i, j);
     const double dt = ds->dt;
     Dual gc[36];
-    load_cent_t(A.gC, A.dgC, z, gc);
+    load_cent_t(P, A.gC, A.dgC, z, gc);
     GeoT<Dual> g;
     geo_from_cent(gc, g);
     Dual pin[NPR], pbz[NPR], Ui[NPR];
@@ -197,12 +197,11 @@ __global__ __launch_bounds__(256) void k_tl_update(KParams P, RKCoef C, TLArrays
     // value-plus-tangent state of the whole update does not fit in registers
     __builtin_amdgcn_sched_barrier(0);
     // source(pb) with the component-major connection and its tangent
-    const size_t nzz = (size_t)(P.n1 + 2 * NG) * P.N2M;
     Dual dUg[NPR];
     source_conn_at(P, pbz, g,
                    [&](int e) {
-                     const size_t o = (size_t)conn_sym(e) * nzz + z;
-                     return Dual(A.gConn[o], A.dgConn[o]);
+                     const int m = conn_sym(e);
+                     return Dual(geo_entry(P, A.gConn, m, z), geo_entry(P, A.dgConn, m, z));
                    },
                    dUg);
     __builtin_amdgcn_sched_barrier(0);
@@ -274,7 +273,7 @@ __device__ void tl_bound_x1(const KParams& P, double* __restrict__ pr, double* _
   load8t(pr, dpr, zidx(P, x1_source(P, i), j), v);
   if (bc == HARM_OUTFLOW) {
     Dual gc[36];
-    load_cent_t(gC, dgC, zidx(P, i, j), gc);
+    load_cent_t(P, gC, dgC, zidx(P, i, j), gc);
     GeoT<Dual> g;
     geo_from_cent(gc, g);
     if (inflow_check_x1(P, i, v, gc, g) >= 1) fail = 1;
@@ -349,7 +348,7 @@ __global__ void k_tl_eflux(KParams P, const double* __restrict__ p, const double
   if (j < P.n2) {
     const int z = zidx(P, i, j);
     Dual gc[36], pr[NPR], F[NPR];
-    load_cent_t(gC, dgC, z, gc);
+    load_cent_t(P, gC, dgC, z, gc);
     GeoT<Dual> g;
     geo_from_cent(gc, g);
     load8t(p, dp, z, pr);
