@@ -1588,9 +1588,10 @@ __device__ __forceinline__ bool interior(const KParams& P, int i, int j) {
 // cs (nullable): zones failed by fixup_checksolution in this pass.  Ghost
 // neighbours carry the flags bound_pflag copied before that check, so a
 // ghost whose source zone was failed by it still counts as good.
-// PF: the neighbours' densities and velocities (components RHO..U3, the ones
-// the repair averages) loaded with the flags (one memory round trip instead
-// of two; the values are those the branch then reads)
+// PF (cs null): the neighbours' densities and velocities (components RHO..U3,
+// the ones the repair averages) and all eight flags loaded together: one memory
+// round trip, where the flags read as the case chain asks for them are up to
+// eight in a row (the values are those the chain then reads)
 template <bool PF = false>
 __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, const int* __restrict__ pflag,
                            const int* __restrict__ cs, double* __restrict__ pfix, const double* __restrict__ gC,
@@ -1598,6 +1599,7 @@ __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, cons
   const int i = z / P.N2M - NG, j = z % P.N2M - NG;
   constexpr int NA = U3 + 1;
   double nb[PF ? 9 : 1][PF ? NA : 1];
+  int nf[PF ? 9 : 1];
   if constexpr (PF) {
 #pragma unroll
     for (int di = -1; di <= 1; di++)
@@ -1607,6 +1609,8 @@ __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, cons
         double* o = nb[(di + 1) * 3 + (dj + 1)];
 #pragma unroll
         for (int k = 0; k < NA; k++) o[k] = a[k];
+        const int zm = pflag_zone(P, i + di, j + dj);
+        nf[(di + 1) * 3 + (dj + 1)] = fixed_x1_ghost(P, i + di) ? PFLAG_INIT : pflag[zm];
       }
   }
   double gc[36];
@@ -1617,11 +1621,15 @@ __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, cons
   load8(pv, z, pz);
   double gamma = gamma_calc(pz, g);
   if (gamma > P.gammamax) gamma = P.gammamax;
-  auto good = [&](int di, int dj) {
+  auto flag_of = [&](int di, int dj) {
     const int a = i + di, b = j + dj, zm = pflag_zone(P, a, b);
     int f = fixed_x1_ghost(P, a) ? PFLAG_INIT : pflag[zm];
     if (cs && !interior(P, a, b) && cs[zm]) f = 0;
-    return f == 0;
+    return f;
+  };
+  auto good = [&](int di, int dj) {
+    if constexpr (PF) return nf[(di + 1) * 3 + (dj + 1)] == 0;
+    else return flag_of(di, dj) == 0;
   };
   auto val = [&](int di, int dj, int k) {
     if constexpr (PF) return nb[(di + 1) * 3 + (dj + 1)][k];
@@ -1645,26 +1653,27 @@ __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, cons
   else if (good(-1, 1)) mode = 12;
   else if (good(0, 1)) mode = 13;
   else mode = 14;
-  for (int k = 0; k <= U3; k++) {
-    double v;
-    switch (mode) {
-      case 0: v = avg41(k); break;
-      case 1: v = avg42(k); break;
-      case 2: v = (0.5 * (val(0, 1, k) + val(0, -1, k))); break;
-      case 3: v = (0.5 * (val(1, 0, k) + val(-1, 0, k))); break;
-      case 4: v = (0.5 * (val(1, 1, k) + val(-1, -1, k))); break;
-      case 5: v = (0.5 * (val(1, -1, k) + val(-1, 1, k))); break;
-      case 6: v = val(1, 1, k); break;
-      case 7: v = val(1, 0, k); break;
-      case 8: v = val(1, -1, k); break;
-      case 9: v = val(0, -1, k); break;
-      case 10: v = val(-1, -1, k); break;
-      case 11: v = val(-1, 0, k); break;
-      case 12: v = val(-1, 1, k); break;
-      case 13: v = val(0, 1, k); break;
-      default: v = 0.5 * (avg41(k) + avg42(k)); break;
-    }
-    pz[k] = v;
+  // the case outside the components: a wavefront runs each case its lanes took once
+  auto all = [&](auto value) {
+#pragma unroll
+    for (int k = 0; k <= U3; k++) pz[k] = value(k);
+  };
+  switch (mode) {
+    case 0: all([&](int k) { return avg41(k); }); break;
+    case 1: all([&](int k) { return avg42(k); }); break;
+    case 2: all([&](int k) { return (0.5 * (val(0, 1, k) + val(0, -1, k))); }); break;
+    case 3: all([&](int k) { return (0.5 * (val(1, 0, k) + val(-1, 0, k))); }); break;
+    case 4: all([&](int k) { return (0.5 * (val(1, 1, k) + val(-1, -1, k))); }); break;
+    case 5: all([&](int k) { return (0.5 * (val(1, -1, k) + val(-1, 1, k))); }); break;
+    case 6: all([&](int k) { return val(1, 1, k); }); break;
+    case 7: all([&](int k) { return val(1, 0, k); }); break;
+    case 8: all([&](int k) { return val(1, -1, k); }); break;
+    case 9: all([&](int k) { return val(0, -1, k); }); break;
+    case 10: all([&](int k) { return val(-1, -1, k); }); break;
+    case 11: all([&](int k) { return val(-1, 0, k); }); break;
+    case 12: all([&](int k) { return val(-1, 1, k); }); break;
+    case 13: all([&](int k) { return val(0, 1, k); }); break;
+    default: all([&](int k) { return 0.5 * (avg41(k) + avg42(k)); }); break;
   }
   const int slot = acct_base(P.n1, P.n2, 3) + (i * P.n2 + j) * 2;
   if (P.acct_flag) {  // the states of fixup.c:850's limit_gamma event: before it ...
@@ -1685,13 +1694,9 @@ __device__ void fixup_zone(const KParams& P, const double* __restrict__ pv, cons
     P.acct_flag[slot] = (lg == -1) ? -1 : -2;  // states stored; k_acct_fixg makes the events
     P.acct_flag[slot + 1] = cat + 1;
   }
-  double* o = pfix + (size_t)z * 8;  // the whole repaired state (the fields unchanged)
+  double* o = keep ? keep : pfix + (size_t)z * 8;  // the whole repaired state (the fields unchanged)
 #pragma unroll
   for (int k = 0; k < NPR; k++) o[k] = pz[k];
-  if (keep) {
-#pragma unroll
-    for (int k = 0; k < NPR; k++) keep[k] = pz[k];
-  }
 }
 
 constexpr int KB_BOUND = 1;     // bound_prim()
@@ -2001,6 +2006,7 @@ __global__ __launch_bounds__(256) void k_fixbound(KParams P, double* __restrict_
                                                   int do_dt) {
   __shared__ double keep[FIX ? FIXKEEP * NPR : 1];
   __shared__ int keepz[FIX ? FIXKEEP : 1];
+  __shared__ int corner_fixed[4];  // pole-row edge zone e is on the list: its images are the list's
   // the t, dt update after the last substage reads only the step's scalars:
   // one thread of the last wavefront, beside the repair
   if (do_dt && threadIdx.x == blockDim.x - 1) dt_update(P, ds);
@@ -2008,56 +2014,72 @@ __global__ __launch_bounds__(256) void k_fixbound(KParams P, double* __restrict_
   int n = FIX ? ds->nlist : 0, fail = 0;
   // the list's first entries read beside its length (used only below n)
   const int z0 = (FIX && (int)threadIdx.x < cap) ? faillist[threadIdx.x] : 0;
+  // column g of pole-row edge zone e (e&1 the x1 side, e&2 the x2 side): the
+  // threads of the second wavefront, their values (computed by k_update from
+  // the zeroed row) read beside the list too
+  const int ct = (int)threadIdx.x - 64, e = ct / NG, g = ct % NG;
+  const int ci = (e & 1) ? P.n1 - 1 : 0, cj = (e & 2) ? P.n2 - 1 : 0;
+  const bool corner = ct >= 0 && ct < 4 * NG && pole_row(P, cj) && P.bc[(e & 1) ? HARM_X1UP : HARM_X1DN] == HARM_OUTFLOW;
+  double cv[NPR];
+  int cfail = 0;
+  if (corner && P.n1 >= 5) {
+#pragma unroll
+    for (int k = 0; k < NPR; k++) cv[k] = ds->pole_x1[e][g][k];
+    cfail = ds->pole_fail[e][g];
+  }
+  if (FIX) {
+    if (threadIdx.x < 4) corner_fixed[threadIdx.x] = 0;
+    __syncthreads();
+  }
   if (n > cap) n = cap;
   for (int t = threadIdx.x; t < n; t += blockDim.x) {
     const int z = (t == (int)threadIdx.x) ? z0 : faillist[t];
     fixup_zone<true>(P, pv, pflag, nullptr, pfix, gC, z, fail, t < FIXKEEP ? keep + (size_t)t * NPR : nullptr);
     if (t < FIXKEEP) keepz[t] = z;
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      if (z == zidx(P, (c & 1) ? P.n1 - 1 : 0, (c & 2) ? P.n2 - 1 : 0)) corner_fixed[c] = 1;
   }
   __syncthreads();  // every repaired state computed from the unrepaired array
-  auto entry = [&](int q, double* v) {
-    const int z = (q < FIXKEEP) ? keepz[q] : faillist[q];
+  auto entry_zone = [&](int q) { return (q < FIXKEEP) ? keepz[q] : faillist[q]; };
+  auto entry = [&](int q, int z, double* v) {
     if (q < FIXKEEP) {
 #pragma unroll
       for (int k = 0; k < NPR; k++) v[k] = keep[q * NPR + k];
     } else {
       load8(pfix, z, v);
     }
-    return z;
   };
   const int nimg = n * NIMG;
-  for (int t = threadIdx.x; t < n + nimg + 4 * NG; t += blockDim.x) {
+  for (int t = threadIdx.x; t < n + nimg; t += blockDim.x) {
     double v[NPR];
     if (t < n) {  // the repaired zone
-      const int z = entry(t, v);
+      const int z = entry_zone(t);
+      entry(t, z, v);
       const bool pole = pole_row(P, z % P.N2M - NG);
 #pragma unroll
       for (int k = 0; k <= U3; k++) pv[(size_t)z * 8 + k] = (pole && k == U2) ? v[k] * 0. : v[k];
       if (pole) pv[(size_t)z * 8 + B2] = v[B2] * 0.;
       pflag[z] = -1;  // UTOPRIMFAILFIXED (global.h:524)
-    } else if (t < n + nimg) {  // one part of its images
+    } else {  // one part of its images
       const int q = (t - n) / NIMG, part = (t - n) % NIMG;
-      const int z = entry(q, v);
-      bound_image_part(P, pv, gC, z / P.N2M - NG, z % P.N2M - NG, v, part, fail);
-    } else {  // column g of pole-row edge zone e (e&1 the x1 side, e&2 the x2 side)
-      const int e = (t - n - nimg) / NG, g = (t - n - nimg) % NG;
-      const int i = (e & 1) ? P.n1 - 1 : 0, j = (e & 2) ? P.n2 - 1 : 0;
-      if (!pole_row(P, j) || P.bc[(e & 1) ? HARM_X1UP : HARM_X1DN] != HARM_OUTFLOW) continue;
-      const int ze = zidx(P, i, j);
-      bool repaired = false;  // then its images are the list's
-      for (int q = 0; q < n && !repaired; q++) repaired = ((q < FIXKEEP) ? keepz[q] : faillist[q]) == ze;
-      if (repaired) continue;
-      const int ig = (e & 1) ? P.n1 + g : -1 - g;
-      if (P.n1 >= 5) {  // computed by k_update from the zeroed row
-#pragma unroll
-        for (int k = 0; k < NPR; k++) v[k] = ds->pole_x1[e][g][k];
-        if (ds->pole_fail[e][g]) fail = 1;
-        store8(pv, zidx(P, ig, j), v);
-        bound_x2_images(P, pv, ig, j, v);
-      } else {
-        load8(pv, ze, v);
-        bound_image_part(P, pv, gC, i, j, v, (e & 1) ? NG + 1 + g : 1 + g, fail);
+      const int z = entry_zone(q), i = z / P.N2M - NG, j = z % P.N2M - NG;
+      if (near_edge(P, i, j)) {
+        entry(q, z, v);
+        bound_image_part(P, pv, gC, i, j, v, part, fail);
       }
+    }
+  }
+  if (corner && !(FIX && corner_fixed[e])) {
+    if (P.n1 >= 5) {
+      const int ig = (e & 1) ? P.n1 + g : -1 - g;
+      if (cfail) fail = 1;
+      store8(pv, zidx(P, ig, cj), cv);
+      bound_x2_images(P, pv, ig, cj, cv);
+    } else {
+      double v[NPR];
+      load8(pv, zidx(P, ci, cj), v);
+      bound_image_part(P, pv, gC, ci, cj, v, (e & 1) ? NG + 1 + g : 1 + g, fail);
     }
   }
   if (fail) atomicOr(&ds->failed, 1);
