@@ -1,0 +1,282 @@
+// harm_fast.h -- the face physics of harm_device.h with fewer instructions,
+// for the flux and update kernels.  Same results: each function computes what
+// its harm_device.h counterpart computes, operation for operation, where its
+// inputs are finite, and reports where they are not (the finiteness sums), so
+// that the caller takes the general function there.
+//
+// What is saved, and why the results stay:
+//  - Quotients by one divisor share its reciprocal.  An IEEE quotient on
+//    gfx950 is a refined reciprocal r of d (v_rcp_f64 and two Newton steps)
+//    and q = n r, q + (n - d q) r, between scalings that act only at extreme
+//    exponents.  Within the range that Divisor checks no scaling acts, its steps
+//    are then the same operations, and v_div_fixup_f64 gives zeros, infinities
+//    and NaN: 6 instructions a further quotient, checks included, instead of 11.
+//  - Minima and maxima are v_min_f64 / v_max_f64 (1 instruction instead of a
+//    compare and two selects); they differ from the reference's comparisons
+//    only for NaN, which the finiteness sums exclude, and in which of +0 and
+//    -0 a tie gives.
+//  - Terms multiplied by zero (the unused flux formula, the off-diagonal
+//    pressure) are left out; with finite operands they add a zero.
+#pragma once
+#include "harm_device.h"
+
+namespace harm {
+
+HARM_HD double fast_rcp(double d) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_rcp(d);
+#else
+  return 1.0 / d;
+#endif
+}
+HARM_HD double fast_fixup(double q, double d, double n) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_div_fixup(q, d, n);
+#else
+  return (n == 0.0 || d == 0.0 || !isfinite(n) || !isfinite(d)) ? n / d : q;
+#endif
+}
+// the binary exponent (fraction in [1/2, 1)); 0 for zeros, infinities and NaN
+HARM_HD int fast_exponent(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_frexp_exp(x);
+#else
+  int e = 0;
+  if (x != 0.0 && isfinite(x)) (void)frexp(x, &e);
+  return e;
+#endif
+}
+
+// Quotients by one divisor.  No scaling acts in n / d if |n| >= 2^-969, d,
+// 1/d and n/d are normal, and the exponents of n and d are less than 768 apart
+// (zeros, infinities and NaN are the fixup's).  Exponents of numerators in
+// [-950, 650] and of the divisor in [-95, 65] are inside that; the divisor's is
+// tested as ten times itself, with the numerators'.  Outside (a field that
+// spreads into a field-free region falls to 1e-300 within some hundred zones)
+// the group's quotients are formed by plain divisions.
+struct Divisor {
+  double d, r;
+  int e10;
+  HARM_HD explicit Divisor(double x) : d(x) {
+    e10 = fast_exponent(x) * 10;
+    r = fast_rcp(x);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  }
+  template <int N>
+  HARM_HD void under(const double (&n)[N], double (&q)[N]) const {
+    int lo = e10, hi = e10;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int e = fast_exponent(n[k]);
+      lo = lo < e ? lo : e;
+      hi = hi > e ? hi : e;
+      const double t = n[k] * r;
+      q[k] = fast_fixup(__builtin_fma(__builtin_fma(-d, t, n[k]), r, t), d, n[k]);
+    }
+    if (__builtin_expect(lo < -950 || hi > 650, 0)) {
+#pragma unroll
+      for (int k = 0; k < N; k++) q[k] = n[k] / d;
+    }
+  }
+};
+
+HARM_HD double vmin(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_fmin(a, b);
+#else
+  return (a > b) ? b : a;
+#endif
+}
+HARM_HD double vmax(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_fmax(a, b);
+#else
+  return (a > b) ? a : b;
+#endif
+}
+
+// para4 for finite values: `z` becomes NaN if one of them or of the slope
+// products is not finite.  A slope's sign is that of its central difference
+// where it is kept (the one-sided differences then agree in sign).
+HARM_HD void para4_fast(double y0, double y1, double y2, double y3, double y4, double& lout, double& rout, double& z) {
+  const double y[5] = {y0, y1, y2, y3, y4};
+  double D[4], dq[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) D[i] = 2.0 * (y[i + 1] - y[i]);
+#pragma unroll
+  for (int i = 1; i < 4; i++) {
+    const double Dqc = 0.5 * (y[i + 1] - y[i - 1]);
+    const double s = D[i - 1] * D[i];
+    z = __builtin_fma(s, 0.0, z);
+    const double m = __builtin_copysign(vmin(fabs(Dqc), vmin(fabs(D[i - 1]), fabs(D[i]))), Dqc);
+    dq[i] = (s <= 0.) ? 0. : m;
+  }
+  double l = 0.5 * (y[2] + y[1]) - (dq[2] - dq[1]) / 8.0;
+  double r = 0.5 * (y[3] + y[2]) - (dq[3] - dq[2]) / 8.0;
+  l = vmin(vmax(y[2], y[1]), vmax(vmin(y[2], y[1]), l));
+  r = vmin(vmax(y[2], y[3]), vmax(vmin(y[2], y[3]), r));
+  const double qa = (r - y[2]) * (y[2] - l);
+  const double qd = (r - l);
+  const double qe = 8.0 * (y[2] - 0.5 * (l + r));
+  const double l1 = (qd * (qd - qe) < 0.0) ? 3.0 * y[2] - 2.0 * r : l;
+  const double r1 = (qd * (qd + qe) < 0.0) ? 3.0 * y[2] - 2.0 * l1 : r;
+  const bool flat = qa <= 0.;
+  lout = flat ? y[2] : l1;
+  rout = flat ? y[2] : r1;
+}
+
+// what the two states of a face share
+struct FaceGeo {
+  Divisor A;  // alpha
+  double beta1, beta2, beta3;
+  HARM_HD explicit FaceGeo(const GeoU& g) : A(1. / sqrt(-g.n00)) {
+    beta1 = g.n01 * A.d * A.d;
+    beta2 = g.n02 * A.d * A.d;
+    beta3 = g.n03 * A.d * A.d;
+  }
+};
+
+// one state of a face: limit_gamma, get_state, primtoflux for F and U, vchar
+template <int DIR>
+HARM_HD void face_state_fast(const KParams& P, double* p, const GeoU& g, const FaceGeo& fg, double* F, double* U,
+                             double& vmx, double& vmn, int& fail) {
+  double gamma = gamma_calc(p, g);
+  if (P.gammamax > 1.0 && gamma > P.gammamax) {
+    if (limit_gamma(P.gammamax, p, g) >= 1) fail = 1;
+    gamma = gamma_calc(p, g);
+  }
+  double uc[4], ul[4], bc[4], bl[4];
+  {
+    const double n[4] = {gamma, gamma * fg.beta1, gamma * fg.beta2, gamma * fg.beta3};
+    double v[4];
+    fg.A.under(n, v);
+    uc[0] = v[0];
+    uc[1] = p[U1] - v[1];
+    uc[2] = p[U2] - v[2];
+    uc[3] = p[U3] - v[3];
+  }
+  lower(uc, g, ul);
+  const Divisor T(uc[0]);
+  bc[0] = p[B1] * ul[1] + p[B2] * ul[2] + p[B3] * ul[3];
+  constexpr int t1 = (DIR == 1) ? 2 : 1, t2 = 3;  // the field components along the face
+  const double Bd = p[B1 + DIR - 1];
+  const double n[5] = {p[B1] + bc[0] * uc[1], p[B2] + bc[0] * uc[2], p[B3] + bc[0] * uc[3],
+                       p[B1 + t1 - 1] * uc[DIR] - Bd * uc[t1], p[B1 + t2 - 1] * uc[DIR] - Bd * uc[t2]};
+  double v[5];
+  T.under(n, v);
+  bc[1] = v[0];
+  bc[2] = v[1];
+  bc[3] = v[2];
+  lower(bc, g, bl);
+  const double bsq = dot4(bc, bl);
+  double Pg = 0., w = 0.;
+  if (P.eomtype == 0) {
+    Pg = (P.gam - 1.) * p[UU];
+    w = Pg + p[RHO] + p[UU];
+  }
+  const double eta = w + bsq, ptot = Pg + bsq * 0.5;
+  auto row = [&](int dir, double* f) {  // T^dir_j and the mass flux
+    const double ed = eta * uc[dir], bd = bc[dir];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      f[UU + j] = ((dir == j) ? ed * ul[j] + ptot : ed * ul[j]) - bd * bl[j];
+    f[RHO] = p[RHO] * uc[dir];
+    if (P.eomtype == 0) f[UU] += f[RHO];
+  };
+  row(DIR, F);
+  row(0, U);
+  F[B1 + DIR - 1] = Bd * uc[DIR] - Bd * uc[DIR];  // +0, as is its quotient
+  F[B1 + t1 - 1] = v[3];
+  F[B1 + t2 - 1] = v[4];
+#pragma unroll
+  for (int k = B1; k <= B3; k++) U[k] = p[k];
+#pragma unroll
+  for (int k = 0; k < NPR; k++) {
+    F[k] = F[k] * g.gdet;
+    U[k] = U[k] * g.gdet;
+  }
+  // vchar
+  const double gam = P.gam, rho = p[RHO], u = p[UU];
+  const double WW0 = rho + gam * u;
+  const bool wpos = WW0 > 0.0;
+  const double cs2w = gam * (gam - 1.) * u / WW0;
+  const double WW = wpos ? WW0 : 0.0, cs2 = wpos ? cs2w : 0.0;
+  const double EF0 = bsq + WW;
+  const double va2e = bsq / EF0;
+  const double va2 = (EF0 > 0.0) ? va2e : 0.0;
+  double cms2 = cs2 + va2 - cs2 * va2;
+  if (cms2 < 0.0) {
+    if (cms2 / (cs2 + va2) > -NUMEPSILON * 100.0) cms2 = 0.0;
+    else fail = 1;
+  } else if (cms2 > 1.) {
+    if (cms2 < 1.0 + NUMEPSILON * 100.0) cms2 = 1.0;
+    else fail = 1;
+  }
+  const double Asq = g.ndd, Bsq = g.n00, AB = (DIR == 1) ? g.n01 : g.n02;
+  const double Au = uc[DIR], Bu = uc[0];
+  const double Au2 = Au * Au, Bu2 = Bu * Bu, AuBu = Au * Bu;
+  const double A = Bu2 - (Bsq + Bu2) * cms2;
+  const double B = 2. * (AuBu - (AB + AuBu) * cms2);
+  const double C = Au2 - (Asq + Au2) * cms2;
+  double discr = B * B - 4. * A * C;
+  if (discr < 0.0) {
+    if (discr < -1E-10) fail = 1;
+    if (discr != -1E-10) discr = 0.0;
+  }
+  discr = sqrt(discr);
+  const double nv[2] = {-(-B + discr), -(-B - discr)};
+  double w2[2];
+  Divisor(2. * A).under(nv, w2);
+  const double vm = w2[0], vp = w2[1];
+  const bool sw = vp < vm;
+  vmx = sw ? vm : vp;
+  vmn = sw ? vp : vm;
+}
+
+// below this sum of the speeds the flux formula that is left out (0 times it is
+// added) may overflow, or the sum is zero
+constexpr double MINSPREAD = 1e-30;
+
+// face_flux: Fo and the largest speed cm (the Courant limit is cour dx / cm).
+// Returns false where the general function has to be taken (on the same states).
+template <int DIR>
+HARM_HD bool face_flux_fast(const KParams& P, const double* p_l0, const double* p_r0, const GeoU& g, double (&Fo)[NPR],
+                            double& cm, int& fail) {
+  constexpr int kb = B1 + DIR - 1;
+  double p_l[NPR], p_r[NPR];
+#pragma unroll
+  for (int k = 0; k < NPR; k++) {
+    p_l[k] = p_l0[k];
+    p_r[k] = p_r0[k];
+  }
+  p_l[kb] = p_r[kb] = 0.5 * (p_l0[kb] + p_r0[kb]);
+  const FaceGeo fg(g);
+  double F_l[NPR], F_r[NPR], U_l[NPR], U_r[NPR];
+  double cmax_l, cmin_l, cmax_r, cmin_r;
+  int f = 0;
+  face_state_fast<DIR>(P, p_l, g, fg, F_l, U_l, cmax_l, cmin_l, f);
+  face_state_fast<DIR>(P, p_r, g, fg, F_r, U_r, cmax_r, cmin_r, f);
+  const double lmin = dmin(cmin_l, cmin_r), lmax = dmax(cmax_l, cmax_r);
+  const double cmin = fabs(dmax(0., -lmin)), cmax = fabs(dmax(0., lmax));
+  cm = dmax(cmax, cmin);
+  double z = 0.;
+  if (P.fluxmethod == 1) {
+    const Divisor S(cmax + cmin);
+    const double cc = cmax * cmin;
+    double n[NPR];
+#pragma unroll
+    for (int k = 0; k < NPR; k++) n[k] = cmax * F_l[k] + cmin * F_r[k] - cc * (U_r[k] - U_l[k]);
+    S.under(n, Fo);
+  } else {
+#pragma unroll
+    for (int k = 0; k < NPR; k++) Fo[k] = (0.5 * (F_l[k] + F_r[k] - cm * (U_r[k] - U_l[k])));
+  }
+#pragma unroll
+  for (int k = 0; k < NPR; k++) z = __builtin_fma(Fo[k], 0.0, z);
+  if (__builtin_expect(!(z == 0.0) || !(cmax + cmin > MINSPREAD), 0)) return false;
+  fail |= f;
+  return true;
+}
+
+}  // namespace harm

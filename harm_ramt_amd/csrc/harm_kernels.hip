@@ -35,7 +35,9 @@
 #include <mutex>
 #include <algorithm>
 #include <stddef.h>
+#include <type_traits>
 #include "harm_device.h"
+#include "harm_fast.h"
 #include "harm_tangent.h"
 #include "harm_adjoint.h"
 #include "harm_eno.h"
@@ -425,17 +427,11 @@ __device__ __forceinline__ void flux_face_single(const KParams& P, const double*
   face_finish<DIR>(P, p_l, p_r, F, q, gF, i, j, dtij, fail);
 }
 
-// everything of a face after the reconstruction: face geometry, fluxes and
-// wave speeds, HLL/LAXF, the fix_flux edge rules, F and the EMF quotient
+// the fix_flux edge rules of a face's flux Fo, then F and the EMF quotient
 template <int DIR>
-__device__ __forceinline__ void face_finish(const KParams& P, double* p_l, double* p_r, double* __restrict__ F,
-                                            double* __restrict__ q, const double* __restrict__ gF, int i, int j,
-                                            double& dtij, int& fail) {
+__device__ __forceinline__ void face_store(const KParams& P, double* Fo, double gdet, double* __restrict__ F,
+                                           double* __restrict__ q, const double* __restrict__ gF, int i, int j) {
   const int z0 = zidx(P, i, j);
-  GeoU g;
-  load_geo_face(P, gF, z0, g);
-  double Fo[NPR];
-  face_flux<DIR>(P, p_l, p_r, g, Fo, dtij, fail);
   bool skip_b2 = false;
   if (P.fixupflux) {
     if (DIR == 1) {
@@ -472,8 +468,21 @@ __device__ __forceinline__ void face_finish(const KParams& P, double* p_l, doubl
       if (k != B2) Fz[k] = Fo[k];
   } else {
     store8(F, z0, Fo);
-    q[z0] = (DIR == 1 ? Fo[B2] : Fo[B1]) / g.gdet;
+    q[z0] = (DIR == 1 ? Fo[B2] : Fo[B1]) / gdet;
   }
+}
+
+// everything of a face after the reconstruction: face geometry, fluxes and
+// wave speeds, HLL/LAXF, the fix_flux edge rules, F and the EMF quotient
+template <int DIR>
+__device__ __forceinline__ void face_finish(const KParams& P, double* p_l, double* p_r, double* __restrict__ F,
+                                            double* __restrict__ q, const double* __restrict__ gF, int i, int j,
+                                            double& dtij, int& fail) {
+  GeoU g;
+  load_geo_face(P, gF, zidx(P, i, j), g);
+  double Fo[NPR];
+  face_flux<DIR>(P, p_l, p_r, g, Fo, dtij, fail);
+  face_store<DIR>(P, Fo, g.gdet, F, q, gF, i, j);
 }
 
 __device__ __forceinline__ void flux_single_body(KParams P, const double* __restrict__ pr,
@@ -523,17 +532,22 @@ __global__ __launch_bounds__(256) void k_flux_single(KParams P, const double* __
 
 using FluxKernel = void (*)(KParams, const double*, double*, double*, double*, double*, const double*, DevScalars*,
                             int);
-// the instantiation for a context's scheme: the torus (PARA, GRMHD, HLL), the
-// force-free problems (MC, FFDE, LAXF) and Orszag-Tang (MC, GRMHD, HLL), or
+// the schemes with kernels of their own: the torus (PARA, GRMHD, HLL), the
+// force-free problems (MC, FFDE, LAXF) and Orszag-Tang (MC, GRMHD, HLL); 0:
 // the general kernel
+int flux_scheme(const KParams& P) {
+  if (P.lim == HARM_PARA && P.eomtype == HARM_EOMGRMHD && P.fluxmethod == HARM_HLLFLUX) return 1;
+  if (P.lim == HARM_MC && P.eomtype == HARM_EOMFFDE && P.fluxmethod == HARM_LAXFFLUX) return 2;
+  if (P.lim == HARM_MC && P.eomtype == HARM_EOMGRMHD && P.fluxmethod == HARM_HLLFLUX) return 3;
+  return 0;
+}
 FluxKernel flux_single_kernel(const KParams& P) {
-  if (P.lim == HARM_PARA && P.eomtype == HARM_EOMGRMHD && P.fluxmethod == HARM_HLLFLUX)
-    return k_flux_single<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>;
-  if (P.lim == HARM_MC && P.eomtype == HARM_EOMFFDE && P.fluxmethod == HARM_LAXFFLUX)
-    return k_flux_single<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>;
-  if (P.lim == HARM_MC && P.eomtype == HARM_EOMGRMHD && P.fluxmethod == HARM_HLLFLUX)
-    return k_flux_single<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>;
-  return k_flux_single<-1, -1, -1>;
+  switch (flux_scheme(P)) {
+    case 1: return k_flux_single<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>;
+    case 2: return k_flux_single<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>;
+    case 3: return k_flux_single<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>;
+    default: return k_flux_single<-1, -1, -1>;
+  }
 }
 
 // Edge states of one zone along DIR from its 5-zone stencil s[0..4]
@@ -553,74 +567,177 @@ __device__ __forceinline__ void zone_edges(const KParams& P, const double (&s)[5
   }
 }
 
+// A value the compiler takes for a new one: what is formed from it again is
+// then formed again (not kept in registers from the first time).
+__device__ __forceinline__ int again(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// zone_edges of zone z (stencil stride zs) with para4 in its shorter form where
+// the stencil is finite.  P0 is the context's parameter block, P the one of
+// the kernel's instantiation: the general code below is compiled for P0, with
+// branches on the scheme, which keeps its registers under the fast path's.
+__device__ __forceinline__ void zone_edges_fast(const KParams& P, const KParams& P0, const double* __restrict__ pr,
+                                                int z, int zs, double* l, double* r) {
+  double s[5][NPR];
+#pragma unroll
+  for (int m = 0; m < 5; m++) load8(pr, z + (m - 2) * zs, s[m]);
+  if (P.lim != 4) {
+    zone_edges(P, s, l, r);
+    return;
+  }
+  double f = 0.;
+#pragma unroll
+  for (int k = 0; k < NPR; k++) para4_fast(s[0][k], s[1][k], s[2][k], s[3][k], s[4][k], l[k], r[k], f);
+  if (!(f == 0.)) {
+    z = again(z);
+#pragma unroll
+    for (int m = 0; m < 5; m++) load8(pr, z + (m - 2) * zs, s[m]);
+    zone_edges(P0, s, l, r);
+  }
+}
+
+// face_finish with the face's flux in its shorter form (the geometry given);
+// where that form does not hold the face is formed from its stencil by the
+// general functions
+template <int DIR>
+__device__ __forceinline__ void face_finish_fast(const KParams& P, const KParams& P0, const double* p_l,
+                                                 const double* p_r, const GeoU& g, const double* __restrict__ pr,
+                                                 double* __restrict__ F, double* __restrict__ q,
+                                                 const double* __restrict__ gF, int i, int j, double& cm,
+                                                 double& dtij, int& fail) {
+  double Fo[NPR];
+  if (face_flux_fast<DIR>(P, p_l, p_r, g, Fo, cm, fail)) {
+    face_store<DIR>(P, Fo, g.gdet, F, q, gF, i, j);
+  } else {
+    cm = 0.;
+    flux_face_single<DIR>(P0, pr, F, q, gF, again(i), j, dtij, fail);
+  }
+}
+
+// the largest of a wavefront's non-negative values, in every lane of its last
+// row's end (lane 63), by register shifts within the wavefront: no LDS round
+// trips; lanes outside a shift keep their own value
+__device__ __forceinline__ double wave_max_dpp(double v) {
+  auto step = [](double a, auto ctrl) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(a);
+    const int lo = __builtin_amdgcn_update_dpp((int)u, (int)u, decltype(ctrl)::value, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(u >> 32), (int)(u >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
+    const double b = __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+    return dmax(a, b);
+  };
+  v = step(v, std::integral_constant<int, 0x111>());  // row_shr:1
+  v = step(v, std::integral_constant<int, 0x112>());  // row_shr:2
+  v = step(v, std::integral_constant<int, 0x114>());  // row_shr:4
+  v = step(v, std::integral_constant<int, 0x118>());  // row_shr:8
+  v = step(v, std::integral_constant<int, 0x142>());  // row_bcast:15
+  v = step(v, std::integral_constant<int, 0x143>());  // row_bcast:31
+  return v;
+}
+
 // fluxcalc() with one thread per zone and direction: each zone's edge states
 // are reconstructed once and shared with the face below it -- along x2
 // between the lanes of a wavefront (63 faces per 64 lanes), along x1 through
-// LDS between the rows of a workgroup (3 face rows per 4).  Workgroup 64x4.
+// LDS between the rows of a workgroup (3 face rows per 4).  The lanes of a
+// wavefront run over the grid's columns as one line (x1: the columns of all
+// groups of rows, x2: all zones), so that no wavefront is left with the few
+// columns beyond a multiple of 64.  Workgroup 64x4, the first nb1 of them x1.
+// Bound by instruction issue: with the scheme a constant, the shorter forms of
+// harm_fast.h and the one-line tiling the 256^2 torus takes 4.0e6 wavefront
+// instructions a launch, 7.0e6 before, and 17.5 us, 21.8 before (512^2: 45.8
+// of 62.1 us; 97x131: 8.5 of 11.9 us).
 constexpr int FSH_ROWS = 4;
-__host__ __device__ __forceinline__ void flux_shared_grid(int n1, int n2, int& gx, int& gy) {
-  const int gx2 = (n2 + 1 + 62) / 63, gy2 = (n1 + 2 + FSH_ROWS - 1) / FSH_ROWS;           // x2 faces
-  const int gx1 = (n2 + 2 + 63) / 64, gy1 = (n1 + 1 + FSH_ROWS - 2) / (FSH_ROWS - 1);     // x1 faces
-  gx = gx2 > gx1 ? gx2 : gx1;
-  gy = gy2 > gy1 ? gy2 : gy1;
+__host__ __device__ __forceinline__ int flux_shared_blocks(int n1, int n2, int dir) {
+  if (dir == 1) {
+    const int groups = (n1 + 1 + FSH_ROWS - 2) / (FSH_ROWS - 1);
+    return (groups * (n2 + 2) + 63) / 64;
+  }
+  return ((n1 + 2) * (n2 + 2) - 1 + 63 * FSH_ROWS - 1) / (63 * FSH_ROWS);
 }
 
-__global__ __launch_bounds__(64 * FSH_ROWS) void k_flux_shared(KParams P, const double* __restrict__ pr,
+__device__ __forceinline__ void flux_shared_body(const KParams& P, const KParams& P0, const double* __restrict__ pr,
+                                                 double* __restrict__ F1, double* __restrict__ F2,
+                                                 double* __restrict__ q1, double* __restrict__ q2,
+                                                 const double* __restrict__ gF, DevScalars* __restrict__ ds, int dir,
+                                                 int blk) {
+  __shared__ double rsh[FSH_ROWS][NPR][64];
+  const int tx = threadIdx.x, ty = threadIdx.y;
+  double cm = 0., dtij = 1.e9;
+  int fail = 0;
+  double l[NPR], r[NPR], p_l[NPR];
+  GeoU g;
+  if (dir == 2) {
+    // lanes along the zones (i, jz) of i in [-1,N1], jz in [-1,N2]; face
+    // (i, jz) takes r of lane tx-1
+    const int id = 63 * (FSH_ROWS * blk + ty) + tx, w = P.n2 + 2;
+    const int i = id / w - 1, jz = id % w - 1;
+    const bool zone_ok = i <= P.n1;
+    const bool face = tx >= 1 && zone_ok && jz >= 0;
+    const double* gF2 = gF + (size_t)P.nz * GF;
+    if (zone_ok) {
+      if (face) load_geo_face(P, gF2, zidx(P, i, jz), g);
+      zone_edges_fast(P, P0, pr, zidx(P, i, jz), 1, l, r);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NPR; k++) l[k] = r[k] = 0.;
+    }
+#pragma unroll
+    for (int k = 0; k < NPR; k++) p_l[k] = __shfl_up(r[k], 1);
+    if (face) face_finish_fast<2>(P, P0, p_l, l, g, pr, F2, q2, gF2, i, jz, cm, dtij, fail);
+  } else {
+    // lanes along the columns j in [-1,N2] of every group of FSH_ROWS-1 face
+    // rows, rows along x1: zone iz of row ty; face (iz, j) takes r of row
+    // ty-1 through LDS
+    const int c = 64 * blk + tx, w = P.n2 + 2;
+    const int j = c % w - 1, iz = (FSH_ROWS - 1) * (c / w) + ty - 1;
+    const bool zone_ok = iz <= P.n1;
+    const bool face = ty >= 1 && zone_ok;
+    if (zone_ok) {
+      if (face) load_geo_face(P, gF, zidx(P, iz, j), g);
+      zone_edges_fast(P, P0, pr, zidx(P, iz, j), P.N2M, l, r);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NPR; k++) l[k] = r[k] = 0.;
+    }
+#pragma unroll
+    for (int k = 0; k < NPR; k++) rsh[ty][k][tx] = r[k];
+    __syncthreads();
+    if (face) {
+#pragma unroll
+      for (int k = 0; k < NPR; k++) p_l[k] = rsh[ty - 1][k][tx];
+      face_finish_fast<1>(P, P0, p_l, l, g, pr, F1, q1, gF, iz, j, cm, dtij, fail);
+    }
+  }
+  // Courant limit: cour dx / cm falls as cm grows, rounding included, so the
+  // wavefront's largest cm gives its smallest quotient (NaN and limits of 1e9
+  // and more count for nothing, as in the reference's running minimum)
+  const double cw = wave_max_dpp(cm);
+  if ((tx & 63) == 63) {
+    const double d = P.cour * ((dir == 1) ? P.dx1 : P.dx2) / cw;
+    if (d < 1.e9) ndt_push(ds, dir, d, dim3(blk, 0, 0));
+  }
+  if (dtij < 1.e9) ndt_push(ds, dir, dtij, dim3(blk, 0, 0));
+  if (fail) atomicOr(&ds->failed, 1);
+}
+
+template <int LIMC, int EOMC, int FMC>
+__global__ __launch_bounds__(64 * FSH_ROWS) void k_flux_shared(KParams P0, const double* __restrict__ pr,
                                                               double* __restrict__ F1, double* __restrict__ F2,
                                                               double* __restrict__ q1, double* __restrict__ q2,
                                                               const double* __restrict__ gF,
-                                                              DevScalars* __restrict__ ds, int dir0) {
-  __shared__ double rsh[FSH_ROWS][64][NPR];
-  const int dir = dir0 + blockIdx.z;
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  double dtij = 1.e9;
-  int fail = 0;
-  double s[5][NPR], l[NPR], r[NPR];
-  if (dir == 2) {
-    // lanes along x2: zone jz, row i; face (i, jz) takes r of lane tx-1
-    const int jz = 63 * (int)blockIdx.x - 1 + tx, i = FSH_ROWS * (int)blockIdx.y + ty - 1;
-    const bool zone_ok = (jz >= -1 && jz <= P.n2 && i >= -1 && i <= P.n1);
-    if (zone_ok) {
-#pragma unroll
-      for (int m = 0; m < 5; m++) load8(pr, zidx(P, i, jz - 2 + m), s[m]);
-      zone_edges(P, s, l, r);
-    } else {
-#pragma unroll
-      for (int k = 0; k < NPR; k++) l[k] = r[k] = 0.;
-    }
-    double p_l[NPR];
-#pragma unroll
-    for (int k = 0; k < NPR; k++) p_l[k] = __shfl_up(r[k], 1);
-    if (tx >= 1 && zone_ok && jz >= 0) {
-      const size_t nz = (size_t)(P.n1 + 2 * NG) * P.N2M;
-      face_finish<2>(P, p_l, l, F2, q2, gF + nz * GF, i, jz, dtij, fail);
-    }
-  } else {
-    // lanes along x2, rows along x1: zone iz of row ty; face (iz, j) takes r
-    // of row ty-1 through LDS
-    const int j = 64 * (int)blockIdx.x + tx - 1, iz = (FSH_ROWS - 1) * (int)blockIdx.y + ty - 1;
-    const bool zone_ok = (j >= -1 && j <= P.n2 && iz >= -1 && iz <= P.n1);
-    if (zone_ok) {
-#pragma unroll
-      for (int m = 0; m < 5; m++) load8(pr, zidx(P, iz - 2 + m, j), s[m]);
-      zone_edges(P, s, l, r);
-    } else {
-#pragma unroll
-      for (int k = 0; k < NPR; k++) l[k] = r[k] = 0.;
-    }
-#pragma unroll
-    for (int k = 0; k < NPR; k++) rsh[ty][tx][k] = r[k];
-    __syncthreads();
-    if (ty >= 1 && zone_ok && iz >= 0) {
-      double p_l[NPR];
-#pragma unroll
-      for (int k = 0; k < NPR; k++) p_l[k] = rsh[ty - 1][tx][k];
-      face_finish<1>(P, p_l, l, F1, q1, gF, iz, j, dtij, fail);
-    }
+                                                              DevScalars* __restrict__ ds, int nb1) {
+  const int b = blockIdx.x;
+  flux_shared_body(specialize<LIMC, EOMC, FMC>(P0), P0, pr, F1, F2, q1, q2, gF, ds, b < nb1 ? 1 : 2, b < nb1 ? b : b - nb1);
+}
+
+FluxKernel flux_shared_kernel(const KParams& P) {
+  switch (flux_scheme(P)) {
+    case 1: return k_flux_shared<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>;
+    case 2: return k_flux_shared<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>;
+    case 3: return k_flux_shared<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>;
+    default: return k_flux_shared<-1, -1, -1>;
   }
-  double wm = wave_min(dtij);
-  if ((tx & 63) == 0 && wm < 1.e9) ndt_push(ds, dir, wm, blockIdx);
-  if (fail) atomicOr(&ds->failed, 1);
 }
 
 // corner EMF of flux_ct() (step_ch.c:1223-1234, CORNGDETVERSION=1) from the
@@ -3084,10 +3201,10 @@ static int launch_flux(harm_ctx* c, int pr_sel, int dir0, int ndir, bool fix = t
       break;
     }
     case HARM_FLUX_SHARED: {
-      int gx, gy;
-      flux_shared_grid(c->kp.n1, c->kp.n2, gx, gy);
-      tlaunch(c,k_flux_shared, dim3(gx, gy, ndir), dim3(64, FSH_ROWS), 0, kp,
-                         c->arr[pr_sel], c->arr[HARM_F1], c->arr[HARM_F2], c->q1, c->q2, c->gF, c->ds, dir0);
+      const int nb1 = dir0 == 1 ? flux_shared_blocks(c->kp.n1, c->kp.n2, 1) : 0;
+      const int nb2 = dir0 + ndir > 2 ? flux_shared_blocks(c->kp.n1, c->kp.n2, 2) : 0;
+      tlaunch(c, flux_shared_kernel(kp), dim3(nb1 + nb2), dim3(64, FSH_ROWS), 0, kp, c->arr[pr_sel], c->arr[HARM_F1],
+              c->arr[HARM_F2], c->q1, c->q2, c->gF, c->ds, nb1);
       break;
     }
     default: {
