@@ -502,7 +502,8 @@ static int adj_step(harm_adj* a, int impose, bool store) {
     const bool bnd = bound_in_update(c);  // the step's own boundary schedule
     if (substage(c, pii[to], pbb[to], pff[to], CUf[to], Cunew[to], to, nto, bnd)) return 1;
     if (launch_boundary(c, pff[to],
-                        KB_BOUND | KB_FIXUP | KB_BOUND2 | ((to == nto - 1) ? KB_DT : 0) | (bnd ? KB_INUPDATE : 0)))
+                        KB_BOUND | KB_FIXUP | KB_BOUND2 | ((to == nto - 1) ? KB_DT : 0) | (bnd ? KB_INUPDATE : 0) |
+                            (one_launch(c, pbb[to], pff[to], bnd) ? KB_TAKE : 0)))
       return 1;
     if (store)
       hipLaunchKernelGGL(k_adj_store, dim3(512), dim3(256), 0, c->stream, c->arr[pff[to]], a->seg, a->d_ctr, nto, to,

@@ -93,7 +93,7 @@ __device__ __forceinline__ void ndt_push(DevScalars* __restrict__ ds, int dir, d
 // lane k taking slot k of both directions (one round trip, the minimum by
 // butterflies; a minimum does not depend on its order)
 static_assert(NSTRIPE == 64, "one slot per lane of a wavefront");
-__device__ __forceinline__ void ndt_take_wave(DevScalars* __restrict__ ds, int lane) {
+__device__ __forceinline__ double2 ndt_take_wave(DevScalars* __restrict__ ds, int lane) {
   const unsigned long long big = (unsigned long long)__double_as_longlong(1.e9);
   unsigned long long m[2] = {ds->ndt_acc[0][lane * SSTR], ds->ndt_acc[1][lane * SSTR]};
 #pragma unroll
@@ -105,10 +105,12 @@ __device__ __forceinline__ void ndt_take_wave(DevScalars* __restrict__ ds, int l
     }
     ds->ndt_acc[d][lane * SSTR] = big;
   }
+  const double2 v = make_double2(__longlong_as_double((long long)m[0]), __longlong_as_double((long long)m[1]));
   if (lane == 0) {
-    ds->ndt_last[0] = __longlong_as_double((long long)m[0]);
-    ds->ndt_last[1] = __longlong_as_double((long long)m[1]);
+    ds->ndt_last[0] = v.x;
+    ds->ndt_last[1] = v.y;
   }
+  return v;  // in every lane
 }
 // the first wavefront of workgroup (0, 0) of a zone launch takes them
 __device__ __forceinline__ void ndt_take_first_wave(DevScalars* __restrict__ ds, const dim3 bi) {
@@ -574,28 +576,41 @@ __device__ __forceinline__ int again(int x) {
   return x;
 }
 
-// zone_edges of zone z (stencil stride zs) with para4 in its shorter form where
-// the stencil is finite.  P0 is the context's parameter block, P the one of
-// the kernel's instantiation: the general code below is compiled for P0, with
-// branches on the scheme, which keeps its registers under the fast path's.
+// zone_edges of zone z (stencil stride zs) from its stencil s (s(m, k):
+// component k of its zone m), with para4 in its shorter form where the stencil
+// is finite.  P0 is the context's parameter block, P the one of the kernel's
+// instantiation: the general code below is compiled for P0, with branches on
+// the scheme, which keeps its registers under the fast path's.
+template <class S>
+__device__ __forceinline__ void zone_edges_fast(const KParams& P, const KParams& P0, const double* __restrict__ pr,
+                                                int z, int zs, const S& s, double* l, double* r) {
+  double f = 0.;
+  if (P.lim == 4) {
+#pragma unroll
+    for (int k = 0; k < NPR; k++) para4_fast(s(0, k), s(1, k), s(2, k), s(3, k), s(4, k), l[k], r[k], f);
+  } else {
+#pragma unroll
+    for (int k = 0; k < NPR; k++) {
+      const double dq = (P.lim == 90) ? csslope(k, s(0, k), s(1, k), s(2, k), s(3, k), s(4, k))
+                                      : slope3(P.lim, s(1, k), s(2, k), s(3, k));
+      r[k] = s(2, k) + 0.5 * dq;
+      l[k] = s(2, k) - 0.5 * dq;
+    }
+  }
+  if (__builtin_expect(!(f == 0.), 0)) {
+    double t[5][NPR];
+    z = again(z);
+#pragma unroll
+    for (int m = 0; m < 5; m++) load8(pr, z + (m - 2) * zs, t[m]);
+    zone_edges(P0, t, l, r);
+  }
+}
 __device__ __forceinline__ void zone_edges_fast(const KParams& P, const KParams& P0, const double* __restrict__ pr,
                                                 int z, int zs, double* l, double* r) {
   double s[5][NPR];
 #pragma unroll
   for (int m = 0; m < 5; m++) load8(pr, z + (m - 2) * zs, s[m]);
-  if (P.lim != 4) {
-    zone_edges(P, s, l, r);
-    return;
-  }
-  double f = 0.;
-#pragma unroll
-  for (int k = 0; k < NPR; k++) para4_fast(s[0][k], s[1][k], s[2][k], s[3][k], s[4][k], l[k], r[k], f);
-  if (!(f == 0.)) {
-    z = again(z);
-#pragma unroll
-    for (int m = 0; m < 5; m++) load8(pr, z + (m - 2) * zs, s[m]);
-    zone_edges(P0, s, l, r);
-  }
+  zone_edges_fast(P, P0, pr, z, zs, [&](int m, int k) { return s[m][k]; }, l, r);
 }
 
 // face_finish with the face's flux in its shorter form (the geometry given);
@@ -1079,8 +1094,29 @@ __device__ __forceinline__ void load_cent(const KParams& P, const double* __rest
       [&](int m) { return v[m]; }, gc);
 }
 
-// flux2dUavg (advance.c:204-265): each direction's flux difference, with the
-// flux-CT B fluxes formed from the corner EMFs (step_ch.c:1223-1234, 1405-1412)
+// flux2dUavg (advance.c:204-265): each direction's flux difference from the
+// zone's lower (a) and upper (b) face fluxes, with the flux-CT B fluxes formed
+// from the corner EMFs e (step_ch.c:1223-1234, 1405-1412)
+__device__ __forceinline__ void flux_diff(const KParams& P, double* f1a, double* f1b, double* f2a, double* f2b,
+                                          bool ct, const double (&e)[4], double* d1, double* d2) {
+  if (ct) {  // e00, e01, e10, e11
+    f1a[B1] = 0.;
+    f1a[B2] = 0.5 * (e[0] + e[1]);
+    f1b[B1] = 0.;
+    f1b[B2] = 0.5 * (e[2] + e[3]);
+    f2a[B1] = -0.5 * (e[0] + e[2]);
+    f2a[B2] = 0.;
+    f2b[B1] = -0.5 * (e[1] + e[3]);
+    f2b[B2] = 0.;
+  }
+  const double idx1 = 1.0 / P.dx1, idx2 = 1.0 / P.dx2;
+#pragma unroll
+  for (int k = 0; k < NPR; k++) {
+    d1[k] = (-(f1b[k] - f1a[k]) * idx1);
+    d2[k] = (-(f2b[k] - f2a[k]) * idx2);
+  }
+}
+
 __device__ __forceinline__ void flux_div(const KParams& P, const double* __restrict__ F1,
                                          const double* __restrict__ F2, const double* __restrict__ q1,
                                          const double* __restrict__ q2, const double* __restrict__ gC, int i, int j,
@@ -1091,23 +1127,27 @@ __device__ __forceinline__ void flux_div(const KParams& P, const double* __restr
   load8(F1, zidx(P, i + 1, j), f1b);
   load8(F2, z, f2a);
   load8(F2, zidx(P, i, j + 1), f2b);
-  if (P.fluxb == HARM_FLUXCTTOTH) {
-    double e00 = emf_at(P, q1, q2, gC, i, j), e01 = emf_at(P, q1, q2, gC, i, j + 1),
-           e10 = emf_at(P, q1, q2, gC, i + 1, j), e11 = emf_at(P, q1, q2, gC, i + 1, j + 1);
-    f1a[B1] = 0.;
-    f1a[B2] = 0.5 * (e00 + e01);
-    f1b[B1] = 0.;
-    f1b[B2] = 0.5 * (e10 + e11);
-    f2a[B1] = -0.5 * (e00 + e10);
-    f2a[B2] = 0.;
-    f2b[B1] = -0.5 * (e01 + e11);
-    f2b[B2] = 0.;
+  double e[4] = {0., 0., 0., 0.};
+  const bool ct = P.fluxb == HARM_FLUXCTTOTH;
+  if (ct) {
+    e[0] = emf_at(P, q1, q2, gC, i, j);
+    e[1] = emf_at(P, q1, q2, gC, i, j + 1);
+    e[2] = emf_at(P, q1, q2, gC, i + 1, j);
+    e[3] = emf_at(P, q1, q2, gC, i + 1, j + 1);
   }
-  const double idx1 = 1.0 / P.dx1, idx2 = 1.0 / P.dx2;
+  flux_diff(P, f1a, f1b, f2a, f2b, ct, e, d1, d2);
+}
+
+// RK combination of one zone (dUtoU, advance.c:273-286)
+__device__ __forceinline__ void rk_combine(const RKCoef& C, double dt, const double* Ui, const double* d1,
+                                           const double* d2, const double* dUg, double* ul, double* un, double* Uf) {
 #pragma unroll
   for (int k = 0; k < NPR; k++) {
-    d1[k] = (-(f1b[k] - f1a[k]) * idx1);
-    d2[k] = (-(f2b[k] - f2a[k]) * idx2);
+    double dUr = d1[k] + d2[k];
+    double dtdU = (dUr + dUg[k]);
+    Uf[k] = C.cuf0 * Ui[k] + C.cuf1 * ul[k] + C.cuf2 * dt * dtdU;
+    un[k] += C.cn0 * Ui[k] + C.cn1 * dt * dtdU + C.cn2 * Uf[k];
+    ul[k] = Uf[k];
   }
 }
 
@@ -1182,15 +1222,14 @@ __host__ __device__ __forceinline__ int acct_base(int n1, int n2, int cls) {
   return cls == 0 ? 0 : cls == 1 ? nA : cls == 2 ? nA + nB : cls == 3 ? nA + nB + nC : nA + nB + nC + nD;
 }
 
-// Utoprimgen of U into pf[z] from the guess pin (the pf=pi assignment,
+// Utoprimgen of U into pout from the guess pin (the pf=pi assignment,
 // advance.c:121), fixup1zone (fixup.c:274-377), the zone's pflag and the
 // failed-zone list read by fixup_utoprim; with accounting on, the state
 // before fixup1zone is kept for its events
 __device__ __forceinline__ void invert_zone(const KParams& P, const double* U, const double* pin, const double* gc,
-                                            const GeoU& g, int z, double* __restrict__ pf,
-                                            int* __restrict__ pflag, int* __restrict__ faillist,
-                                            DevScalars* __restrict__ ds, int& niter, int& failz, int& fail) {
-  double pout[NPR];
+                                            const GeoU& g, int z, double* pout, int* __restrict__ pflag,
+                                            int* __restrict__ faillist, DevScalars* __restrict__ ds, int& niter,
+                                            int& failz, int& fail) {
 #pragma unroll
   for (int k = 0; k < NPR; k++) pout[k] = pin[k];
   int pfl = utoprimgen(P, U, gc, pout, niter);
@@ -1217,7 +1256,6 @@ __device__ __forceinline__ void invert_zone(const KParams& P, const double* U, c
     if (fu > pout[UU]) pout[UU] = fu;
   }
   if (limit_gamma(P.gammamax, pout, g) >= 1) fail = 1;
-  store8(pf, z, pout);
 }
 
 // Newton iterations, failed zones and the fatal flag of a wavefront
@@ -1318,21 +1356,15 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
       load8(ulast, z, ul);
       load8(unew, z, un);
     }
-#pragma unroll
-    for (int k = 0; k < NPR; k++) {
-      double dUr = d1[k] + d2[k];
-      // dUtoU (advance.c:273-286)
-      double dtdU = (dUr + dUg[k]);
-      Uf[k] = C.cuf0 * Ui[k] + C.cuf1 * ul[k] + C.cuf2 * dt * dtdU;
-      un[k] += C.cn0 * Ui[k] + C.cn1 * dt * dtdU + C.cn2 * Uf[k];
-      ul[k] = Uf[k];
-    }
+    rk_combine(C, dt, Ui, d1, d2, dUg, ul, un, Uf);
     store8(ulast, z, ul);
     store8(unew, z, un);
     if constexpr (ENO == 1) {
       store8(eA, z, C.last ? un : Uf);
     } else {
-      invert_zone(P, C.last ? un : Uf, pin, gc, g, z, pf, pflag, faillist, ds, niter, failz, fail);
+      double pout[NPR];
+      invert_zone(P, C.last ? un : Uf, pin, gc, g, z, pout, pflag, faillist, ds, niter, failz, fail);
+      store8(pf, z, pout);
       if constexpr (BND == 1) {  // (the edge block's other rows continue below)
         if (near_edge(P, i, j)) {
           double v[NPR];
@@ -1473,7 +1505,9 @@ __global__ __launch_bounds__(256) void k_eno_invert(KParams P, const double* __r
     double pin[NPR], U[NPR];
     load8(pi, z, pin);
     eno_cvt_zone<ENO_A2C, 2>(P, in, i, j, U);
-    invert_zone(P, U, pin, gc, g, z, pf, pflag, faillist, ds, niter, failz, fail);
+    double pout[NPR];
+    invert_zone(P, U, pin, gc, g, z, pout, pflag, faillist, ds, niter, failz, fail);
+    store8(pf, z, pout);
   }
   count_zone(ds, niter, failz, fail, blockIdx);
 }
@@ -1820,12 +1854,13 @@ constexpr int KB_BOUND = 1;     // bound_prim()
 constexpr int KB_FIXUP = 2;     // post_fixup(): bound_pflag + fixup_utoprim on the failed-zone list
 constexpr int KB_BOUND2 = 8;    // bound_prim() after the fixup (step_ch.c:124)
 constexpr int KB_DT = 4;        // t,dt update (step_ch.c:174-183)
+constexpr int KB_TAKE = 32;     // the Courant limits taken here (k_substage formed them)
 constexpr int KB_INUPDATE = 16; // the first bound_prim() done by k_update (HARM_BOUND_INUPDATE)
 
 // step_ch.c:174-183 with advance.c:190: the new dt from the last substage's
 // Courant limits, clipped to SAFE*dt and to tf
-__device__ inline void dt_update(const KParams& P, DevScalars* ds) {
-  double ndt = P.defcon * 1. / (1. / ds->ndt_last[0] + 1. / ds->ndt_last[1]);
+__device__ inline void dt_update(const KParams& P, DevScalars* ds, double ndt1, double ndt2) {
+  double ndt = P.defcon * 1. / (1. / ndt1 + 1. / ndt2);
   double dt = ds->dt;
   ds->dt_step = dt;
   ds->t += dt;
@@ -1833,6 +1868,10 @@ __device__ inline void dt_update(const KParams& P, DevScalars* ds) {
   dt = ndt;
   if (ds->t + dt > ds->tf) dt = ds->tf - ds->t;
   ds->dt = dt;
+}
+
+__device__ inline void dt_update(const KParams& P, DevScalars* ds) {
+  dt_update(P, ds, ds->ndt_last[0], ds->ndt_last[1]);
 }
 
 // Everything between two advance() calls, as one workgroup with barriers
@@ -2120,13 +2159,21 @@ template <bool FIX>
 __global__ __launch_bounds__(256) void k_fixbound(KParams P, double* __restrict__ pv, int* __restrict__ pflag,
                                                   const int* __restrict__ faillist, double* __restrict__ pfix,
                                                   const double* __restrict__ gC, DevScalars* __restrict__ ds,
-                                                  int do_dt) {
+                                                  int do_dt, int take) {
   __shared__ double keep[FIX ? FIXKEEP * NPR : 1];
   __shared__ int keepz[FIX ? FIXKEEP : 1];
   __shared__ int corner_fixed[4];  // pole-row edge zone e is on the list: its images are the list's
-  // the t, dt update after the last substage reads only the step's scalars:
-  // one thread of the last wavefront, beside the repair
-  if (do_dt && threadIdx.x == blockDim.x - 1) dt_update(P, ds);
+  // the substage's Courant limits (take: k_substage's, k_update took its own)
+  // and the t, dt update after the last substage read only the step's
+  // scalars: the last wavefront, beside the repair
+  if (threadIdx.x >= blockDim.x - 64) {
+    if (take) {
+      const double2 ndt = ndt_take_wave(ds, threadIdx.x & 63);
+      if (do_dt && threadIdx.x == blockDim.x - 1) dt_update(P, ds, ndt.x, ndt.y);
+    } else if (do_dt && threadIdx.x == blockDim.x - 1) {
+      dt_update(P, ds);
+    }
+  }
   const int cap = P.n1 * P.n2;
   int n = FIX ? ds->nlist : 0, fail = 0;
   // the list's first entries read beside its length (used only below n)
@@ -2590,6 +2637,9 @@ __global__ void k_pflag_expand(int nz, const int* __restrict__ pf, const int* __
   out[(size_t)z * 5 + 3] = bsqf[z] >> 8;       // FLAGBSQOU
   out[(size_t)z * 5 + 4] = 0;                  // FLAGREALFLUX (FLUXADJUST=0)
 }
+
+
+#include "harm_substage.inl"
 
 
 // ---------------------------------------------------------------------------
@@ -3301,13 +3351,13 @@ static int launch_boundary(harm_ctx* c, int sel, int mode) {
   }
   if (prof_begin(c, HARM_K_BOUNDARY)) return 1;
   if (mode & KB_INUPDATE) {  // the first bound_prim() was k_update's
-    const int do_dt = (mode & KB_DT) ? 1 : 0;
+    const int do_dt = (mode & KB_DT) ? 1 : 0, take = (mode & KB_TAKE) ? 1 : 0;
     if (mode & KB_FIXUP) {
       tlaunch(c, k_fixbound<true>, dim3(1), dim3(256), 0, c->kp, c->arr[sel], c->pflag, c->faillist, c->pfix,
-              c->gC, c->ds, do_dt);
+              c->gC, c->ds, do_dt, take);
     } else if ((mode & KB_BOUND2) || do_dt) {
       tlaunch(c, k_fixbound<false>, dim3(1), dim3(256), 0, c->kp, c->arr[sel], c->pflag, c->faillist, c->pfix,
-              c->gC, c->ds, do_dt);
+              c->gC, c->ds, do_dt, take);
     }
   } else if (c->bound_variant == HARM_BOUND_BLOCK && !c->kp.checksolution) {
     tlaunch(c,k_boundary, dim3(1), dim3(1024), 0, c->kp, c->arr[sel], c->gC, c->pflag,
@@ -3403,6 +3453,20 @@ static void rk_setup(int timeorder, int* nto, double CUf[4][3], double Cunew[4][
   }
 }
 
+// fluxes and update of a substage with the in-update fill in one launch
+// (k_substage): the zone-shared fluxes with that fill, the states' array not
+// the one written (neighbouring tiles read it meanwhile: RK1 writes it).  Up to
+// two tiles a compute unit, which run beside each other: above, a second turn
+// begins and the rim's arithmetic costs more than the traffic it saves.
+// Measured, us a substage with its repair, torus, against two launches: 32x64
+// 20.8 (26.4), 97x131 20.8 (27.5), 128x128 21.5 (28.7), 144x144 27.4 (31.0),
+// 128x256 (512 tiles) 29.8 (36.8); past the line 192x192 39.5 (37.1), 256x256
+// 48.8 (45.3), 512x512 173 (139).  Not while the stages are timed one by one.
+static bool one_launch(const harm_ctx* c, int pb, int pf, bool bnd) {
+  const int nt = ((c->kp.n1 + tile::TI - 1) / tile::TI) * ((c->kp.n2 + tile::TJ - 1) / tile::TJ);
+  return bnd && c->flux_variant == HARM_FLUX_SHARED && pb != pf && !c->prof && nt <= 2 * 256;
+}
+
 // advance(): fluxcalc both directions (+ fix_flux, flux_ct formed in k_update), update
 static int substage(harm_ctx* c, int pi, int pb, int pf, const double* CUf, const double* Cunew, int to, int nto,
                     bool bnd = false) {
@@ -3411,6 +3475,14 @@ static int substage(harm_ctx* c, int pi, int pb, int pf, const double* CUf, cons
   C.cn0 = Cunew[0]; C.cn1 = Cunew[1]; C.cn2 = Cunew[2];
   C.timeorder = to;
   C.last = (to == nto - 1);
+  if (one_launch(c, pb, pf, bnd)) {
+    const int nti = (c->kp.n1 + tile::TI - 1) / tile::TI, ntj = (c->kp.n2 + tile::TJ - 1) / tile::TJ;
+    hipLaunchKernelGGL(substage_kernel(c->kp), dim3((nti * ntj + 7) / 8 * 8), dim3(64 * tile::NW), 0, c->stream, c->kp,
+                       C, c->arr[pi], c->arr[pb], c->arr[pf], c->arr[HARM_ULAST], c->arr[HARM_UNEW], c->arr[HARM_F1],
+                       c->arr[HARM_F2], c->q1, c->q2, c->gF, c->gC, c->gConn, c->pflag, c->faillist, c->ds, nti, ntj);
+    HIPCHK(hipGetLastError());
+    return 0;
+  }
   if (launch_flux(c, pb, 1, 2)) return 1;
   if (launch_update(c, pi, pb, pf, C, bnd)) return 1;
   return 0;
@@ -3440,7 +3512,8 @@ static int enqueue_step(harm_ctx* c) {
     if (substage(c, pii[to], pbb[to], pff[to], CUf[to], Cunew[to], to, nto, bnd)) return 1;
     if (acct && acct_zones(c, to == nto - 1)) return 1;
     // step_ch.c:104-124 bound_prim, post_fixup, bound_prim; then :174-183 after the last substage
-    int mode = KB_BOUND | KB_FIXUP | KB_BOUND2 | ((to == nto - 1) ? KB_DT : 0) | (bnd ? KB_INUPDATE : 0);
+    int mode = KB_BOUND | KB_FIXUP | KB_BOUND2 | ((to == nto - 1) ? KB_DT : 0) | (bnd ? KB_INUPDATE : 0) |
+               (one_launch(c, pbb[to], pff[to], bnd) ? KB_TAKE : 0);
     if (launch_boundary(c, pff[to], mode)) return 1;
     if (acct && acct_merge(c, to == nto - 1)) return 1;
   }

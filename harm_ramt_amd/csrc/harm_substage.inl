@@ -1,0 +1,328 @@
+// harm_substage.inl -- fluxcalc() and advance() of one substage in one launch
+// (included by harm_kernels.hip, inside its namespace).
+//
+// A workgroup of four wavefronts takes a tile of 8 x 8 zones.  With the zones'
+// states and three more around them in LDS it forms the edge states of the
+// tile and one zone around it, the fluxes and EMF quotients of every face that
+// its zones and their corners need (those on the rim are formed by the
+// neighbouring tile too), and from them the update of k_update<0, ., 1>, the
+// first bound_prim() included: the functions, so the bits, of k_flux_shared and
+// k_update.  What it saves is the fluxes' way through memory (F1, F2, q1, q2
+// written and read, the states read again: 310 of 1,620 bytes a zone and
+// substage), a launch, and on small grids the wait for one wavefront's chain of
+// a zone's whole update: U(pi) and the source term are formed beside it.  What
+// it costs is the rim, 100 edge and face tasks a direction for 64 zones.  F1,
+// F2 and the quotients are written by the step's last substage alone, which
+// leaves them as a step always does.
+//
+// A wavefront takes 64 zones of one direction, their edges in a first pass and
+// their lower faces in a second: two wavefronts a direction, the second of them
+// with 36 zones.  Then the last does the update of the 64 zones and the two
+// before it the update's parts that need no flux.  Bound by the issue of 64-bit
+// arithmetic (9,000 wave instructions on the longest chain, 4.5 cycles each),
+// so by the number of workgroups a compute unit has to take: two fit beside
+// each other (194 registers, 40 KB of LDS), and fill each other's waits.
+namespace tile {
+constexpr int TI = 8, TJ = 8, NW = 4;
+constexpr int HI = TI + 2, HJ = TJ + 2, NZH = HI * HJ;              // zones with edges
+constexpr int PI = TI + 2 * NG, PJ = TJ + 2 * NG, NZP = PI * PJ;    // zones with states
+constexpr int WD = (NZH + 63) / 64, NTASK = 2 * WD;                 // tasks a direction, in all
+constexpr int NZT = TI * TJ;
+static_assert(NZT == 64 && NTASK == NW, "one wavefront a task, one for the update");
+}  // namespace tile
+
+// the fix_flux rules of a face's own flux (face_store applies them too)
+template <int DIR>
+__device__ __forceinline__ void face_rules(const KParams& P, double* Fo, int i, int j) {
+  if (!P.fixupflux) return;
+  if (DIR == 1) {
+    if (i == 0 && P.bc[HARM_X1DN] == HARM_OUTFLOW && j < P.n2 && Fo[RHO] > 0) Fo[RHO] = 0;
+    if (i == P.n1 && P.bc[HARM_X1UP] == HARM_OUTFLOW && j < P.n2 && Fo[RHO] < 0) Fo[RHO] = 0;
+  } else {
+    const bool polar_dn = (j == 0 && P.bc[HARM_X2DN] == HARM_POLARAXIS && i < P.n1);
+    const bool polar_up = (j == P.n2 && P.bc[HARM_X2UP] == HARM_POLARAXIS && i < P.n1);
+    const bool equator = (i >= 0 && i < P.n1 && j == (P.n2 - 1) / 2);
+    if (polar_dn || polar_up || equator) {
+#pragma unroll
+      for (int k = 0; k < NPR; k++)
+        if (k != U2) Fo[k] = 0.;
+    }
+  }
+}
+
+// a face's flux from its two states, by the general functions where the
+// shorter form does not hold
+template <int DIR>
+__device__ __forceinline__ void face_value(const KParams& P, const KParams& P0, const double* p_l, const double* p_r,
+                                           const double* __restrict__ pb, const double* __restrict__ gF, int i, int j,
+                                           double (&Fo)[NPR], double& gdet, double& cm, double& dtij, int& fail) {
+  GeoU g;
+  load_geo_face(P, gF, zidx(P, i, j), g);
+  gdet = g.gdet;
+  if (__builtin_expect(!face_flux_fast<DIR>(P, p_l, p_r, g, Fo, cm, fail), 0)) {
+    cm = 0.;
+    double a[NPR], b[NPR];
+    const int i2 = again(i);
+    face_recon<DIR>(P0, pb, i2, j, a, b);
+    load_geo_face(P0, gF, zidx(P0, i2, j), g);
+    face_flux<DIR>(P0, a, b, g, Fo, dtij, fail);
+  }
+}
+
+template <int LIMC, int EOMC, int FMC>
+__global__ __launch_bounds__(64 * tile::NW) void k_substage(
+    KParams P0, RKCoef C, const double* pi, const double* __restrict__ pb, double* pf, double* __restrict__ ulast,
+    double* __restrict__ unew, double* __restrict__ F1, double* __restrict__ F2, double* __restrict__ q1,
+    double* __restrict__ q2, const double* __restrict__ gF, const double* __restrict__ gC,
+    const double* __restrict__ gConn, int* __restrict__ pflag, int* __restrict__ faillist, DevScalars* __restrict__ ds,
+    int nti, int ntj) {
+  using namespace tile;
+  const KParams P = specialize<LIMC, EOMC, FMC>(P0);
+  // neighbouring tiles on one XCD (workgroups go round over the eight), so
+  // that its L2 serves the rims
+  const int nt = nti * ntj, per = (nt + 7) / 8, tl = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (tl >= nt) return;
+  const int i0 = (tl / ntj) * TI, j0 = (tl % ntj) * TJ;
+  __shared__ double sp[NPR][NZP];        // the states, from (i0-3, j0-3)
+  __shared__ double sl[2][NPR][NZH];     // lower edge states from (i0-1, j0-1), then the lower faces' fluxes
+  __shared__ double sr[2][NPR][NZH];     // upper edge states
+  __shared__ double sq[2][NZH];          // the faces' EMF quotients
+  __shared__ double sm[2][HI];       // F1's mirrored across the poles, columns j = -1 and N2
+  __shared__ double smax[NTASK];     // largest speed of each task
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int fail = 0;
+  {
+    constexpr int NL = (NZP * 4 + 64 * NW - 1) / (64 * NW);
+    double2 t[NL];
+#pragma unroll
+    for (int m = 0; m < NL; m++) {
+      const int x = min(tid + 64 * NW * m, NZP * 4 - 1), z = x >> 2;
+      const int zi = min(i0 - NG + z / PJ, P.n1 + NG - 1), zj = min(j0 - NG + z % PJ, P.n2 + NG - 1);
+      t[m] = reinterpret_cast<const double2*>(pb)[(size_t)zidx(P, zi, zj) * 4 + (x & 3)];
+    }
+#pragma unroll
+    for (int m = 0; m < NL; m++) {
+      const int x = tid + 64 * NW * m;
+      if (x < NZP * 4) {
+        sp[2 * (x & 3)][x >> 2] = t[m].x;
+        sp[2 * (x & 3) + 1][x >> 2] = t[m].y;
+      }
+    }
+  }
+  __syncthreads();
+  // edge states
+  const int d = w >= WD, eid = 64 * (w - d * WD) + lane;  // this lane's edge zone and direction
+  const int hi = eid / HJ, hj = eid % HJ, ei = i0 - 1 + hi, ej = j0 - 1 + hj;
+  const bool edge = eid < NZH && ei <= P.n1 && ej <= P.n2;
+  if (edge) {
+    const int c = (hi + 2) * PJ + hj + 2, st = d ? 1 : PJ;
+    double l[NPR], r[NPR];
+    zone_edges_fast(P, P0, pb, zidx(P, ei, ej), d ? 1 : P.N2M, [&](int m, int k) { return sp[k][c + (m - 2) * st]; }, l, r);
+#pragma unroll
+    for (int k = 0; k < NPR; k++) {
+      sl[d][k][eid] = l[k];
+      sr[d][k][eid] = r[k];
+    }
+  }
+  __syncthreads();
+  // the zones' lower faces
+  double cm = 0., dtij = 1.e9;
+  if (edge && (d ? hj : hi) >= 1) {
+    double p_l[NPR], p_r[NPR], Fo[NPR], gdet;
+#pragma unroll
+    for (int k = 0; k < NPR; k++) {
+      p_l[k] = sr[d][k][eid - (d ? 1 : HJ)];
+      p_r[k] = sl[d][k][eid];
+    }
+    // the tile that holds the face's zone (the nearest, outside the grid) writes it
+    const bool own = C.last && max(0, min(ei, P.n1 - 1)) / TI * TI == i0 && max(0, min(ej, P.n2 - 1)) / TJ * TJ == j0;
+    if (d == 0) {
+      face_value<1>(P, P0, p_l, p_r, pb, gF, ei, ej, Fo, gdet, cm, dtij, fail);
+      face_rules<1>(P, Fo, ei, ej);
+      sq[0][eid] = Fo[B2] / gdet;
+      if (P.fixupflux && ei < P.n1) {
+        if (ej == 0 && P.bc[HARM_X2DN] == HARM_POLARAXIS) sm[0][hi] = (-Fo[B2]) / face_gdet(P, gF, zidx(P, ei, -1));
+        if (ej == P.n2 - 1 && P.bc[HARM_X2UP] == HARM_POLARAXIS)
+          sm[1][hi] = (-Fo[B2]) / face_gdet(P, gF, zidx(P, ei, P.n2));
+      }
+      if (own) face_store<1>(P, Fo, gdet, F1, q1, gF, ei, ej);
+    } else {
+      const double* gF2 = gF + (size_t)P.nz * GF;
+      face_value<2>(P, P0, p_l, p_r, pb, gF2, ei, ej, Fo, gdet, cm, dtij, fail);
+      face_rules<2>(P, Fo, ei, ej);
+      sq[1][eid] = Fo[B1] / gdet;
+      if (own) face_store<2>(P, Fo, gdet, F2, q2, gF2, ei, ej);
+    }
+#pragma unroll
+    for (int k = 0; k < NPR; k++) sl[d][k][eid] = Fo[k];
+  }
+  cm = wave_max_dpp(cm);
+  if (lane == 63) smax[w] = cm;
+  if (dtij < 1.e9) ndt_push(ds, d + 1, dtij, dim3(tl, 0, 0));
+  __syncthreads();
+  if (tid < 2) {  // the tile's Courant limits (k_flux_shared: from the largest speeds)
+    double cw = 0.;
+    for (int m = 0; m < WD; m++) cw = dmax(smax[tid * WD + m], cw);
+    const double dt = P.cour * ((tid == 0) ? P.dx1 : P.dx2) / cw;
+    if (dt < 1.e9) ndt_push(ds, tid + 1, dt, dim3(tl, 0, 0));
+  }
+  // outflow edge rows in this tile: their zones' values go to LDS, for the
+  // whole workgroup to form the x1 ghost columns from them
+  const bool edge_dn = i0 == 0 && P.bc[HARM_X1DN] == HARM_OUTFLOW;
+  const bool edge_up = i0 + TI >= P.n1 && P.bc[HARM_X1UP] == HARM_OUTFLOW;
+  double (*ev)[NPR] = reinterpret_cast<double (*)[NPR]>(&sr[0][0][0]);  // [2 TJ][NPR]
+  static_assert(2 * TJ <= 2 * NZH, "the edge rows' values fit where the edge states were");
+  // the update's parts that need no flux, U(pi) and the source term, by the two
+  // wavefronts before the last, to LDS
+  double (*pu)[NZT] = reinterpret_cast<double (*)[NZT]>(&sr[0][0][0] + 2 * TJ * NPR);  // [8 + 4]
+  static_assert(2 * TJ * NPR + 12 * NZT <= 2 * NPR * NZH, "the rows' values and the parts fit where the edge states were");
+  const int zi = lane / TJ, zj = lane % TJ, i = i0 + zi, j = j0 + zj;
+  const int z = zidx(P, min(i, P.n1 - 1), min(j, P.n2 - 1));
+  const bool zone = i < P.n1 && j < P.n2;
+  const int h = (zi + 1) * HJ + zj + 1;
+  if ((w == NW - 3 || w == NW - 2) && zone) {
+    double gc[36], v[NPR];
+    load_cent(P, gC, z, gc);
+    GeoU g;
+    geo_from_cent(gc, g);
+    if (w == NW - 3) {  // T^j_k Gamma^k_{lj} contraction (phys.c:475-619)
+      double pbz[NPR];
+#pragma unroll
+      for (int k = 0; k < NPR; k++) pbz[k] = sp[k][(zi + NG) * PJ + zj + NG];
+      source_conn_at(P, pbz, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, v);
+#pragma unroll
+      for (int k = 0; k < 4; k++) pu[8 + k][lane] = v[UU + k];
+    } else {
+      State q;
+      double pin[NPR];
+      load8(pi, z, pin);
+      get_state(pin, g, q);
+      primtoflux(P, pin, q, 0, g.gdet, v);
+#pragma unroll
+      for (int k = 0; k < NPR; k++) pu[k][lane] = v[k];
+    }
+  }
+  int niter = 0, failz = 0;
+  double gc[36], pin[NPR], ul[NPR], un[NPR], d1[NPR], d2[NPR];
+  GeoU g;
+  const bool upd = w == NW - 1;
+  if (upd && zone) {
+    load_cent(P, gC, z, gc);
+    geo_from_cent(gc, g);
+    load8(pi, z, pin);
+    if (C.timeorder == 0) {
+#pragma unroll
+      for (int k = 0; k < NPR; k++) ul[k] = un[k] = 0.0;
+    } else {
+      load8(ulast, z, ul);
+      load8(unew, z, un);
+    }
+    double f1a[NPR], f1b[NPR], f2a[NPR], f2b[NPR], e[4] = {0., 0., 0., 0.};
+#pragma unroll
+    for (int k = 0; k < NPR; k++) {
+      f1a[k] = sl[0][k][h];
+      f1b[k] = sl[0][k][h + HJ];
+      f2a[k] = sl[1][k][h];
+      f2b[k] = sl[1][k][h + 1];
+    }
+    const bool ct = P.fluxb == HARM_FLUXCTTOTH;
+    if (ct) {
+      const bool mdn = P.fixupflux && P.bc[HARM_X2DN] == HARM_POLARAXIS;
+      const bool mup = P.fixupflux && P.bc[HARM_X2UP] == HARM_POLARAXIS;
+      auto emf = [&](int a, int b) {  // at corner (i+a, j+b)
+        const int m = h + a * HJ + b;
+        double qa = sq[0][m], qb = sq[0][m - 1];
+        if (i + a < P.n1) {
+          if (mdn && j + b == 0) qb = sm[0][zi + 1 + a];
+          if (mup && j + b == P.n2) qa = sm[1][zi + 1 + a];
+        }
+        return 0.25 * geo_entry(P, gC, GC_GDETC, z + a * P.N2M + b) * (qa + qb - sq[1][m] - sq[1][m - HJ]);
+      };
+      e[0] = emf(0, 0);
+      e[1] = emf(0, 1);
+      e[2] = emf(1, 0);
+      e[3] = emf(1, 1);
+    }
+    flux_diff(P, f1a, f1b, f2a, f2b, ct, e, d1, d2);
+  }
+  __syncthreads();
+  if (upd) {
+    if (zone) {
+      double Ui[NPR], dUg[NPR], Uf[NPR], pout[NPR];
+#pragma unroll
+      for (int k = 0; k < NPR; k++) Ui[k] = pu[k][lane];
+      dUg[RHO] = dUg[B1] = dUg[B2] = dUg[B3] = g.gdet * 0.;
+#pragma unroll
+      for (int k = 0; k < 4; k++) dUg[UU + k] = pu[8 + k][lane];
+      rk_combine(C, ds->dt, Ui, d1, d2, dUg, ul, un, Uf);
+      store8(ulast, z, ul);
+      store8(unew, z, un);
+      invert_zone(P, C.last ? un : Uf, pin, gc, g, z, pout, pflag, faillist, ds, niter, failz, fail);
+      // the first bound_prim(): this zone's images, but for the outflow columns
+      if (near_edge(P, i, j)) {
+        const bool hdn = edge_dn && i == 0, hup = edge_up && i == P.n1 - 1;
+        for (int part = 0; part < NIMG; part++)
+          if (!(part > 0 && (part > NG ? hup : hdn))) bound_image_part(P, pf, gC, i, j, pout, part, fail);
+        if (hdn) {
+#pragma unroll
+          for (int k = 0; k < NPR; k++) ev[zj][k] = pout[k];
+        }
+        if (hup) {
+#pragma unroll
+          for (int k = 0; k < NPR; k++) ev[TJ + zj][k] = pout[k];
+        }
+        if (pole_row(P, j)) {  // POLEDEATH of the pole row, after its images
+          pout[U2] *= 0.;
+          pout[B2] *= 0.;
+        }
+      }
+      store8(pf, z, pout);
+    }
+    count_zone(ds, niter, failz, fail, dim3(tl, 0, 0));
+    fail = 0;
+  }
+  if (edge_dn || edge_up) {  // block-uniform
+    __syncthreads();
+    for (int x = tid; x < 2 * NG * TJ; x += 64 * NW) {  // the outflow columns of the edge rows
+      const int up = x / (NG * TJ), g = x / TJ % NG, zj = x % TJ, j = j0 + zj;
+      if (!(up ? edge_up : edge_dn) || j >= P.n2) continue;
+      double v[NPR];
+#pragma unroll
+      for (int k = 0; k < NPR; k++) v[k] = ev[up * TJ + zj][k];
+      bound_image_part(P, pf, gC, up ? P.n1 - 1 : 0, j, v, (up ? NG + 1 : 1) + g, fail);
+    }
+    // the second bound_prim()'s values of the pole rows' outflow columns, from
+    // the rows after POLEDEATH (DevScalars::pole_x1): the last threads
+    const int x = 64 * NW - 1 - tid;
+    if (x < 4 * NG && P.n1 >= 5) {
+      const int e = x / NG, g = x % NG, up = e & 1, jp = (e & 2) ? P.n2 - 1 : 0;
+      if ((up ? edge_up : edge_dn) && jp >= j0 && jp < j0 + TJ && pole_row(P, jp)) {
+        double v[NPR];
+#pragma unroll
+        for (int k = 0; k < NPR; k++) v[k] = ev[up * TJ + jp - j0][k];
+        int f2 = 0;
+        v[U2] *= 0.;
+        v[B2] *= 0.;
+        x1_value(P, gC, up ? P.n1 + g : -1 - g, jp, v, f2);
+        v[U2] *= 0.;
+        v[B2] *= 0.;
+#pragma unroll
+        for (int k = 0; k < NPR; k++) ds->pole_x1[e][g][k] = v[k];
+        ds->pole_fail[e][g] = f2;
+      }
+    }
+  }
+  if (fail) atomicOr(&ds->failed, 1);
+}
+
+using SubstageKernel = void (*)(KParams, RKCoef, const double*, const double*, double*, double*, double*, double*,
+                                double*, double*, double*, const double*, const double*, const double*, int*, int*,
+                                DevScalars*, int, int);
+SubstageKernel substage_kernel(const KParams& P) {
+  switch (flux_scheme(P)) {
+    case 1: return k_substage<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>;
+    case 2: return k_substage<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>;
+    case 3: return k_substage<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>;
+    default: return k_substage<-1, -1, -1>;
+  }
+}
