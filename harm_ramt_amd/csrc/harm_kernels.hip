@@ -2156,10 +2156,10 @@ __global__ __launch_bounds__(1024) void k_fixall(KParams P, double* __restrict__
 // it is.  Then the t,dt update after the last substage.
 constexpr int FIXKEEP = 512;
 template <bool FIX>
-__global__ __launch_bounds__(256) void k_fixbound(KParams P, double* __restrict__ pv, int* __restrict__ pflag,
-                                                  const int* __restrict__ faillist, double* __restrict__ pfix,
-                                                  const double* __restrict__ gC, DevScalars* __restrict__ ds,
-                                                  int do_dt, int take) {
+__device__ __forceinline__ void fixbound_body(const KParams& P, double* __restrict__ pv, int* __restrict__ pflag,
+                                              const int* __restrict__ faillist, double* __restrict__ pfix,
+                                              const double* __restrict__ gC, DevScalars* __restrict__ ds,
+                                              int do_dt, int take) {
   __shared__ double keep[FIX ? FIXKEEP * NPR : 1];
   __shared__ int keepz[FIX ? FIXKEEP : 1];
   __shared__ int corner_fixed[4];  // pole-row edge zone e is on the list: its images are the list's
@@ -2248,6 +2248,13 @@ __global__ __launch_bounds__(256) void k_fixbound(KParams P, double* __restrict_
   }
   if (fail) atomicOr(&ds->failed, 1);
   if (FIX && threadIdx.x == 0) ds->nlist = 0;  // every thread read nlist before the barrier
+}
+template <bool FIX>
+__global__ __launch_bounds__(256) void k_fixbound(KParams P, double* __restrict__ pv, int* __restrict__ pflag,
+                                                  const int* __restrict__ faillist, double* __restrict__ pfix,
+                                                  const double* __restrict__ gC, DevScalars* __restrict__ ds,
+                                                  int do_dt, int take) {
+  fixbound_body<FIX>(P, pv, pflag, faillist, pfix, gC, ds, do_dt, take);
 }
 
 // ---- bound_prim() with the general rules: the outflow extrapolation
@@ -2692,6 +2699,68 @@ __global__ void kb_bx2(const RunDesc* __restrict__ runs, const int4* __restrict_
   const int4 e = tab[blockIdx.x];
   const RunDesc& r = runs[e.x];
   bx2_body(r.P, r.arr[sel], r.ds, do_dt, dim3(e.y, e.z, e.w), dim3(0, 0, 0));
+}
+
+// the zone-shared fluxes (table: run, block, direction), the update with the
+// in-update fill, both of them in one launch (table: run, tile), and the rest
+// of the substage, a workgroup a run
+template <int LIMC, int EOMC, int FMC>
+__global__ __launch_bounds__(64 * FSH_ROWS) void kb_flux_shared(const RunDesc* __restrict__ runs,
+                                                               const int4* __restrict__ tab, int pr_sel) {
+  const int4 e = tab[blockIdx.x];
+  const RunDesc& r = runs[e.x];
+  const KParams P0 = r.P;
+  flux_shared_body(specialize<LIMC, EOMC, FMC>(P0), P0, r.arr[pr_sel], r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gF,
+                   r.ds, e.z, e.y);
+}
+
+template <int LIMC, int EOMC, int FMC>
+__global__ __launch_bounds__(256) void kb_update_fill(const RunDesc* __restrict__ runs, const int4* __restrict__ tab,
+                                                      RKCoef C, int pi, int pb, int pf) {
+  const int4 e = tab[blockIdx.x];
+  const RunDesc& r = runs[e.x];
+  update_body<0, 1>(specialize<LIMC, EOMC, FMC>(r.P), C, r.arr[pi], r.arr[pb], r.arr[pf], r.arr[HARM_ULAST],
+                    r.arr[HARM_UNEW], r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gC, r.gConn, r.pflag, r.faillist,
+                    r.ds, nullptr, nullptr, dim3(e.y, e.z, e.w), dim3(0, 0, 0));
+}
+
+template <int LIMC, int EOMC, int FMC>
+__global__ __launch_bounds__(64 * tile::NW) void kb_substage(const RunDesc* __restrict__ runs,
+                                                            const int4* __restrict__ tab, RKCoef C, int pi, int pb,
+                                                            int pf) {
+  const int4 e = tab[blockIdx.x];
+  const RunDesc& r = runs[e.x];
+  const KParams P0 = r.P;
+  substage_body<LIMC, EOMC, FMC>(P0, C, r.arr[pi], r.arr[pb], r.arr[pf], r.arr[HARM_ULAST], r.arr[HARM_UNEW],
+                                 r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gF, r.gC, r.gConn, r.pflag, r.faillist,
+                                 r.ds, (P0.n2 + tile::TJ - 1) / tile::TJ, e.y);
+}
+
+__global__ __launch_bounds__(256) void kb_fixbound(const RunDesc* __restrict__ runs, int sel, int do_dt, int take) {
+  const RunDesc& r = runs[blockIdx.x];
+  if (r.P.eomtype == HARM_EOMGRMHD)
+    fixbound_body<true>(r.P, r.arr[sel], r.pflag, r.faillist, r.pfix, r.gC, r.ds, do_dt, take);
+  else
+    fixbound_body<false>(r.P, r.arr[sel], r.pflag, r.faillist, r.pfix, r.gC, r.ds, do_dt, take);
+}
+
+// a batch's kernels for its runs' scheme (0: not one scheme, the general ones)
+struct BatchKernels {
+  void (*flux)(const RunDesc*, const int4*, int);
+  void (*update)(const RunDesc*, const int4*, RKCoef, int, int, int);
+  void (*one)(const RunDesc*, const int4*, RKCoef, int, int, int);
+};
+template <int LIMC, int EOMC, int FMC>
+BatchKernels batch_kernels_of() {
+  return {kb_flux_shared<LIMC, EOMC, FMC>, kb_update_fill<-1, EOMC, -1>, kb_substage<LIMC, EOMC, FMC>};
+}
+BatchKernels batch_kernels(int scheme) {
+  switch (scheme) {
+    case 1: return batch_kernels_of<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>();
+    case 2: return batch_kernels_of<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>();
+    case 3: return batch_kernels_of<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>();
+    default: return batch_kernels_of<-1, -1, -1>();
+  }
 }
 
 // failed-list kernels: FIXBLK blocks per run, block b of run r is blockIdx.x = r*FIXBLK+b
@@ -3462,9 +3531,12 @@ static void rk_setup(int timeorder, int* nto, double CUf[4][3], double Cunew[4][
 // 20.8 (26.4), 97x131 20.8 (27.5), 128x128 21.5 (28.7), 144x144 27.4 (31.0),
 // 128x256 (512 tiles) 29.8 (36.8); past the line 192x192 39.5 (37.1), 256x256
 // 48.8 (45.3), 512x512 173 (139).  Not while the stages are timed one by one.
+constexpr int ONE_LAUNCH_TILES = 2 * 256;
+static int tile_count(const KParams& P) {
+  return ((P.n1 + tile::TI - 1) / tile::TI) * ((P.n2 + tile::TJ - 1) / tile::TJ);
+}
 static bool one_launch(const harm_ctx* c, int pb, int pf, bool bnd) {
-  const int nt = ((c->kp.n1 + tile::TI - 1) / tile::TI) * ((c->kp.n2 + tile::TJ - 1) / tile::TJ);
-  return bnd && c->flux_variant == HARM_FLUX_SHARED && pb != pf && !c->prof && nt <= 2 * 256;
+  return bnd && c->flux_variant == HARM_FLUX_SHARED && pb != pf && !c->prof && tile_count(c->kp) <= ONE_LAUNCH_TILES;
 }
 
 // advance(): fluxcalc both directions (+ fix_flux, flux_ct formed in k_update), update
@@ -3479,7 +3551,7 @@ static int substage(harm_ctx* c, int pi, int pb, int pf, const double* CUf, cons
     const int nti = (c->kp.n1 + tile::TI - 1) / tile::TI, ntj = (c->kp.n2 + tile::TJ - 1) / tile::TJ;
     hipLaunchKernelGGL(substage_kernel(c->kp), dim3((nti * ntj + 7) / 8 * 8), dim3(64 * tile::NW), 0, c->stream, c->kp,
                        C, c->arr[pi], c->arr[pb], c->arr[pf], c->arr[HARM_ULAST], c->arr[HARM_UNEW], c->arr[HARM_F1],
-                       c->arr[HARM_F2], c->q1, c->q2, c->gF, c->gC, c->gConn, c->pflag, c->faillist, c->ds, nti, ntj);
+                       c->arr[HARM_F2], c->q1, c->q2, c->gF, c->gC, c->gConn, c->pflag, c->faillist, c->ds, nti * ntj, ntj);
     HIPCHK(hipGetLastError());
     return 0;
   }
@@ -3938,7 +4010,7 @@ extern "C" int harm_get_tuning(harm_ctx* c, int* flux_variant, int* bound_varian
 // ===========================================================================
 // Batched runs (C-ABI): contexts advanced together, one launch per stage
 // ===========================================================================
-enum { BT_FLUX4 = 0, BT_FLUX2, BT_UPDATE, BT_BX1, BT_BX2, BT_N };
+enum { BT_FLUX4 = 0, BT_FLUX2, BT_UPDATE, BT_BX1, BT_BX2, BT_SHARED, BT_TILES, BT_N };
 
 struct harm_batch {
   int n;
@@ -3952,6 +4024,8 @@ struct harm_batch {
   bool tuned;
   int flux_variant;   // HARM_FLUX_FACE_64x4 or HARM_FLUX_FACE_64x2
   int bound_variant;  // HARM_BOUND_*
+  bool fill;          // zone-shared fluxes, the fill in the update (batch_substage_fill), not the variants
+  BatchKernels kern;  // its kernels
   int timeorder;
 };
 
@@ -3959,6 +4033,28 @@ static void add_blocks(std::vector<int4>& v, int run, dim3 g) {
   for (unsigned z = 0; z < g.z; z++)
     for (unsigned y = 0; y < g.y; y++)
       for (unsigned x = 0; x < g.x; x++) v.push_back(make_int4(run, (int)x, (int)y, (int)z));
+}
+
+// One substage of every run with the zone-shared fluxes and the first
+// bound_prim() in the update, where every run's boundaries allow that fill and
+// the caller has set no variants: in one launch up to ONE_LAUNCH_TILES tiles
+// over all runs, the line measured there.  Twelve tori of 88 to 256 zones a
+// side (450K zones), 4 steps: 4329 us, 5005 with the thread-per-face fluxes and
+// the fills in launches of their own.
+static int batch_substage_fill(harm_batch* b, const RKCoef& C, int pi, int pb, int pf) {
+  const bool one = pb != pf && b->ntab[BT_TILES] <= ONE_LAUNCH_TILES;
+  if (one) {
+    hipLaunchKernelGGL(b->kern.one, dim3(b->ntab[BT_TILES]), dim3(64 * tile::NW), 0, b->stream, b->d_runs,
+                       b->d_tab[BT_TILES], C, pi, pb, pf);
+  } else {
+    hipLaunchKernelGGL(b->kern.flux, dim3(b->ntab[BT_SHARED]), dim3(64, FSH_ROWS), 0, b->stream, b->d_runs,
+                       b->d_tab[BT_SHARED], pb);
+    hipLaunchKernelGGL(b->kern.update, dim3(b->ntab[BT_UPDATE]), dim3(64, 4), 0, b->stream, b->d_runs,
+                       b->d_tab[BT_UPDATE], C, pi, pb, pf);
+  }
+  hipLaunchKernelGGL(kb_fixbound, dim3(b->n), dim3(256), 0, b->stream, b->d_runs, pf, C.last ? 1 : 0, one ? 1 : 0);
+  HIPCHK(hipGetLastError());
+  return 0;
 }
 
 static int batch_flux(harm_batch* b, int pr_sel) {
@@ -4004,6 +4100,10 @@ static int batch_enqueue_step(harm_batch* b) {
     C.cn0 = Cunew[to][0]; C.cn1 = Cunew[to][1]; C.cn2 = Cunew[to][2];
     C.timeorder = to;
     C.last = (to == nto - 1);
+    if (b->fill) {
+      if (batch_substage_fill(b, C, pii[to], pbb[to], pff[to])) return 1;
+      continue;
+    }
     if (batch_flux(b, pbb[to])) return 1;
     hipLaunchKernelGGL(kb_update, dim3(b->ntab[BT_UPDATE]), dim3(64, 4), 0, b->stream, b->d_runs,
                        b->d_tab[BT_UPDATE], C, pii[to], pbb[to], pff[to]);
@@ -4059,8 +4159,10 @@ extern "C" int harm_batch_create(harm_ctx* const* ctxs, int n, harm_batch** out)
   b->timeorder = ctxs[0]->prm.timeorder;
   b->flux_variant = HARM_FLUX_FACE_64x4;
   b->bound_variant = HARM_BOUND_KERNELS;
+  b->fill = true;
+  int scheme = flux_scheme(ctxs[0]->kp);
   std::vector<RunDesc> hr(n);
-  std::vector<int4> tab[BT_N];
+  std::vector<int4> tab[BT_N], tiles;
   for (int r = 0; r < n; r++) {
     harm_ctx* c = ctxs[r];
     RunDesc& d = hr[r];
@@ -4079,7 +4181,17 @@ extern "C" int harm_batch_create(harm_ctx* const* ctxs, int n, harm_batch** out)
     add_blocks(tab[BT_UPDATE], r, grid2(n2, n1, dim3(64, 4)));
     add_blocks(tab[BT_BX1], r, dim3((n2 + 63) / 64, 2 * NG));
     add_blocks(tab[BT_BX2], r, dim3((n1 + 2 * NG + 63) / 64, 2 * NG + 2));
+    for (int dir = 1; dir <= 2; dir++)
+      for (int k = 0; k < flux_shared_blocks(n1, n2, dir); k++) tab[BT_SHARED].push_back(make_int4(r, k, dir, 0));
+    for (int k = 0; k < tile_count(c->kp); k++) tiles.push_back(make_int4(r, k, 0, 0));
+    b->fill = b->fill && bound_images_ok(c->kp);
+    if (flux_scheme(c->kp) != scheme) scheme = 0;
   }
+  b->kern = batch_kernels(scheme);
+  const size_t per = (tiles.size() + 7) / 8;  // neighbouring tiles on one XCD, as k_substage
+  for (size_t k = 0; k < per; k++)
+    for (size_t x = 0; x < 8; x++)
+      if (x * per + k < tiles.size()) tab[BT_TILES].push_back(tiles[x * per + k]);
   hipError_t e = hipMalloc(&b->d_runs, sizeof(RunDesc) * n);
   if (e == hipSuccess) e = hipMemcpy(b->d_runs, hr.data(), sizeof(RunDesc) * n, hipMemcpyHostToDevice);
   for (int t = 0; t < BT_N && e == hipSuccess; t++) {
@@ -4097,10 +4209,10 @@ extern "C" int harm_batch_create(harm_ctx* const* ctxs, int n, harm_batch** out)
   return 0;
 }
 
-// Batch autotuner: the same four variant combinations as one-step batch
-// graphs, timed from the live state of every run, which is then restored.
+// Batch autotuner, for batches without that fill: the four variant
+// combinations as one-step batch graphs, timed from the live state of every run, which is then restored.
 static int batch_autotune(harm_batch* b) {
-  if (b->tuned) return 0;
+  if (b->tuned || b->fill) return 0;
   const int n = b->n;
   std::vector<DevScalars*> save(n, nullptr);  // device copies of each run's scalars
   std::vector<double*> keep(n, nullptr);
@@ -4187,6 +4299,7 @@ extern "C" int harm_batch_set_tuning(harm_batch* b, int flux_variant, int bound_
   b->flux_variant = flux_variant;
   b->bound_variant = bound_variant;
   b->tuned = true;
+  b->fill = false;
   if (b->graph_ok) {
     (void)hipGraphExecDestroy(b->graph);
     b->graph_ok = false;

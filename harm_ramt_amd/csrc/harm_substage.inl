@@ -70,18 +70,14 @@ __device__ __forceinline__ void face_value(const KParams& P, const KParams& P0, 
 }
 
 template <int LIMC, int EOMC, int FMC>
-__global__ __launch_bounds__(64 * tile::NW) void k_substage(
-    KParams P0, RKCoef C, const double* pi, const double* __restrict__ pb, double* pf, double* __restrict__ ulast,
-    double* __restrict__ unew, double* __restrict__ F1, double* __restrict__ F2, double* __restrict__ q1,
-    double* __restrict__ q2, const double* __restrict__ gF, const double* __restrict__ gC,
+__device__ __forceinline__ void substage_body(
+    const KParams& P0, const RKCoef& C, const double* pi, const double* __restrict__ pb, double* pf,
+    double* __restrict__ ulast, double* __restrict__ unew, double* __restrict__ F1, double* __restrict__ F2,
+    double* __restrict__ q1, double* __restrict__ q2, const double* __restrict__ gF, const double* __restrict__ gC,
     const double* __restrict__ gConn, int* __restrict__ pflag, int* __restrict__ faillist, DevScalars* __restrict__ ds,
-    int nti, int ntj) {
+    int ntj, int tl) {
   using namespace tile;
   const KParams P = specialize<LIMC, EOMC, FMC>(P0);
-  // neighbouring tiles on one XCD (workgroups go round over the eight), so
-  // that its L2 serves the rims
-  const int nt = nti * ntj, per = (nt + 7) / 8, tl = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if (tl >= nt) return;
   const int i0 = (tl / ntj) * TI, j0 = (tl % ntj) * TJ;
   __shared__ double sp[NPR][NZP];        // the states, from (i0-3, j0-3)
   __shared__ double sl[2][NPR][NZH];     // lower edge states from (i0-1, j0-1), then the lower faces' fluxes
@@ -313,6 +309,21 @@ __global__ __launch_bounds__(64 * tile::NW) void k_substage(
     }
   }
   if (fail) atomicOr(&ds->failed, 1);
+}
+
+template <int LIMC, int EOMC, int FMC>
+__global__ __launch_bounds__(64 * tile::NW) void k_substage(
+    KParams P0, RKCoef C, const double* pi, const double* __restrict__ pb, double* pf, double* __restrict__ ulast,
+    double* __restrict__ unew, double* __restrict__ F1, double* __restrict__ F2, double* __restrict__ q1,
+    double* __restrict__ q2, const double* __restrict__ gF, const double* __restrict__ gC,
+    const double* __restrict__ gConn, int* __restrict__ pflag, int* __restrict__ faillist, DevScalars* __restrict__ ds,
+    int nt, int ntj) {
+  // neighbouring tiles on one XCD (workgroups go round over the eight), so
+  // that its L2 serves the rims
+  const int per = (nt + 7) / 8, tl = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (tl >= nt) return;
+  substage_body<LIMC, EOMC, FMC>(P0, C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gF, gC, gConn, pflag, faillist, ds, ntj,
+                                 tl);
 }
 
 using SubstageKernel = void (*)(KParams, RKCoef, const double*, const double*, double*, double*, double*, double*,

@@ -52,3 +52,43 @@ def _same_fluxes(a, b, n1, n2, what):
     i in [-1,N1], j in [0,N2]"""
     for sel, w in ((H.F1, np.s_[NG:NG + n1 + 1, NG - 1:NG + n2 + 1]), (H.F2, np.s_[NG - 1:NG + n1 + 1, NG:NG + n2 + 1])):
         assert np.array_equal(bits(a.get_array(sel)[w]), bits(b.get_array(sel)[w])), what + ": fluxes"
+
+
+BATCHES = {  # runs (kind, n1, n2, order): one scheme or several, below and above 512 tiles together
+    "tori": [("ks", 33, 47, 4), ("ks", 64, 60, 4), ("ks", 4, 9, 4)],
+    "tori_large": [("ks", 117, 160, 4), ("ks", 120, 163, 4)],
+    "vortices": [("mink", 15, 23, 2), ("mink", 32, 32, 2)],
+    "vortices_large": [("mink", 170, 200, 4)],
+    "mixed_large": [("mink", 130, 161, 2), ("ks", 101, 131, 2), ("ffde", 16, 30, 2)],
+    "first_order": [("ks", 24, 24, 1), ("ks", 17, 66, 1)],
+}
+
+
+@pytest.mark.parametrize("case", sorted(BATCHES))
+def test_batch_with_the_fill_in_the_update(case):
+    """Every run of a batch against the same run alone with the fills in
+    launches of their own: state, flags, fluxes, time, counts."""
+    print(f"[case] batch {case}: {BATCHES[case]}, 12 steps", flush=True)
+    runs, alone = [], []
+    for kind, n1, n2, order in BATCHES[case]:
+        flux = H.LAXFFLUX if kind == "ffde" else H.HLLFLUX
+        lim = H.PARA if kind == "ks" else H.MC
+        g, geom, p0, prm = problem(kind, n1, n2, lim=lim, fluxmethod=flux, timeorder=order)
+        p0 = p0.copy()
+        if kind == "ks" and n1 > 4:
+            strong_field_at_edges(p0, n1, n2)
+        for out in (runs, alone):
+            out.append(gpu_ctx(geom, prm, p0, 1e-4 if kind == "mink" else 1e-3))
+        alone[-1].set_tuning(H.FLUX_SHARED, H.BOUND_FUSED)
+    b = H.Batch(runs)
+    for n in (1, 11):
+        b.step_n(n)
+        for k, (x, y) in enumerate(zip(runs, alone)):
+            y.step_n(n)
+            what = f"run {k}"
+            assert x.get_time() == y.get_time(), what
+            assert np.array_equal(bits(x.get_array(H.P)), bits(y.get_array(H.P))), what + ": state"
+            assert np.array_equal(x.get_pflag(), y.get_pflag()), what + ": flags"
+            assert x.nstroke() == y.nstroke() and x.failures() == y.failures(), what
+            _same_fluxes(x, y, *BATCHES[case][k][1:3], what)
+    b.close()
