@@ -179,7 +179,7 @@ __global__ void k_acct_srcterm(KParams P, AcctRegions R, const double* __restric
   geo_from_cent(gc, g);
   double pr[NPR], dU[NPR], ft[NPR], fd[NPR];
   load8(pb, z, pr);
-  source_conn_at(P, pr, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, dU);
+  source_conn_at(P, pr, g, [&](int e) { return conn_entry(P, gConn, conn_sym(e), z); }, dU);
   const double Dt = ds->dt;
 #pragma unroll
   for (int k = 0; k < NPR; k++) ft[k] = Dt * R.dVF * (0.0 + dU[k]);  // dUcomp[GEOMSOURCE] = 0 e + e dUconn

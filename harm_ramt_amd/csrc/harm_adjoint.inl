@@ -342,7 +342,7 @@ __global__ __launch_bounds__(256) void k_adj_gather(KParams P0, const double* co
     double pr[NPR], ldu[NPR];
     load8(pb, z, pr);
     load8(ldU, z, ldu);
-    source_rev_at(P, pr, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, ldu, l);
+    source_rev_at(P, pr, g, [&](int e) { return conn_entry(P, gConn, conn_sym(e), z); }, ldu, l);
   }
   store8(lp, z, l);
 }

@@ -28,6 +28,7 @@ constexpr double NUMEPSILON = 2.2204460492503131e-16;
 // kernel-side parameter block (by value in kernel arguments)
 struct KParams {
   int n1, n2, N2M, nz;  // nz = (n1 + 6) N2M zones, ghosts included
+  int zmask;            // 0 where every zone has the same geometry (GEO_UNIFORM), else -1
   int eomtype, lim, fluxmethod, fluxb;
   int bc[4];
   int fixupflux, poledeath, checksolution, eno;

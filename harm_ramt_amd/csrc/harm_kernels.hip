@@ -162,12 +162,56 @@ __device__ __forceinline__ double geo_entry(const KParams& P, const double* __re
   return *reinterpret_cast<const double*>(b + (unsigned)z * 8u);
 }
 
+// Geometry patterns: the entries that hold one value, to the bit, over all
+// zones (found when the tables are set, geo_pattern).  Kernels compiled for a
+// pattern read such an entry once a wavefront, from zone 0 (a scalar load), and
+// those compiled for none read zone 0 throughout where every entry is one value
+// (KParams::zmask).  A Kerr-Schild metric in theta-warped coordinates has 18
+// of its 86 entries so (no t-theta, r-theta, theta-phi), a Cartesian one all but
+// the floors.  The step is bound by its bytes on large grids, mostly these: us
+// a substage at 512^2, before -> after: torus 136.8 -> 130.6, monopole 102.0 ->
+// 95.9, Orszag-Tang 120.6 -> 96.1 (at 256^2, bound by a wavefront's chain, the
+// same).
+enum { GEO_ANY = 0, GEO_KS = 1, GEO_UNIFORM = 2 };
+struct GeoMask {
+  unsigned face, cent;
+  unsigned long long conn;
+};
+constexpr unsigned bit_of(int m) { return 1u << m; }
+constexpr GeoMask geo_mask(int geo) {
+  return geo == GEO_KS ? GeoMask{bit_of(2) | bit_of(5) | bit_of(8) | bit_of(12) | bit_of(13),
+                                 bit_of(2) | bit_of(5) | bit_of(8) | bit_of(12) | bit_of(13) | bit_of(16) | bit_of(18) |
+                                     bit_of(19) | bit_of(21) | bit_of(22) | bit_of(24),
+                                 1ull << 22 | 1ull << 28}
+         : geo == GEO_UNIFORM
+             ? GeoMask{0xffffu, ((1u << GCN) - 1u) & ~(bit_of(GC_GDET + 1) | bit_of(GC_GDET + 2)), (1ull << NCONN) - 1}
+             : GeoMask{0u, 0u, 0ull};
+}
+template <int GEO>
+__device__ __forceinline__ int geo_zone(const KParams& P, bool one, int z) {
+  return (GEO == GEO_ANY) ? (z & P.zmask) : one ? 0 : z;
+}
+template <int GEO = GEO_ANY>
+__device__ __forceinline__ double face_entry(const KParams& P, const double* __restrict__ gF, int m, int z) {
+  return geo_entry(P, gF, m, geo_zone<GEO>(P, geo_mask(GEO).face >> m & 1, z));
+}
+template <int GEO = GEO_ANY>
+__device__ __forceinline__ double cent_entry(const KParams& P, const double* __restrict__ gC, int m, int z) {
+  if (m == GC_GDET + 1 || m == GC_GDET + 2) return geo_entry(P, gC, m, z);  // the floors
+  return geo_entry(P, gC, m, geo_zone<GEO>(P, geo_mask(GEO).cent >> m & 1, z));
+}
+template <int GEO = GEO_ANY>
+__device__ __forceinline__ double conn_entry(const KParams& P, const double* __restrict__ gConn, int m, int z) {
+  return geo_entry(P, gConn, m, geo_zone<GEO>(P, geo_mask(GEO).conn >> m & 1, z));
+}
+
 // entries GF of the face records: gcov upper 10, gcon^{00..03}, gcon^{dd}, gdet
 __device__ __forceinline__ double face_gdet(const KParams& P, const double* __restrict__ gF, int z) {
   return geo_entry(P, gF, 15, z);
 }
+template <int GEO = GEO_ANY>
 __device__ __forceinline__ void load_geo_face(const KParams& P, const double* __restrict__ gF, int z, GeoU& g) {
-  auto a = [&](int m) { return geo_entry(P, gF, m, z); };
+  auto a = [&](int m) { return face_entry<GEO>(P, gF, m, z); };
   g.g00 = a(0); g.g01 = a(1); g.g02 = a(2); g.g03 = a(3); g.g11 = a(4); g.g12 = a(5);
   g.g13 = a(6); g.g22 = a(7); g.g23 = a(8); g.g33 = a(9);
   g.n00 = a(10); g.n01 = a(11); g.n02 = a(12); g.n03 = a(13); g.ndd = a(14); g.gdet = a(15);
@@ -671,6 +715,7 @@ __host__ __device__ __forceinline__ int flux_shared_blocks(int n1, int n2, int d
   return ((n1 + 2) * (n2 + 2) - 1 + 63 * FSH_ROWS - 1) / (63 * FSH_ROWS);
 }
 
+template <int GEO>
 __device__ __forceinline__ void flux_shared_body(const KParams& P, const KParams& P0, const double* __restrict__ pr,
                                                  double* __restrict__ F1, double* __restrict__ F2,
                                                  double* __restrict__ q1, double* __restrict__ q2,
@@ -691,7 +736,7 @@ __device__ __forceinline__ void flux_shared_body(const KParams& P, const KParams
     const bool face = tx >= 1 && zone_ok && jz >= 0;
     const double* gF2 = gF + (size_t)P.nz * GF;
     if (zone_ok) {
-      if (face) load_geo_face(P, gF2, zidx(P, i, jz), g);
+      if (face) load_geo_face<GEO>(P, gF2, zidx(P, i, jz), g);
       zone_edges_fast(P, P0, pr, zidx(P, i, jz), 1, l, r);
     } else {
 #pragma unroll
@@ -709,7 +754,7 @@ __device__ __forceinline__ void flux_shared_body(const KParams& P, const KParams
     const bool zone_ok = iz <= P.n1;
     const bool face = ty >= 1 && zone_ok;
     if (zone_ok) {
-      if (face) load_geo_face(P, gF, zidx(P, iz, j), g);
+      if (face) load_geo_face<GEO>(P, gF, zidx(P, iz, j), g);
       zone_edges_fast(P, P0, pr, zidx(P, iz, j), P.N2M, l, r);
     } else {
 #pragma unroll
@@ -736,31 +781,49 @@ __device__ __forceinline__ void flux_shared_body(const KParams& P, const KParams
   if (fail) atomicOr(&ds->failed, 1);
 }
 
-template <int LIMC, int EOMC, int FMC>
+template <int LIMC, int EOMC, int FMC, int GEO>
 __global__ __launch_bounds__(64 * FSH_ROWS) void k_flux_shared(KParams P0, const double* __restrict__ pr,
                                                               double* __restrict__ F1, double* __restrict__ F2,
                                                               double* __restrict__ q1, double* __restrict__ q2,
                                                               const double* __restrict__ gF,
                                                               DevScalars* __restrict__ ds, int nb1) {
   const int b = blockIdx.x;
-  flux_shared_body(specialize<LIMC, EOMC, FMC>(P0), P0, pr, F1, F2, q1, q2, gF, ds, b < nb1 ? 1 : 2, b < nb1 ? b : b - nb1);
+  flux_shared_body<GEO>(specialize<LIMC, EOMC, FMC>(P0), P0, pr, F1, F2, q1, q2, gF, ds, b < nb1 ? 1 : 2, b < nb1 ? b : b - nb1);
 }
 
-FluxKernel flux_shared_kernel(const KParams& P) {
-  switch (flux_scheme(P)) {
-    case 1: return k_flux_shared<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>;
-    case 2: return k_flux_shared<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>;
-    case 3: return k_flux_shared<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>;
-    default: return k_flux_shared<-1, -1, -1>;
+// the kernel f(LIM, EOM, FM, GEO) of a scheme on a geometry pattern; a pattern
+// that a scheme is not compiled for reads its geometry as any
+template <int V>
+using Const = std::integral_constant<int, V>;
+template <class F>
+auto by_scheme(int scheme, int geo, const F& f) {
+  using G = Const<HARM_EOMGRMHD>;
+  using M = Const<HARM_MC>;
+  switch (scheme * 3 + geo) {
+    case 3 + GEO_ANY: return f(Const<HARM_PARA>(), G(), Const<HARM_HLLFLUX>(), Const<GEO_ANY>());
+    case 3 + GEO_KS: return f(Const<HARM_PARA>(), G(), Const<HARM_HLLFLUX>(), Const<GEO_KS>());
+    case 6 + GEO_ANY: return f(M(), Const<HARM_EOMFFDE>(), Const<HARM_LAXFFLUX>(), Const<GEO_ANY>());
+    case 6 + GEO_KS: return f(M(), Const<HARM_EOMFFDE>(), Const<HARM_LAXFFLUX>(), Const<GEO_KS>());
+    case 9 + GEO_ANY: return f(M(), G(), Const<HARM_HLLFLUX>(), Const<GEO_ANY>());
+    case 9 + GEO_KS: return f(M(), G(), Const<HARM_HLLFLUX>(), Const<GEO_KS>());
+    case 9 + GEO_UNIFORM: return f(M(), G(), Const<HARM_HLLFLUX>(), Const<GEO_UNIFORM>());
+    case GEO_KS: return f(Const<-1>(), Const<-1>(), Const<-1>(), Const<GEO_KS>());
+    default: return f(Const<-1>(), Const<-1>(), Const<-1>(), Const<GEO_ANY>());
   }
+}
+FluxKernel flux_shared_kernel(const KParams& P, int geo) {
+  return by_scheme(flux_scheme(P), geo, [](auto l, auto e, auto f, auto g) -> FluxKernel {
+    return k_flux_shared<decltype(l)::value, decltype(e)::value, decltype(f)::value, decltype(g)::value>;
+  });
 }
 
 // corner EMF of flux_ct() (step_ch.c:1223-1234, CORNGDETVERSION=1) from the
 // per-face quotients written by k_flux
+template <int GEO = GEO_ANY>
 __device__ __forceinline__ double emf_at(const KParams& P, const double* __restrict__ q1,
                                          const double* __restrict__ q2, const double* __restrict__ gC, int i, int j) {
   const int z = zidx(P, i, j);
-  return 0.25 * (geo_entry(P, gC, GC_GDETC, z)) *
+  return 0.25 * (cent_entry<GEO>(P, gC, GC_GDETC, z)) *
          (q1[z] + q1[zidx(P, i, j - 1)] - q2[z] - q2[zidx(P, i - 1, j)]);
 }
 
@@ -1086,10 +1149,11 @@ __device__ __forceinline__ void cent_expand(const R& r, T* gc) {
 }
 
 // full CENT geometry record of zone z
+template <int GEO = GEO_ANY>
 __device__ __forceinline__ void load_cent(const KParams& P, const double* __restrict__ gC, int z, double* gc) {
   double v[GCN];
 #pragma unroll
-  for (int m = 0; m < GCN; m++) v[m] = geo_entry(P, gC, m, z);
+  for (int m = 0; m < GCN; m++) v[m] = cent_entry<GEO>(P, gC, m, z);
   cent_expand(
       [&](int m) { return v[m]; }, gc);
 }
@@ -1117,6 +1181,7 @@ __device__ __forceinline__ void flux_diff(const KParams& P, double* f1a, double*
   }
 }
 
+template <int GEO = GEO_ANY>
 __device__ __forceinline__ void flux_div(const KParams& P, const double* __restrict__ F1,
                                          const double* __restrict__ F2, const double* __restrict__ q1,
                                          const double* __restrict__ q2, const double* __restrict__ gC, int i, int j,
@@ -1130,10 +1195,10 @@ __device__ __forceinline__ void flux_div(const KParams& P, const double* __restr
   double e[4] = {0., 0., 0., 0.};
   const bool ct = P.fluxb == HARM_FLUXCTTOTH;
   if (ct) {
-    e[0] = emf_at(P, q1, q2, gC, i, j);
-    e[1] = emf_at(P, q1, q2, gC, i, j + 1);
-    e[2] = emf_at(P, q1, q2, gC, i + 1, j);
-    e[3] = emf_at(P, q1, q2, gC, i + 1, j + 1);
+    e[0] = emf_at<GEO>(P, q1, q2, gC, i, j);
+    e[1] = emf_at<GEO>(P, q1, q2, gC, i, j + 1);
+    e[2] = emf_at<GEO>(P, q1, q2, gC, i + 1, j);
+    e[3] = emf_at<GEO>(P, q1, q2, gC, i + 1, j + 1);
   }
   flux_diff(P, f1a, f1b, f2a, f2b, ct, e, d1, d2);
 }
@@ -1304,7 +1369,7 @@ static_assert(NG == 3, "an edge block has NG rows besides the edge row");
 // zone near an edge writes its ghost images after its inversion; an outflow
 // edge row hands its values to the other rows of its workgroup (LDS, one
 // barrier), which write the NG x1 ghost columns, one column per row
-template <int ENO, int BND = 0>
+template <int ENO, int BND = 0, int GEO = GEO_ANY>
 __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* __restrict__ pi,
                                                 const double* __restrict__ pb, double* __restrict__ pf,
                                                 double* __restrict__ ulast, double* __restrict__ unew,
@@ -1324,7 +1389,7 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
     const int z = zidx(P, i, j);
     const double dt = ds->dt;
     double gc[36];
-    load_cent(P, gC, z, gc);
+    load_cent<GEO>(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     double pin[NPR], pbz[NPR];
@@ -1340,13 +1405,13 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
     }
     // source(pb): T^j_k Gamma^k_{lj} contraction (phys.c:475-619)
     double dUg[NPR];
-    source_conn_at(P, pbz, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, dUg);
+    source_conn_at(P, pbz, g, [&](int e) { return conn_entry<GEO>(P, gConn, conn_sym(e), z); }, dUg);
     double d1[NPR], d2[NPR];
     if constexpr (ENO == 2) {
       eno_cvt_zone<ENO_A2C, 1>(P, eA, i, j, d1);
       eno_cvt_zone<ENO_A2C, 2>(P, eB, i, j, d2);
     } else {
-      flux_div(P, F1, F2, q1, q2, gC, i, j, d1, d2);
+      flux_div<GEO>(P, F1, F2, q1, q2, gC, i, j, d1, d2);
     }
     double ul[NPR], un[NPR], Uf[NPR];
     if (C.timeorder == 0) {
@@ -1424,7 +1489,7 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
 
 // EOMC >= 0: the equations of motion as a compile-time constant (the
 // inversion and the fluxes without the other branch)
-template <int ENO, int EOMC = -1, int BND = 0>
+template <int ENO, int EOMC = -1, int BND = 0, int GEO = GEO_ANY>
 __global__ __launch_bounds__(256) void k_update(KParams P, RKCoef C, const double* __restrict__ pi,
                                                 const double* __restrict__ pb, double* __restrict__ pf,
                                                 double* __restrict__ ulast, double* __restrict__ unew,
@@ -1433,7 +1498,7 @@ __global__ __launch_bounds__(256) void k_update(KParams P, RKCoef C, const doubl
                                                 const double* __restrict__ gC, const double* __restrict__ gConn,
                                                 int* __restrict__ pflag, int* __restrict__ faillist,
                                                 DevScalars* __restrict__ ds, double* eA, const double* eB) {
-  update_body<ENO, BND>(specialize<-1, EOMC, -1>(P), C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gC, gConn, pflag,
+  update_body<ENO, BND, GEO>(specialize<-1, EOMC, -1>(P), C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gC, gConn, pflag,
                    faillist, ds, eA, eB, dim3(blockIdx.x, blockIdx.y, blockIdx.z),
                    dim3(gridDim.x, gridDim.y, gridDim.z));
 }
@@ -2704,34 +2769,34 @@ __global__ void kb_bx2(const RunDesc* __restrict__ runs, const int4* __restrict_
 // the zone-shared fluxes (table: run, block, direction), the update with the
 // in-update fill, both of them in one launch (table: run, tile), and the rest
 // of the substage, a workgroup a run
-template <int LIMC, int EOMC, int FMC>
+template <int LIMC, int EOMC, int FMC, int GEO>
 __global__ __launch_bounds__(64 * FSH_ROWS) void kb_flux_shared(const RunDesc* __restrict__ runs,
                                                                const int4* __restrict__ tab, int pr_sel) {
   const int4 e = tab[blockIdx.x];
   const RunDesc& r = runs[e.x];
   const KParams P0 = r.P;
-  flux_shared_body(specialize<LIMC, EOMC, FMC>(P0), P0, r.arr[pr_sel], r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gF,
+  flux_shared_body<GEO>(specialize<LIMC, EOMC, FMC>(P0), P0, r.arr[pr_sel], r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gF,
                    r.ds, e.z, e.y);
 }
 
-template <int LIMC, int EOMC, int FMC>
+template <int EOMC, int GEO>
 __global__ __launch_bounds__(256) void kb_update_fill(const RunDesc* __restrict__ runs, const int4* __restrict__ tab,
                                                       RKCoef C, int pi, int pb, int pf) {
   const int4 e = tab[blockIdx.x];
   const RunDesc& r = runs[e.x];
-  update_body<0, 1>(specialize<LIMC, EOMC, FMC>(r.P), C, r.arr[pi], r.arr[pb], r.arr[pf], r.arr[HARM_ULAST],
+  update_body<0, 1, GEO>(specialize<-1, EOMC, -1>(r.P), C, r.arr[pi], r.arr[pb], r.arr[pf], r.arr[HARM_ULAST],
                     r.arr[HARM_UNEW], r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gC, r.gConn, r.pflag, r.faillist,
                     r.ds, nullptr, nullptr, dim3(e.y, e.z, e.w), dim3(0, 0, 0));
 }
 
-template <int LIMC, int EOMC, int FMC>
+template <int LIMC, int EOMC, int FMC, int GEO>
 __global__ __launch_bounds__(64 * tile::NW) void kb_substage(const RunDesc* __restrict__ runs,
                                                             const int4* __restrict__ tab, RKCoef C, int pi, int pb,
                                                             int pf) {
   const int4 e = tab[blockIdx.x];
   const RunDesc& r = runs[e.x];
   const KParams P0 = r.P;
-  substage_body<LIMC, EOMC, FMC>(P0, C, r.arr[pi], r.arr[pb], r.arr[pf], r.arr[HARM_ULAST], r.arr[HARM_UNEW],
+  substage_body<LIMC, EOMC, FMC, GEO>(P0, C, r.arr[pi], r.arr[pb], r.arr[pf], r.arr[HARM_ULAST], r.arr[HARM_UNEW],
                                  r.arr[HARM_F1], r.arr[HARM_F2], r.q1, r.q2, r.gF, r.gC, r.gConn, r.pflag, r.faillist,
                                  r.ds, (P0.n2 + tile::TJ - 1) / tile::TJ, e.y);
 }
@@ -2750,17 +2815,15 @@ struct BatchKernels {
   void (*update)(const RunDesc*, const int4*, RKCoef, int, int, int);
   void (*one)(const RunDesc*, const int4*, RKCoef, int, int, int);
 };
-template <int LIMC, int EOMC, int FMC>
+template <int LIMC, int EOMC, int FMC, int GEO>
 BatchKernels batch_kernels_of() {
-  return {kb_flux_shared<LIMC, EOMC, FMC>, kb_update_fill<-1, EOMC, -1>, kb_substage<LIMC, EOMC, FMC>};
+  return {kb_flux_shared<LIMC, EOMC, FMC, GEO>, kb_update_fill<EOMC, GEO>, kb_substage<LIMC, EOMC, FMC, GEO>};
 }
-BatchKernels batch_kernels(int scheme) {
-  switch (scheme) {
-    case 1: return batch_kernels_of<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>();
-    case 2: return batch_kernels_of<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>();
-    case 3: return batch_kernels_of<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>();
-    default: return batch_kernels_of<-1, -1, -1>();
-  }
+BatchKernels batch_kernels(int scheme, int geo) {
+  if (scheme == 1 && geo == GEO_KS) return batch_kernels_of<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX, GEO_KS>();
+  if (scheme == 2 && geo == GEO_KS) return batch_kernels_of<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX, GEO_KS>();
+  if (scheme == 3 && geo == GEO_UNIFORM) return batch_kernels_of<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX, GEO_UNIFORM>();
+  return batch_kernels_of<-1, -1, -1, GEO_ANY>();
 }
 
 // failed-list kernels: FIXBLK blocks per run, block b of run r is blockIdx.x = r*FIXBLK+b
@@ -2839,6 +2902,7 @@ struct harm_ctx {
   hipGraphExec_t graphK;            // STEPS_PER_GRAPH steps in one graph (harm_step_n)
   bool graphK_ok;
   bool geometry_set;
+  int geo;            // GEO_*: the pattern of its tables
   bool prof;
   int flux_variant;   // HARM_FLUX_* chosen by the autotuner or the caller
   int bound_variant;  // HARM_BOUND_*
@@ -2928,7 +2992,7 @@ extern "C" int harm_create(const harm_params* prm, harm_ctx** out) {
   c->N2M = prm->n2 + 2 * NG;
   c->nz = c->N1M * c->N2M;
   KParams& k = c->kp;
-  k.n1 = prm->n1; k.n2 = prm->n2; k.N2M = c->N2M; k.nz = c->nz;
+  k.n1 = prm->n1; k.n2 = prm->n2; k.N2M = c->N2M; k.nz = c->nz; k.zmask = -1;
   k.eomtype = prm->eomtype; k.lim = prm->lim; k.fluxmethod = prm->fluxmethod; k.fluxb = prm->fluxb;
   for (int b = 0; b < 4; b++) k.bc[b] = prm->bc[b];
   // advance_eno_u calls fix_flux whatever FIXUPFLUX says (advance.c:355)
@@ -3144,6 +3208,26 @@ static bool pack_geometry(size_t nz, const double* gcov, const double* gcon, con
   return true;
 }
 
+// the pattern whose entries hold one value over all nz zones
+static int geo_pattern(size_t nz, const std::vector<double>& hF, const std::vector<double>& hC,
+                       const std::vector<double>& hT) {
+  auto one = [&](const double* t) {
+    for (size_t z = 1; z < nz; z++)
+      if (memcmp(t + z, t, sizeof(double))) return false;
+    return true;
+  };
+  auto fits = [&](const GeoMask& g) {
+    for (int m = 0; m < 2 * GF; m++)
+      if ((g.face >> (m % GF) & 1) && !one(&hF[m * nz])) return false;
+    for (int m = 0; m < GCN; m++)
+      if ((g.cent >> m & 1) && !one(&hC[m * nz])) return false;
+    for (int m = 0; m < NCONN; m++)
+      if ((g.conn >> m & 1) && !one(&hT[m * nz])) return false;
+    return true;
+  };
+  return fits(geo_mask(GEO_UNIFORM)) ? GEO_UNIFORM : fits(geo_mask(GEO_KS)) ? GEO_KS : GEO_ANY;
+}
+
 extern "C" int harm_set_geometry(harm_ctx* c, const double* gcov, const double* gcon, const double* gdet,
                                  const double* conn, const double* floors) {
   if (!c || !gcov || !gcon || !gdet || !conn || !floors) return seterr("null argument");
@@ -3153,6 +3237,10 @@ extern "C" int harm_set_geometry(harm_ctx* c, const double* gcov, const double* 
   HIPCHK(hipMemcpy(c->gF, hF.data(), hF.size() * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->gC, hC.data(), hC.size() * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->gConn, hT.data(), hT.size() * sizeof(double), hipMemcpyHostToDevice));
+  const int geo = geo_pattern((size_t)c->nz, hF, hC, hT);
+  if (geo != c->geo) drop_graphs(c);  // their kernels are the old pattern's
+  c->geo = geo;
+  c->kp.zmask = (geo == GEO_UNIFORM) ? 0 : -1;
   c->geometry_set = true;
   return 0;
 }
@@ -3322,7 +3410,7 @@ static int launch_flux(harm_ctx* c, int pr_sel, int dir0, int ndir, bool fix = t
     case HARM_FLUX_SHARED: {
       const int nb1 = dir0 == 1 ? flux_shared_blocks(c->kp.n1, c->kp.n2, 1) : 0;
       const int nb2 = dir0 + ndir > 2 ? flux_shared_blocks(c->kp.n1, c->kp.n2, 2) : 0;
-      tlaunch(c, flux_shared_kernel(kp), dim3(nb1 + nb2), dim3(64, FSH_ROWS), 0, kp, c->arr[pr_sel], c->arr[HARM_F1],
+      tlaunch(c, flux_shared_kernel(kp, c->geo), dim3(nb1 + nb2), dim3(64, FSH_ROWS), 0, kp, c->arr[pr_sel], c->arr[HARM_F1],
               c->arr[HARM_F2], c->q1, c->q2, c->gF, c->ds, nb1);
       break;
     }
@@ -3341,6 +3429,22 @@ static int launch_flux(harm_ctx* c, int pr_sel, int dir0, int ndir, bool fix = t
 // along x1 A -> B, update (c2a along x2 of B; averaged Uf -> A), a2c along
 // x1 A -> B, inversion (a2c along x2 of B).  DOENO=2: the two flux
 // divergences -> A, B, then the update converts them.
+// the update for the equations of motion, with or without the first fill, on a
+// geometry pattern (uniform: for GRMHD, else any)
+template <int EOMC, int BND>
+static auto update_kernel_geo(int geo) {
+  return geo == GEO_KS ? k_update<0, EOMC, BND, GEO_KS>
+         : (geo == GEO_UNIFORM && EOMC == HARM_EOMGRMHD) ? k_update<0, EOMC, BND, EOMC == HARM_EOMGRMHD ? GEO_UNIFORM : GEO_ANY>
+                                                          : k_update<0, EOMC, BND, GEO_ANY>;
+}
+static auto update_kernel(const KParams& P, bool bnd, int geo) {
+  if (P.eno == 1) return k_update<1>;
+  if (P.eno == 2) return k_update<2>;
+  if (P.eomtype == HARM_EOMGRMHD)
+    return bnd ? update_kernel_geo<HARM_EOMGRMHD, 1>(geo) : update_kernel_geo<HARM_EOMGRMHD, 0>(geo);
+  return bnd ? update_kernel_geo<HARM_EOMFFDE, 1>(geo) : update_kernel_geo<HARM_EOMFFDE, 0>(geo);
+}
+
 static int launch_update(harm_ctx* c, int pi, int pb, int pf, const RKCoef& C, bool bnd = false) {
   const dim3 b(64, 4);
   const dim3 gz = grid2(c->kp.n2, c->kp.n1, b);
@@ -3355,13 +3459,7 @@ static int launch_update(harm_ctx* c, int pi, int pb, int pf, const RKCoef& C, b
     tlaunch(c,k_eno_fluxdiv, gz, b, 0, c->kp, c->arr[HARM_F1], c->arr[HARM_F2], c->q1, c->q2,
                        c->gC, c->enoA, c->enoB);
   }
-  auto* kup = (c->kp.eno == 1)                        ? k_update<1>
-              : (c->kp.eno == 2)                      ? k_update<2>
-              : (c->kp.eomtype == HARM_EOMGRMHD)      ? (bnd ? k_update<0, HARM_EOMGRMHD, 1>
-                                                             : k_update<0, HARM_EOMGRMHD>)
-              : (c->kp.eomtype == HARM_EOMFFDE)       ? (bnd ? k_update<0, HARM_EOMFFDE, 1>
-                                                             : k_update<0, HARM_EOMFFDE>)
-                                                      : (bnd ? k_update<0, -1, 1> : k_update<0>);
+  auto* kup = update_kernel(c->kp, bnd, c->geo);
   tlaunch(c,kup, gz, b, 0, c->kp, C, c->arr[pi], c->arr[pbs], c->arr[pf], c->arr[HARM_ULAST],
                      c->arr[HARM_UNEW], c->arr[HARM_F1], c->arr[HARM_F2], c->q1, c->q2, c->gC, c->gConn, c->pflag,
                      c->faillist, c->ds, c->enoA, c->enoB);
@@ -3549,7 +3647,7 @@ static int substage(harm_ctx* c, int pi, int pb, int pf, const double* CUf, cons
   C.last = (to == nto - 1);
   if (one_launch(c, pb, pf, bnd)) {
     const int nti = (c->kp.n1 + tile::TI - 1) / tile::TI, ntj = (c->kp.n2 + tile::TJ - 1) / tile::TJ;
-    hipLaunchKernelGGL(substage_kernel(c->kp), dim3((nti * ntj + 7) / 8 * 8), dim3(64 * tile::NW), 0, c->stream, c->kp,
+    hipLaunchKernelGGL(substage_kernel(c->kp, c->geo), dim3((nti * ntj + 7) / 8 * 8), dim3(64 * tile::NW), 0, c->stream, c->kp,
                        C, c->arr[pi], c->arr[pb], c->arr[pf], c->arr[HARM_ULAST], c->arr[HARM_UNEW], c->arr[HARM_F1],
                        c->arr[HARM_F2], c->q1, c->q2, c->gF, c->gC, c->gConn, c->pflag, c->faillist, c->ds, nti * ntj, ntj);
     HIPCHK(hipGetLastError());
@@ -4026,8 +4124,32 @@ struct harm_batch {
   int bound_variant;  // HARM_BOUND_*
   bool fill;          // zone-shared fluxes, the fill in the update (batch_substage_fill), not the variants
   BatchKernels kern;  // its kernels
+  std::vector<RunDesc>* runs;
+  std::vector<int>* geo;  // the runs' geometry patterns that kern and runs hold
   int timeorder;
 };
+
+// The runs' geometry patterns, into the descriptors and the choice of kernels:
+// at the batch's creation, and again where a context has been given tables of
+// another pattern since (its tables' addresses stay).
+static int batch_geometry(harm_batch* b) {
+  bool same = true;
+  for (int r = 0; r < b->n; r++) same = same && (*b->ctx)[r]->geo == (*b->geo)[r];
+  if (same) return 0;
+  int scheme = flux_scheme((*b->ctx)[0]->kp), geo = (*b->ctx)[0]->geo;
+  for (int r = 0; r < b->n; r++) {
+    const harm_ctx* c = (*b->ctx)[r];
+    (*b->geo)[r] = c->geo;
+    (*b->runs)[r].P.zmask = c->kp.zmask;
+    if (flux_scheme(c->kp) != scheme) scheme = 0;
+    if (c->geo != geo) geo = GEO_ANY;
+  }
+  b->kern = batch_kernels(scheme, geo);
+  if (b->graph_ok) (void)hipGraphExecDestroy(b->graph);
+  b->graph_ok = false;
+  HIPCHK(hipMemcpy(b->d_runs, b->runs->data(), sizeof(RunDesc) * b->n, hipMemcpyHostToDevice));
+  return 0;
+}
 
 static void add_blocks(std::vector<int4>& v, int run, dim3 g) {
   for (unsigned z = 0; z < g.z; z++)
@@ -4133,6 +4255,8 @@ extern "C" int harm_batch_destroy(harm_batch* b) {
   (void)hipFree(b->d_runs);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b->ctx;
+  delete b->runs;
+  delete b->geo;
   delete b;
   return 0;
 }
@@ -4160,8 +4284,9 @@ extern "C" int harm_batch_create(harm_ctx* const* ctxs, int n, harm_batch** out)
   b->flux_variant = HARM_FLUX_FACE_64x4;
   b->bound_variant = HARM_BOUND_KERNELS;
   b->fill = true;
-  int scheme = flux_scheme(ctxs[0]->kp);
-  std::vector<RunDesc> hr(n);
+  b->runs = new std::vector<RunDesc>(n);
+  b->geo = new std::vector<int>(n, -1);
+  std::vector<RunDesc>& hr = *b->runs;
   std::vector<int4> tab[BT_N], tiles;
   for (int r = 0; r < n; r++) {
     harm_ctx* c = ctxs[r];
@@ -4185,15 +4310,16 @@ extern "C" int harm_batch_create(harm_ctx* const* ctxs, int n, harm_batch** out)
       for (int k = 0; k < flux_shared_blocks(n1, n2, dir); k++) tab[BT_SHARED].push_back(make_int4(r, k, dir, 0));
     for (int k = 0; k < tile_count(c->kp); k++) tiles.push_back(make_int4(r, k, 0, 0));
     b->fill = b->fill && bound_images_ok(c->kp);
-    if (flux_scheme(c->kp) != scheme) scheme = 0;
   }
-  b->kern = batch_kernels(scheme);
   const size_t per = (tiles.size() + 7) / 8;  // neighbouring tiles on one XCD, as k_substage
   for (size_t k = 0; k < per; k++)
     for (size_t x = 0; x < 8; x++)
       if (x * per + k < tiles.size()) tab[BT_TILES].push_back(tiles[x * per + k]);
   hipError_t e = hipMalloc(&b->d_runs, sizeof(RunDesc) * n);
-  if (e == hipSuccess) e = hipMemcpy(b->d_runs, hr.data(), sizeof(RunDesc) * n, hipMemcpyHostToDevice);
+  if (e == hipSuccess && batch_geometry(b)) {
+    harm_batch_destroy(b);
+    return 1;
+  }
   for (int t = 0; t < BT_N && e == hipSuccess; t++) {
     b->ntab[t] = (int)tab[t].size();
     e = hipMalloc(&b->d_tab[t], sizeof(int4) * tab[t].size());
@@ -4280,6 +4406,7 @@ static int batch_autotune(harm_batch* b) {
 extern "C" int harm_batch_step_n(harm_batch* b, int nsteps) {
   if (!b) return seterr("null batch");
   if (nsteps < 0) return seterr("nsteps < 0");
+  if (batch_geometry(b)) return 1;
   if (batch_autotune(b)) return 1;
   if (!b->graph_ok) {
     if (batch_capture(b, &b->graph)) return 1;

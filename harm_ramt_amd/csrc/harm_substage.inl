@@ -52,12 +52,12 @@ __device__ __forceinline__ void face_rules(const KParams& P, double* Fo, int i, 
 
 // a face's flux from its two states, by the general functions where the
 // shorter form does not hold
-template <int DIR>
+template <int DIR, int GEO>
 __device__ __forceinline__ void face_value(const KParams& P, const KParams& P0, const double* p_l, const double* p_r,
                                            const double* __restrict__ pb, const double* __restrict__ gF, int i, int j,
                                            double (&Fo)[NPR], double& gdet, double& cm, double& dtij, int& fail) {
   GeoU g;
-  load_geo_face(P, gF, zidx(P, i, j), g);
+  load_geo_face<GEO>(P, gF, zidx(P, i, j), g);
   gdet = g.gdet;
   if (__builtin_expect(!face_flux_fast<DIR>(P, p_l, p_r, g, Fo, cm, fail), 0)) {
     cm = 0.;
@@ -69,7 +69,7 @@ __device__ __forceinline__ void face_value(const KParams& P, const KParams& P0, 
   }
 }
 
-template <int LIMC, int EOMC, int FMC>
+template <int LIMC, int EOMC, int FMC, int GEO>
 __device__ __forceinline__ void substage_body(
     const KParams& P0, const RKCoef& C, const double* pi, const double* __restrict__ pb, double* pf,
     double* __restrict__ ulast, double* __restrict__ unew, double* __restrict__ F1, double* __restrict__ F2,
@@ -133,7 +133,7 @@ __device__ __forceinline__ void substage_body(
     // the tile that holds the face's zone (the nearest, outside the grid) writes it
     const bool own = C.last && max(0, min(ei, P.n1 - 1)) / TI * TI == i0 && max(0, min(ej, P.n2 - 1)) / TJ * TJ == j0;
     if (d == 0) {
-      face_value<1>(P, P0, p_l, p_r, pb, gF, ei, ej, Fo, gdet, cm, dtij, fail);
+      face_value<1, GEO>(P, P0, p_l, p_r, pb, gF, ei, ej, Fo, gdet, cm, dtij, fail);
       face_rules<1>(P, Fo, ei, ej);
       sq[0][eid] = Fo[B2] / gdet;
       if (P.fixupflux && ei < P.n1) {
@@ -144,7 +144,7 @@ __device__ __forceinline__ void substage_body(
       if (own) face_store<1>(P, Fo, gdet, F1, q1, gF, ei, ej);
     } else {
       const double* gF2 = gF + (size_t)P.nz * GF;
-      face_value<2>(P, P0, p_l, p_r, pb, gF2, ei, ej, Fo, gdet, cm, dtij, fail);
+      face_value<2, GEO>(P, P0, p_l, p_r, pb, gF2, ei, ej, Fo, gdet, cm, dtij, fail);
       face_rules<2>(P, Fo, ei, ej);
       sq[1][eid] = Fo[B1] / gdet;
       if (own) face_store<2>(P, Fo, gdet, F2, q2, gF2, ei, ej);
@@ -178,14 +178,14 @@ __device__ __forceinline__ void substage_body(
   const int h = (zi + 1) * HJ + zj + 1;
   if ((w == NW - 3 || w == NW - 2) && zone) {
     double gc[36], v[NPR];
-    load_cent(P, gC, z, gc);
+    load_cent<GEO>(P, gC, z, gc);
     GeoU g;
     geo_from_cent(gc, g);
     if (w == NW - 3) {  // T^j_k Gamma^k_{lj} contraction (phys.c:475-619)
       double pbz[NPR];
 #pragma unroll
       for (int k = 0; k < NPR; k++) pbz[k] = sp[k][(zi + NG) * PJ + zj + NG];
-      source_conn_at(P, pbz, g, [&](int e) { return geo_entry(P, gConn, conn_sym(e), z); }, v);
+      source_conn_at(P, pbz, g, [&](int e) { return conn_entry<GEO>(P, gConn, conn_sym(e), z); }, v);
 #pragma unroll
       for (int k = 0; k < 4; k++) pu[8 + k][lane] = v[UU + k];
     } else {
@@ -203,7 +203,7 @@ __device__ __forceinline__ void substage_body(
   GeoU g;
   const bool upd = w == NW - 1;
   if (upd && zone) {
-    load_cent(P, gC, z, gc);
+    load_cent<GEO>(P, gC, z, gc);
     geo_from_cent(gc, g);
     load8(pi, z, pin);
     if (C.timeorder == 0) {
@@ -232,7 +232,7 @@ __device__ __forceinline__ void substage_body(
           if (mdn && j + b == 0) qb = sm[0][zi + 1 + a];
           if (mup && j + b == P.n2) qa = sm[1][zi + 1 + a];
         }
-        return 0.25 * geo_entry(P, gC, GC_GDETC, z + a * P.N2M + b) * (qa + qb - sq[1][m] - sq[1][m - HJ]);
+        return 0.25 * cent_entry<GEO>(P, gC, GC_GDETC, z + a * P.N2M + b) * (qa + qb - sq[1][m] - sq[1][m - HJ]);
       };
       e[0] = emf(0, 0);
       e[1] = emf(0, 1);
@@ -311,7 +311,7 @@ __device__ __forceinline__ void substage_body(
   if (fail) atomicOr(&ds->failed, 1);
 }
 
-template <int LIMC, int EOMC, int FMC>
+template <int LIMC, int EOMC, int FMC, int GEO>
 __global__ __launch_bounds__(64 * tile::NW) void k_substage(
     KParams P0, RKCoef C, const double* pi, const double* __restrict__ pb, double* pf, double* __restrict__ ulast,
     double* __restrict__ unew, double* __restrict__ F1, double* __restrict__ F2, double* __restrict__ q1,
@@ -322,18 +322,15 @@ __global__ __launch_bounds__(64 * tile::NW) void k_substage(
   // that its L2 serves the rims
   const int per = (nt + 7) / 8, tl = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (tl >= nt) return;
-  substage_body<LIMC, EOMC, FMC>(P0, C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gF, gC, gConn, pflag, faillist, ds, ntj,
+  substage_body<LIMC, EOMC, FMC, GEO>(P0, C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gF, gC, gConn, pflag, faillist, ds, ntj,
                                  tl);
 }
 
 using SubstageKernel = void (*)(KParams, RKCoef, const double*, const double*, double*, double*, double*, double*,
                                 double*, double*, double*, const double*, const double*, const double*, int*, int*,
                                 DevScalars*, int, int);
-SubstageKernel substage_kernel(const KParams& P) {
-  switch (flux_scheme(P)) {
-    case 1: return k_substage<HARM_PARA, HARM_EOMGRMHD, HARM_HLLFLUX>;
-    case 2: return k_substage<HARM_MC, HARM_EOMFFDE, HARM_LAXFFLUX>;
-    case 3: return k_substage<HARM_MC, HARM_EOMGRMHD, HARM_HLLFLUX>;
-    default: return k_substage<-1, -1, -1>;
-  }
+SubstageKernel substage_kernel(const KParams& P, int geo) {
+  return by_scheme(flux_scheme(P), geo, [](auto l, auto e, auto f, auto g) -> SubstageKernel {
+    return k_substage<decltype(l)::value, decltype(e)::value, decltype(f)::value, decltype(g)::value>;
+  });
 }
