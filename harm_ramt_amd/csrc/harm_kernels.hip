@@ -1203,6 +1203,14 @@ __device__ __forceinline__ void flux_div(const KParams& P, const double* __restr
   flux_diff(P, f1a, f1b, f2a, f2b, ct, e, d1, d2);
 }
 
+// Makes index j one that the compiler knows only once the values v are formed:
+// what is loaded by it is loaded after them.
+template <int N>
+__device__ __forceinline__ void after(int& j, double (&v)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; k++) asm volatile("" : "+v"(j), "+v"(v[k]));
+}
+
 // RK combination of one zone (dUtoU, advance.c:273-286)
 __device__ __forceinline__ void rk_combine(const RKCoef& C, double dt, const double* Ui, const double* d1,
                                            const double* d2, const double* dUg, double* ul, double* un, double* Uf) {
@@ -1365,6 +1373,17 @@ __device__ __forceinline__ int edge_block_side(const KParams& P, const dim3 bi) 
 }
 static_assert(NG == 3, "an edge block has NG rows besides the edge row");
 
+// Two wavefronts a SIMD (ENO 0; a wavefront's chain is latency: 2,700 64-bit
+// operations in 40,000 cycles): the compiler, left alone, loads all of a zone's
+// values at the top and holds 298 to 326 registers, which leaves one.  So what
+// the flux difference and the RK combination read is loaded once U(pi) and the
+// source term are formed (after()): 174 to 239 registers, nothing spilled.  us a
+// launch, before -> after: torus 512x512 79.4 -> 63.6, monopole 512x512 60.1 ->
+// 50.4, twelve tori of 88 to 256 zones a side 154.8 -> 111.9, Orszag-Tang 256x256
+// 22.5 -> 21.3; torus 256x256, one wavefront a SIMD in all, 23.2 -> 23.5 (without
+// the fill 20.2 -> 18.8).  Three wavefronts (loads in four groups, 168 registers)
+// cost the twelve tori 146.8 and gain nothing elsewhere.
+//
 // BND: the first bound_prim() of the substage done here (ENO 0 only): each
 // zone near an edge writes its ghost images after its inversion; an outflow
 // edge row hands its values to the other rows of its workgroup (LDS, one
@@ -1406,20 +1425,26 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
     // source(pb): T^j_k Gamma^k_{lj} contraction (phys.c:475-619)
     double dUg[NPR];
     source_conn_at(P, pbz, g, [&](int e) { return conn_entry<GEO>(P, gConn, conn_sym(e), z); }, dUg);
+    int jf = j;
+    if constexpr (ENO == 0) {
+      after(jf, dUg);
+      after(jf, Ui);
+    }
+    const int zf = zidx(P, i, jf);
     double d1[NPR], d2[NPR];
     if constexpr (ENO == 2) {
       eno_cvt_zone<ENO_A2C, 1>(P, eA, i, j, d1);
       eno_cvt_zone<ENO_A2C, 2>(P, eB, i, j, d2);
     } else {
-      flux_div<GEO>(P, F1, F2, q1, q2, gC, i, j, d1, d2);
+      flux_div<GEO>(P, F1, F2, q1, q2, gC, i, jf, d1, d2);
     }
     double ul[NPR], un[NPR], Uf[NPR];
     if (C.timeorder == 0) {
 #pragma unroll
       for (int k = 0; k < NPR; k++) ul[k] = un[k] = 0.0;
     } else {
-      load8(ulast, z, ul);
-      load8(unew, z, un);
+      load8(ulast, zf, ul);
+      load8(unew, zf, un);
     }
     rk_combine(C, dt, Ui, d1, d2, dUg, ul, un, Uf);
     store8(ulast, z, ul);
@@ -1490,7 +1515,7 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
 // EOMC >= 0: the equations of motion as a compile-time constant (the
 // inversion and the fluxes without the other branch)
 template <int ENO, int EOMC = -1, int BND = 0, int GEO = GEO_ANY>
-__global__ __launch_bounds__(256) void k_update(KParams P, RKCoef C, const double* __restrict__ pi,
+__global__ __launch_bounds__(256, ENO == 0 ? 2 : 1) void k_update(KParams P, RKCoef C, const double* __restrict__ pi,
                                                 const double* __restrict__ pb, double* __restrict__ pf,
                                                 double* __restrict__ ulast, double* __restrict__ unew,
                                                 const double* __restrict__ F1, const double* __restrict__ F2,
@@ -2780,7 +2805,7 @@ __global__ __launch_bounds__(64 * FSH_ROWS) void kb_flux_shared(const RunDesc* _
 }
 
 template <int EOMC, int GEO>
-__global__ __launch_bounds__(256) void kb_update_fill(const RunDesc* __restrict__ runs, const int4* __restrict__ tab,
+__global__ __launch_bounds__(256, 2) void kb_update_fill(const RunDesc* __restrict__ runs, const int4* __restrict__ tab,
                                                       RKCoef C, int pi, int pb, int pf) {
   const int4 e = tab[blockIdx.x];
   const RunDesc& r = runs[e.x];
