@@ -8,10 +8,10 @@
 // dump_ener.c:449-486) and conserved totals (constotal, dump_ener.c:562-590).
 // Its sums are serial loops, so each total here is formed in two phases:
 // every face or zone term in parallel (the same FP64 operations as the
-// reference, one thread each), then one lane per accumulator adding the terms
-// in the reference's loop order.  The serial phase is a single wavefront;
-// its length is one boundary (diag_flux), one grid row (frdot, lumvsr) or the
-// region's zones (sourceadd, constotal, divbavg).
+// reference, one thread each), then one chain per accumulator adding the terms
+// in the reference's loop order.  A chain's length is one boundary (diag_flux),
+// one grid row (frdot, lumvsr), the region's zones (sourceadd, constotal,
+// divbavg) or a substage's fixup events; chain_sum forms the long ones of a step.
 
 namespace {
 
@@ -52,10 +52,13 @@ struct AcctState {
   double* uin;      // the conserved state each force-free inversion took [nz][8]
   int* flag;        // [nslots], category + 1 of the event in the slot
   double* val;      // [nslots][8]
-  int* list;        // [nslots][2]: slot, category of the events in order
-  double* cval;     // [nslots][8]: their values in that order
-  int* cnt;         // [nblocks] events per block of 256 slots, then their offsets
-  int* off;
+  int* list;        // [nslots]: the events' keys (acct_slot_key) in order
+  double* cval;     // [8][nslots]: their values in that order
+  int* cnt;         // [nblocks] events per block of 256 slots
+  double* sterm;    // [8][n1*n2]: the source terms of a step, and ...
+  hipStream_t side; // ... the stream that adds them beside the rest of the step,
+  hipEvent_t fork, join;  // forked off and joined again within it
+  bool forked;
   int* total;
   int nslots, nblocks;
   bool tree;        // HARM_ACCT_TREE: source and fixup totals by reduction trees
@@ -164,6 +167,149 @@ __device__ __forceinline__ void box_rows(int first, int cnt, const double* b, in
   }
 }
 
+// A serial sum (harm_chain.h) by a workgroup of four wavefronts: the term of
+// item m is term(m), the sum so far s; the result in every lane of wavefront 0.
+// Wavefronts 1-3 stage chunks of 1024 terms in LDS while wavefront 0 adds the
+// chunk before: a run of 16 terms a lane as a map, the 64 maps composed by a
+// scan, and the runs whose map does not hold (the sum enters another binade)
+// term by term.  A sum that crosses binades all the time (terms of its own size
+// and both signs) is added term by term for some chunks before maps are tried
+// again.  Bound by the latency of a dependent addition, 7 cycles, where they do
+// not hold (the slowest of a 256x256 torus's source sums, 65,536 terms: 198 us;
+// 474 when all 24 sums shared one wavefront), by the scans where they do (a
+// substage's fixup events, 220 sums: 11 us, 150 before).
+constexpr int CH_RUN = 16, CH_N = 64 * CH_RUN, CH_STR = CH_RUN + 1;  // stride: no bank conflicts
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double a) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(a);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, CTRL, ROWS, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// one step of the scan: the map of the lanes before, by a register shift (2: the
+// parities of a map that changes nothing, where no lane is before)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void chain_step(double& d0, double& d1, int& q) {
+  const double a0 = dpp_or_zero<CTRL, ROWS>(d0), a1 = dpp_or_zero<CTRL, ROWS>(d1);
+  const int aq = __builtin_amdgcn_update_dpp(2, q, CTRL, ROWS, 0xf, false);
+  chain_then(a0, a1, aq, d0, d1, q);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)u, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(u >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// the runs [r0, r1) of a chunk, term by term
+__device__ __forceinline__ double chain_serial(const double* b, int r0, int r1, double s) {
+  double v[CH_RUN];
+#pragma unroll
+  for (int k = 0; k < CH_RUN; k++) v[k] = b[r0 * CH_STR + k];
+  for (int r = r0; r < r1; r++) {
+    double w[CH_RUN];
+    const double* n = b + min(r + 1, 63) * CH_STR;  // read ahead
+#pragma unroll
+    for (int k = 0; k < CH_RUN; k++) w[k] = n[k];
+#pragma unroll
+    for (int k = 0; k < CH_RUN; k++) s += v[k];
+#pragma unroll
+    for (int k = 0; k < CH_RUN; k++) v[k] = w[k];
+  }
+  return s;
+}
+// one chunk; wait: chunks still to be added term by term
+__device__ __forceinline__ double chain_chunk(const double* b, double s, int& wait) {
+  const int lane = threadIdx.x & 63;
+  double t[CH_RUN];
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < CH_RUN; k++) {
+    t[k] = b[lane * CH_STR + k];
+    any |= !(t[k] == 0.0);
+  }
+  const unsigned long long used = __ballot(any);
+  // zeros of either sign change no sum but -0
+  const bool minus_zero = chain_bits(s) == 1ull << 63;
+  if (used == 0 && !minus_zero) return s;
+  if (wait > 0 || minus_zero) {
+    wait = max(wait - 1, 0);
+    return chain_serial(b, 0, 64, s);
+  }
+  int from = 0;
+  for (int tries = 0; from < 64; tries++) {
+    const unsigned long long left = used >> from << from;
+    if (left == 0) break;
+    from = __builtin_ctzll(left);
+    if (tries == 6) {
+      wait = 4;
+      return chain_serial(b, from, 64, s);
+    }
+    const ChainScale c(s);
+    int bad = from;  // the first run whose map does not hold
+    if (c.e >= 0) {
+      ChainMap m = chain_map(c, t);
+      const bool out = lane < from;
+      double d0 = out ? 0.0 : m.d0, d1 = out ? 0.0 : m.d1;
+      int q = out ? 2 : m.q;
+      const double mn = out ? c.C : m.mn, mx = out ? c.C : m.mx;
+      chain_step<0x111, 0xf>(d0, d1, q);  // row_shr:1
+      chain_step<0x112, 0xf>(d0, d1, q);  // row_shr:2
+      chain_step<0x114, 0xf>(d0, d1, q);  // row_shr:4
+      chain_step<0x118, 0xf>(d0, d1, q);  // row_shr:8
+      chain_step<0x142, 0xa>(d0, d1, q);  // row_bcast:15 into rows 1 and 3
+      chain_step<0x143, 0xc>(d0, d1, q);  // row_bcast:31 into rows 2 and 3
+      const double size = fabs(s);
+      const double after = (chain_bits(s) & 1) ? d1 : d0;  // through this lane's run
+      const double before = __shfl_up(after, 1);
+      const double at = size + (lane > 0 ? before : 0.0);
+      const unsigned long long no = __ballot(!out && !chain_holds(c, at, mn, mx));
+      bad = no ? __builtin_ctzll(no) : 64;
+      if (bad > from) {
+        const double end = size + lane_value(after, bad - 1);
+        s = chain_bits(s) >> 63 ? -end : end;
+      }
+    }
+    if (bad < 64) s = chain_serial(b, bad, bad + 1, s);
+    from = bad + 1;
+  }
+  return s;
+}
+template <class Term>
+__device__ __forceinline__ double chain_sum(int n, double s, Term term) {
+  __shared__ double lds[2][64 * CH_STR];
+  constexpr int PER = (CH_N + 191) / 192;
+  const int tid = threadIdx.x, nch = (n + CH_N - 1) / CH_N;
+  double v[PER];  // the chunk after the one staged last, on its way
+  auto fetch = [&](int c) {
+#pragma unroll
+    for (int k = 0; k < PER; k++) v[k] = term(min(c * CH_N + tid - 64 + 192 * k, n - 1));
+  };
+  auto stage = [&](int c) {
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int m = tid - 64 + 192 * k;
+      if (m < CH_N) lds[c & 1][m / CH_RUN * CH_STR + m % CH_RUN] = (c * CH_N + m < n) ? v[k] : -0.0;
+    }
+    if (c + 1 < nch) fetch(c + 1);
+  };
+  if (tid >= 64 && nch > 0) {
+    fetch(0);
+    stage(0);
+  }
+  __syncthreads();
+  int wait = 0;
+  for (int c = 0; c < nch; c++) {
+    if (tid >= 64) {
+      if (c + 1 < nch) stage(c + 1);
+    } else {
+      s = chain_chunk(lds[c & 1], s, wait);
+    }
+    __syncthreads();
+  }
+  return s;
+}
+
 // diag_source's term of each interior zone (diag.c:1247-1259 with the
 // geometric source only; cooling is off): UDIAG form of Dt dVF dUcomp[0]
 __global__ void k_acct_srcterm(KParams P, AcctRegions R, const double* __restrict__ pb, const double* __restrict__ gC,
@@ -184,54 +330,61 @@ __global__ void k_acct_srcterm(KParams P, AcctRegions R, const double* __restric
 #pragma unroll
   for (int k = 0; k < NPR; k++) ft[k] = Dt * R.dVF * (0.0 + dU[k]);  // dUcomp[GEOMSOURCE] = 0 e + e dUconn
   evolve_to_diag(P, g.gdet, ft, fd);
-  store8(out, i * P.n2 + j, fd);
+#pragma unroll
+  for (int k = 0; k < NPR; k++) out[((size_t)k * P.n1 + i) * P.n2 + j] = fd[k];
 }
 
-// sourceadd and sourceaddterms[0] (lane = region*8 + k) over the region's
+// sourceadd and sourceaddterms[0] (workgroup = region*8 + k) over the region's
 // zones in ZLOOP order.  The reference also adds the six cooling sources,
 // all +0.0 here; x + 0.0 differs from x only for x = -0.0, and a sum that
 // starts at +0.0 never becomes -0.0 (a sum is -0.0 only if both terms are),
 // so those adds change nothing and are left out.
 __global__ __launch_bounds__(256) void k_acct_srcsum(KParams P, AcctRegions R, const double* __restrict__ term,
                                                      double* __restrict__ acc) {
-  __shared__ double lds[2 * STG_CH * 8];
-  const int l = threadIdx.x;
-  const int r = l / 8, k = l % 8;
-  const int rr = r < ACC_NREG ? r : 0;
-  const int i0 = max(R.ep[rr][HARM_X1DN], 0), i1 = min(R.ep[rr][HARM_X1UP], P.n1 - 1);
-  const int j0 = max(R.ep[rr][HARM_X2DN], 0), j1 = min(R.ep[rr][HARM_X2UP], P.n2 - 1);
+  const int r = blockIdx.x / 8, k = blockIdx.x % 8;
+  const int i0 = max(R.ep[r][HARM_X1DN], 0), i1 = min(R.ep[r][HARM_X1UP], P.n1 - 1);
+  const int j0 = max(R.ep[r][HARM_X2DN], 0), j1 = min(R.ep[r][HARM_X2UP], P.n2 - 1);
+  const int w = max(j1 - j0 + 1, 0), n = max(i1 - i0 + 1, 0) * w;
+  const double* t = term + ((size_t)k * P.n1 + i0) * P.n2 + j0;
   // sourceadd and sourceaddterms[GEOMSOURCE] receive the same terms from the
-  // same start (both zeroed together): one chain serves both
-  double ch[1] = {0};
-  if (l < ACC_NREG * 8) ch[0] = acc[r * REG_D + OFF_SRC + k];
-  const int n2 = P.n2;
-  staged_items<8>(P.n1 * n2, lds, [&](int z, int w) { return term[(size_t)z * 8 + w]; },
-                  [&](int first, int cnt, const double* b) {
-                    if (l < ACC_NREG * 8) box_rows<1>(first, cnt, b, k, n2, i0, i1, j0, j1, ch);
-                  });
-  if (l < ACC_NREG * 8) {
-    acc[r * REG_D + OFF_SRC + k] = ch[0];
-    acc[r * REG_D + OFF_SRCT + k] = ch[0];
+  // same start (both zeroed together): one sum serves both
+  const double s = chain_sum(n, acc[r * REG_D + OFF_SRC + k], [&](int m) {
+    const int i = m / w;
+    return t[(size_t)i * P.n2 + (m - i * w)];
+  });
+  if (threadIdx.x == 0) {
+    acc[r * REG_D + OFF_SRC + k] = s;
+    acc[r * REG_D + OFF_SRCT + k] = s;
   }
 }
 
-// lumvsr (region 0, k = UU): one lane per x1 row, x2 in order
-__global__ void k_acct_lumsum(KParams P, AcctRegions R, const double* __restrict__ term, double* __restrict__ lumvsr) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int* ep = R.ep[0];
-  if (i >= P.n1 || i < ep[HARM_X1DN] || i > ep[HARM_X1UP]) return;
-  const int j0 = max(ep[HARM_X2DN], 0), j1 = min(ep[HARM_X2UP], P.n2 - 1);
-  const double* row = term + (size_t)i * P.n2 * 8 + UU;
-  double l = lumvsr[i];
-  for (int j = j0; j <= j1; j += 16) {
-    double v[16];
+// the serial sum s of n adjacent terms by one wavefront: 256 loads in flight,
+// the terms handed to the chain of additions lane by lane
+__device__ __forceinline__ double row_sum(const double* __restrict__ t, int n, double s) {
+  const int lane = threadIdx.x & 63;
+  for (int m = 0; m < n; m += 256) {
+    double v[4];
 #pragma unroll
-    for (int m = 0; m < 16; m++) v[m] = (j + m <= j1) ? row[(size_t)(j + m) * 8] : 0.0;
+    for (int q = 0; q < 4; q++) v[q] = (m + 64 * q + lane < n) ? t[m + 64 * q + lane] : -0.0;  // x + -0.0 is x
 #pragma unroll
-    for (int m = 0; m < 16; m++)
-      if (j + m <= j1) l += v[m];
+    for (int q = 0; q < 4; q++) {
+      if (m + 64 * q >= n) break;
+#pragma unroll
+      for (int l = 0; l < 64; l++) s += lane_value(v[q], l);
+    }
   }
-  lumvsr[i] = l;
+  return s;
+}
+
+// lumvsr (region 0, k = UU): one wavefront per x1 row, x2 in order
+__global__ __launch_bounds__(64) void k_acct_lumsum(KParams P, AcctRegions R, const double* __restrict__ term,
+                                                    double* __restrict__ lumvsr) {
+  const int i = blockIdx.x;
+  const int* ep = R.ep[0];
+  if (i < ep[HARM_X1DN] || i > ep[HARM_X1UP]) return;
+  const int j0 = max(ep[HARM_X2DN], 0), j1 = min(ep[HARM_X2UP], P.n2 - 1);
+  const double l = row_sum(term + ((size_t)UU * P.n1 + i) * P.n2 + j0, j1 - j0 + 1, lumvsr[i]);
+  if (threadIdx.x == 0) lumvsr[i] = l;
 }
 
 // diag_flux's terms of each boundary face (diag.c:649-803)
@@ -309,10 +462,10 @@ __global__ void k_acct_faceterm(KParams P, AcctRegions R, const int* __restrict_
 // the boundary sums of diag_flux, one lane per (region, dir, quantity):
 // slots 0-7 pdot (then pcum += pdot Dt), 8-63 pdotterms, 64-119 jet2
 // (region 0); boundaries with no flux are zeroed as the reference zeroes them
-__global__ void k_acct_facesum(AcctRegions R, const double* __restrict__ term, double* __restrict__ acc,
+__global__ __launch_bounds__(64) void k_acct_facesum(AcctRegions R, const double* __restrict__ term, double* __restrict__ acc,
                                const DevScalars* __restrict__ ds, double Dt, int dt_from_step) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  constexpr int NS = 8 + 2 * ACC_NFL * 8;
+  constexpr int NS = 8 + 2 * ACC_NFL * 8, AHEAD = 32;
   if (t >= ACC_NREG * 4 * NS) return;
   const int r = t / (4 * NS), dir = (t / NS) % 4, slot = t % NS;
   const bool jet = slot >= 8 + ACC_NFL * 8;
@@ -321,17 +474,20 @@ __global__ void k_acct_facesum(AcctRegions R, const double* __restrict__ term, d
   const int off = R.off[r][dir], len = flux ? R.len[r][dir] : 0;
   const int col = jet ? slot - ACC_NFL * 8 : slot;  // column of the face record
   double s = 0.0;
-  for (int e = off; e < off + len; e += 16) {
-    double v[16], cnd[16];
+  const int cond = jet ? FACE_SLOTS - 1 : col;  // loaded by every lane: no branch between the loads
+  for (int e = off; e < off + len; e += AHEAD) {
+    double v[AHEAD], w[AHEAD];
 #pragma unroll
-    for (int m = 0; m < 16; m++) {
-      const bool in = e + m < off + len;
-      v[m] = in ? term[(size_t)(e + m) * FACE_SLOTS + col] : 0.0;
-      cnd[m] = (in && jet) ? term[(size_t)(e + m) * FACE_SLOTS + FACE_SLOTS - 1] : 1.0;
+    for (int m = 0; m < AHEAD; m++) {
+      const double* f = term + (size_t)min(e + m, off + len - 1) * FACE_SLOTS;
+      v[m] = f[col];
+      w[m] = f[cond];
     }
 #pragma unroll
-    for (int m = 0; m < 16; m++)
-      if (e + m < off + len && cnd[m] != 0.0) s += v[m];
+    for (int m = 0; m < AHEAD; m++) {
+      const bool take = e + m < off + len && (!jet || w[m] != 0.0);
+      s += take ? v[m] : -0.0;  // x + -0.0 is x
+    }
   }
   double* a = acc + r * REG_D;
   if (jet) {
@@ -347,7 +503,7 @@ __global__ void k_acct_facesum(AcctRegions R, const double* __restrict__ term, d
   }
 }
 
-// frdot (diag.c:816-827): the x1 face terms of the interior, then one lane
+// frdot (diag.c:816-827): the x1 face terms of the interior, then one wavefront
 // per (row, quantity) summing over x2
 __global__ void k_acct_frterm(KParams P, AcctRegions R, const double* __restrict__ F1, const double* __restrict__ q1,
                               const double* __restrict__ q2, const double* __restrict__ gF,
@@ -361,24 +517,15 @@ __global__ void k_acct_frterm(KParams P, AcctRegions R, const double* __restrict
 #pragma unroll
   for (int k = 0; k < NPR; k++) ft[k] = f[k] * surface;
   evolve_to_diag(P, face_gdet(P, gF, zidx(P, i, j)), ft, fd);
-  store8(out, i * P.n2 + j, fd);
+#pragma unroll
+  for (int k = 0; k < NPR; k++) out[((size_t)k * P.n1 + i) * P.n2 + j] = fd[k];
 }
 
-__global__ void k_acct_frsum(KParams P, const double* __restrict__ term, double* __restrict__ frdot) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= P.n1 * 8) return;
-  const int i = t / 8, k = t % 8;
-  const double* row = term + (size_t)i * P.n2 * 8 + k;
-  double s = 0;
-  for (int j = 0; j < P.n2; j += 16) {
-    double v[16];
-#pragma unroll
-    for (int m = 0; m < 16; m++) v[m] = (j + m < P.n2) ? row[(size_t)(j + m) * 8] : 0.0;
-#pragma unroll
-    for (int m = 0; m < 16; m++)
-      if (j + m < P.n2) s += v[m];
-  }
-  frdot[t] = s;
+__global__ __launch_bounds__(64) void k_acct_frsum(KParams P, const double* __restrict__ term,
+                                                   double* __restrict__ frdot) {
+  const int i = blockIdx.x / 8, k = blockIdx.x % 8;
+  const double s = row_sum(term + ((size_t)k * P.n1 + i) * P.n2, P.n2, 0.0);
+  if (threadIdx.x == 0) frdot[blockIdx.x] = s;
 }
 
 // |div B| at corner (i,j) (SETFDIVBFLUXCT, global.h:1152-1175), zero on
@@ -692,57 +839,44 @@ __global__ __launch_bounds__(256) void k_acct_fixg(KParams P, const double* __re
   acct_event(P, g, pr0, pfin, slot + 1, P.acct_flag[slot + 1] - 1);
 }
 
-// ordered compaction of the used slots: counts per block of 256, offsets,
-// then each block writes its events at its offset in slot order
+// ordered compaction of the used slots: counts per block of 256, then each block
+// writes its events in slot order behind those of the blocks before it, whose
+// counts it adds up itself (2,317 for a 256x256 grid: no launch between)
 __global__ __launch_bounds__(256) void k_acct_count(int nslots, const int* __restrict__ flag, int* __restrict__ cnt) {
   const int s = blockIdx.x * 256 + threadIdx.x;
   const int c = __syncthreads_count((s < nslots) && flag[s] != 0);
   if (threadIdx.x == 0) cnt[blockIdx.x] = c;
 }
 
-__global__ __launch_bounds__(256) void k_acct_scan(int nblocks, const int* __restrict__ cnt, int* __restrict__ off,
-                                                   int* __restrict__ total) {
-  __shared__ int part[256];
-  const int t = threadIdx.x;
-  const int per = (nblocks + 255) / 256, b0 = t * per, b1 = min(b0 + per, nblocks);
-  int sum = 0;
-  for (int b = b0; b < b1; b++) sum += cnt[b];
-  part[t] = sum;
-  __syncthreads();
-  if (t == 0) {
-    int run = 0;
-    for (int u = 0; u < 256; u++) {
-      const int v = part[u];
-      part[u] = run;
-      run += v;
-    }
-    *total = run;
-  }
-  __syncthreads();
-  int run = part[t];
-  for (int b = b0; b < b1; b++) {
-    off[b] = run;
-    run += cnt[b];
-  }
-}
-
-__global__ __launch_bounds__(256) void k_acct_compact(int nslots, int* __restrict__ flag, const int* __restrict__ off,
+__device__ __forceinline__ int acct_slot_key(int n1, int n2, const AcctRegions& R, int slot, int cc, int finalstep);
+__global__ __launch_bounds__(256) void k_acct_compact(KParams P, AcctRegions R, int nslots, int* __restrict__ flag,
+                                                      const int* __restrict__ cnt, int* __restrict__ total,
                                                       int* __restrict__ list, const double* __restrict__ val,
-                                                      double* __restrict__ cval) {
-  __shared__ int wcount[4];
+                                                      double* __restrict__ cval, int finalstep) {
+  __shared__ int wcount[4], wbefore[4];
+  const bool end = blockIdx.x == gridDim.x - 1;
+  if (cnt[blockIdx.x] == 0 && !end) return;  // block-uniform
   const int s = blockIdx.x * 256 + threadIdx.x;
   const int f = (s < nslots) ? flag[s] : 0;
   const unsigned long long m = __ballot(f != 0);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) wcount[w] = __popcll(m);
-  __syncthreads();
-  if (f != 0) {
-    int pos = off[blockIdx.x] + __popcll(m & ((1ull << lane) - 1ull));
-    for (int v = 0; v < w; v++) pos += wcount[v];
-    list[2 * pos] = s;
-    list[2 * pos + 1] = f - 1;
+  int before = 0;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += 256) before += cnt[b];
 #pragma unroll
-    for (int m = 0; m < 8; m++) cval[(size_t)pos * 8 + m] = val[(size_t)s * 8 + m];
+  for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off);
+  if (lane == 0) {
+    wcount[w] = __popcll(m);
+    wbefore[w] = before;
+  }
+  __syncthreads();
+  before = wbefore[0] + wbefore[1] + wbefore[2] + wbefore[3];
+  if (end && threadIdx.x == 0) *total = before + wcount[0] + wcount[1] + wcount[2] + wcount[3];
+  if (f != 0) {
+    int pos = before + __popcll(m & ((1ull << lane) - 1ull));
+    for (int v = 0; v < w; v++) pos += wcount[v];
+    list[pos] = acct_slot_key(P.n1, P.n2, R, s, f - 1, finalstep);
+#pragma unroll
+    for (int m = 0; m < 8; m++) cval[(size_t)m * nslots + pos] = val[(size_t)s * 8 + m];
     flag[s] = 0;
   }
 }
@@ -803,59 +937,19 @@ struct FixLane {
 };
 constexpr int FIX_LANES = ACC_NREG * 8 * (1 + ACC_NFLOOR);
 
-// the substage's events added in order: lanes 0-23 fladd[r][k], then
-// fladdterms[r][cat][k]; floor and repair events count on the last substage
-__global__ __launch_bounds__(512) void k_acct_merge(KParams P, AcctRegions R, const int* __restrict__ list,
+// the substage's events added in order, a workgroup per accumulator (FixLane);
+// an event that an accumulator does not take is -0.0 to it, which changes no sum
+__global__ __launch_bounds__(256) void k_acct_merge(int nslots, const int* __restrict__ key,
                                                     const int* __restrict__ total, const double* __restrict__ cval,
-                                                    double* __restrict__ acc, int finalstep) {
-  __shared__ double ev_val[2][256 * 8];
-  // an event's key: bit r set when region r holds it, category + 1 above the
-  // region bits; 0 when it does not count on this substage
-  __shared__ int ev_key[2][256];
-  const int t = threadIdx.x;
-  const bool lane = t < FIX_LANES;  // waves 0-3 add, waves 4-7 stage the next 256 events
-  const FixLane L(lane ? t : 0);
-  const int n1 = P.n1, n2 = P.n2;
+                                                    double* __restrict__ acc) {
+  const FixLane L(blockIdx.x);
+  const double* v = cval + (size_t)L.k * nslots;
   double* dst = acc + L.dst();
-  double s = lane ? *dst : 0.0;
-  const int E = *total;
-  const int nch = (E + 255) / 256;
-  const int kmask = L.kmask, kwant = L.kwant;
-  // where an event lies and whether it counts on this substage
-  auto stage = [&](int c, int h) {
-    const int u = t - 256, e = c * 256 + u;
-    if (u < 0 || e >= E) return;
-    ev_key[h][u] = acct_slot_key(n1, n2, R, list[2 * e], list[2 * e + 1], finalstep);
-#pragma unroll
-    for (int m = 0; m < 8; m++) ev_val[h][u * 8 + m] = cval[(size_t)e * 8 + m];
-  };
-  if (nch > 0) stage(0, 0);
-  __syncthreads();
-  for (int c = 0; c < nch; c++) {
-    const int h = c & 1;
-    if (t >= 256) {
-      if (c + 1 < nch) stage(c + 1, h ^ 1);
-    } else if (lane) {
-      const int cnt = min(256, E - c * 256);
-      for (int m0 = 0; m0 < cnt; m0 += 8) {  // eight events read ahead of the adds
-        int kk[8];
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int m = min(m0 + u, 255);
-          kk[u] = (m0 + u < cnt) ? ev_key[h][m] : 0;
-          v[u] = ev_val[h][m * 8 + L.k];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const bool take = (kk[u] & kmask) == kwant;
-          if (take) s += v[u];
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (lane) *dst = s;
+  const double s = chain_sum(*total, *dst, [&](int m) {
+    const double x = v[m];  // loaded whatever its key is
+    return (key[m] & L.kmask) == L.kwant ? x : -0.0;
+  });
+  if (threadIdx.x == 0) *dst = s;
 }
 
 // ---- tree sums (HARM_ACCT_TREE) ----
@@ -888,7 +982,8 @@ __global__ __launch_bounds__(256) void k_acct_srcsum_part(KParams P, AcctRegions
   for (int z = blockIdx.x * 256 + threadIdx.x; z < nzz; z += TREE_SRC_NB * 256) {
     const int i = z / P.n2, j = z - i * P.n2;
     double v[NPR];
-    load8(term, z, v);
+#pragma unroll
+    for (int k = 0; k < NPR; k++) v[k] = term[(size_t)k * nzz + z];
 #pragma unroll
     for (int r = 0; r < ACC_NREG; r++) {
       const bool in = i >= R.ep[r][HARM_X1DN] && i <= R.ep[r][HARM_X1UP] && j >= R.ep[r][HARM_X2DN] &&
@@ -990,10 +1085,13 @@ static int acct_alloc(harm_ctx* c) {
   if (e == hipSuccess) e = hipMalloc(&a->flag, (size_t)a->nslots * sizeof(int));
   if (e == hipSuccess) e = hipMemset(a->flag, 0, (size_t)a->nslots * sizeof(int));
   if (e == hipSuccess) e = hipMalloc(&a->val, (size_t)a->nslots * 8 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&a->list, (size_t)a->nslots * 2 * sizeof(int));
+  if (e == hipSuccess) e = hipMalloc(&a->list, (size_t)a->nslots * sizeof(int));
   if (e == hipSuccess) e = hipMalloc(&a->cval, (size_t)a->nslots * 8 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&a->cnt, (size_t)a->nblocks * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&a->off, (size_t)a->nblocks * sizeof(int));
+  if (e == hipSuccess) e = hipMalloc(&a->sterm, (size_t)n1 * n2 * 8 * sizeof(double));
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&a->side, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&a->fork, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&a->join, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&a->total, sizeof(int));
   if (e == hipSuccess)
     e = hipMalloc(&a->part, (size_t)std::max(TREE_SRC_NB * TREE_SRC_N, a->nblocks * FIX_LANES) * sizeof(double));
@@ -1006,9 +1104,12 @@ static void acct_free(harm_ctx* c) {
   AcctState* a = c->acct;
   if (!a) return;
   void* bufs[16] = {a->acc,  a->frdot, a->lumvsr, a->scratch, a->out, a->faces, a->pre,  a->uin,
-                     a->flag, a->val,   a->list,   a->cval,    a->cnt, a->off,   a->total, a->part};
+                     a->flag, a->val,   a->list,   a->cval,    a->cnt, a->sterm, a->total, a->part};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  if (a->fork) (void)hipEventDestroy(a->fork);
+  if (a->join) (void)hipEventDestroy(a->join);
+  if (a->side) (void)hipStreamDestroy(a->side);
   delete a;
   c->acct = nullptr;
 }
@@ -1020,18 +1121,36 @@ static int acct_source(harm_ctx* c, int pi, int pb, int pf) {
   const int pbs = (pf == pb) ? pi : pb;
   const dim3 b(64, 4);
   hipLaunchKernelGGL(k_acct_srcterm, grid2(c->kp.n2, c->kp.n1, b), b, 0, c->stream, c->kp, a->R, c->arr[pbs], c->gC,
-                     c->gConn, c->ds, a->scratch);
+                     c->gConn, c->ds, a->sterm);
+  hipStream_t st = c->stream;
   if (a->tree) {
-    hipLaunchKernelGGL(k_acct_srcsum_part, dim3(TREE_SRC_NB), dim3(256), 0, c->stream, c->kp, a->R, a->scratch,
+    hipLaunchKernelGGL(k_acct_srcsum_part, dim3(TREE_SRC_NB), dim3(256), 0, c->stream, c->kp, a->R, a->sterm,
                        a->part);
     hipLaunchKernelGGL(k_acct_tree_final, dim3(TREE_SRC_N), dim3(256), 0, c->stream, a->part, TREE_SRC_NB,
                        TREE_SRC_N, 0, a->acc);
   } else {
-    hipLaunchKernelGGL(k_acct_srcsum, dim3(1), dim3(256), 0, c->stream, c->kp, a->R, a->scratch, a->acc);
+    // The slowest ordered chain (the x2 momentum's terms change sign over the
+    // equator and pass all binades) is 65,536 dependent additions for a 256x256
+    // grid, 198 us on one compute unit: it runs beside the rest of the step.
+    HIPCHK(hipEventRecord(a->fork, c->stream));
+    HIPCHK(hipStreamWaitEvent(a->side, a->fork, 0));
+    st = a->side;
+    hipLaunchKernelGGL(k_acct_srcsum, dim3(ACC_NREG * 8), dim3(256), 0, st, c->kp, a->R, a->sterm, a->acc);
   }
-  hipLaunchKernelGGL(k_acct_lumsum, dim3((c->kp.n1 + 63) / 64), dim3(64), 0, c->stream, c->kp, a->R, a->scratch,
-                     a->lumvsr);
+  hipLaunchKernelGGL(k_acct_lumsum, dim3(c->kp.n1), dim3(64), 0, st, c->kp, a->R, a->sterm, a->lumvsr);
+  if (!a->tree) {
+    HIPCHK(hipEventRecord(a->join, a->side));
+    a->forked = true;
+  }
   HIPCHK(hipGetLastError());
+  return 0;
+}
+// what acct_source forked off is part of the step again
+static int acct_join(harm_ctx* c) {
+  AcctState* a = c->acct;
+  if (!a->forked) return 0;
+  a->forked = false;
+  HIPCHK(hipStreamWaitEvent(c->stream, a->join, 0));
   return 0;
 }
 
@@ -1068,12 +1187,10 @@ static int acct_merge(harm_ctx* c, int finalstep) {
     return 0;
   }
   hipLaunchKernelGGL(k_acct_count, dim3(a->nblocks), dim3(256), 0, c->stream, a->nslots, a->flag, a->cnt);
-  hipLaunchKernelGGL(k_acct_scan, dim3(1), dim3(256), 0, c->stream, a->nblocks, a->cnt, a->off, a->total);
-  hipLaunchKernelGGL(k_acct_compact, dim3(a->nblocks), dim3(256), 0, c->stream, a->nslots, a->flag, a->off, a->list,
-                     a->val, a->cval);
-  static_assert(FIX_LANES <= 256, "one workgroup holds every accumulator lane");
-  hipLaunchKernelGGL(k_acct_merge, dim3(1), dim3(512), 0, c->stream, c->kp, a->R, a->list, a->total, a->cval, a->acc,
-                     finalstep);
+  hipLaunchKernelGGL(k_acct_compact, dim3(a->nblocks), dim3(256), 0, c->stream, c->kp, a->R, a->nslots, a->flag,
+                     a->cnt, a->total, a->list, a->val, a->cval, finalstep);
+  hipLaunchKernelGGL(k_acct_merge, dim3(FIX_LANES), dim3(256), 0, c->stream, a->nslots, a->list, a->total, a->cval,
+                     a->acc);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1094,7 +1211,7 @@ static int acct_flux(harm_ctx* c, double Dt) {
   const dim3 b(64, 4);
   hipLaunchKernelGGL(k_acct_frterm, grid2(c->kp.n2, c->kp.n1, b), b, 0, c->stream, c->kp, a->R, c->arr[HARM_F1],
                      c->q1, c->q2, c->gF, c->gC, a->scratch);
-  hipLaunchKernelGGL(k_acct_frsum, dim3((c->kp.n1 * 8 + 63) / 64), dim3(64), 0, c->stream, c->kp, a->scratch,
+  hipLaunchKernelGGL(k_acct_frsum, dim3(c->kp.n1 * 8), dim3(64), 0, c->stream, c->kp, a->scratch,
                      a->frdot);
   HIPCHK(hipGetLastError());
   return 0;

@@ -38,6 +38,7 @@
 #include <type_traits>
 #include "harm_device.h"
 #include "harm_fast.h"
+#include "harm_chain.h"
 #include "harm_tangent.h"
 #include "harm_adjoint.h"
 #include "harm_eno.h"
@@ -2958,6 +2959,7 @@ static bool acct_on(const harm_ctx* c);
 static void acct_set_on(harm_ctx* c, bool on);
 static int acct_source(harm_ctx* c, int pi, int pb, int pf);
 static int acct_flux(harm_ctx* c, double Dt);
+static int acct_join(harm_ctx* c);
 static int acct_faces(harm_ctx* c, int pb);
 static int acct_zones(harm_ctx* c, int finalstep);
 static int acct_merge(harm_ctx* c, int finalstep);
@@ -3714,7 +3716,7 @@ static int enqueue_step(harm_ctx* c) {
   }
   // step_ch.c:143-153 the current, :160 diag_flux, with the step's dt
   if (cur_on(c) && cur_step(c)) return 1;
-  if (acct_on(c) && acct_flux(c, -1.0)) return 1;
+  if (acct_on(c) && (acct_flux(c, -1.0) || acct_join(c))) return 1;
   return 0;
 }
 

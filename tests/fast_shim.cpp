@@ -1,7 +1,9 @@
 // fast_shim.cpp -- TEST INFRASTRUCTURE.  A host-only build of the face physics
-// (harm_device.h) and of its shorter form (harm_fast.h), so that the CPU tests
-// can compare the two.  Built by the tests with
+// (harm_device.h), of its shorter form (harm_fast.h) and of the serial sum by
+// runs (harm_chain.h), so that the CPU tests can compare them with the plain
+// forms.  Built by the tests with
 //   hipcc -x hip --offload-host-only -O2 -ffp-contract=off -shared -fPIC
+#include "../harm_ramt_amd/csrc/harm_chain.h"
 #include "../harm_ramt_amd/csrc/harm_fast.h"
 
 using namespace harm;
@@ -71,4 +73,41 @@ void shim_quotients(long n, const double* a, const double* d, double* q) {
     q[m] = out[0];
   }
 }
+
+// the sum s + t[0] + t[1] + ... (n a multiple of 16) by runs of 16, their maps
+// composed from each start on as a scan does; *by_map: the runs whose map held
+double shim_chain(long n, const double* t, double s, long* by_map) {
+  const long runs = n / 16;
+  *by_map = 0;
+  for (long r = 0; r < runs;) {
+    const ChainScale c(s);
+    double d0 = 0., d1 = 0.;
+    int q = 2;
+    long k = r;
+    if (c.e >= 0)
+      for (; k < runs; k++) {
+        double v[16];
+        memcpy(v, t + 16 * k, sizeof(v));
+        ChainMap m = chain_map(c, v);
+        const double at = fabs(s) + ((chain_bits(s) & 1) ? d1 : d0);
+        if (!chain_holds(c, at, m.mn, m.mx)) break;
+        double a0 = m.d0, a1 = m.d1;
+        int aq = m.q;
+        chain_then(d0, d1, q, a0, a1, aq);
+        d0 = a0;
+        d1 = a1;
+        q = aq;
+      }
+    *by_map += k - r;
+    if (k > r) {
+      const double end = fabs(s) + ((chain_bits(s) & 1) ? d1 : d0);
+      s = (chain_bits(s) >> 63) ? -end : end;
+    }
+    if (k < runs)
+      for (int m = 0; m < 16; m++) s += t[16 * k + m];
+    r = k + 1;
+  }
+  return s;
+}
+
 }
