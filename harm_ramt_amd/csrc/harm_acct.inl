@@ -195,12 +195,6 @@ __device__ __forceinline__ void chain_step(double& d0, double& d1, int& q) {
   const int aq = __builtin_amdgcn_update_dpp(2, q, CTRL, ROWS, 0xf, false);
   chain_then(a0, a1, aq, d0, d1, q);
 }
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)u, lane);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(u >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
 // the runs [r0, r1) of a chunk, term by term
 __device__ __forceinline__ double chain_serial(const double* b, int r0, int r1, double s) {
   double v[CH_RUN];
@@ -356,24 +350,6 @@ __global__ __launch_bounds__(256) void k_acct_srcsum(KParams P, AcctRegions R, c
     acc[r * REG_D + OFF_SRC + k] = s;
     acc[r * REG_D + OFF_SRCT + k] = s;
   }
-}
-
-// the serial sum s of n adjacent terms by one wavefront: 256 loads in flight,
-// the terms handed to the chain of additions lane by lane
-__device__ __forceinline__ double row_sum(const double* __restrict__ t, int n, double s) {
-  const int lane = threadIdx.x & 63;
-  for (int m = 0; m < n; m += 256) {
-    double v[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = (m + 64 * q + lane < n) ? t[m + 64 * q + lane] : -0.0;  // x + -0.0 is x
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      if (m + 64 * q >= n) break;
-#pragma unroll
-      for (int l = 0; l < 64; l++) s += lane_value(v[q], l);
-    }
-  }
-  return s;
 }
 
 // lumvsr (region 0, k = UU): one wavefront per x1 row, x2 in order

@@ -23,17 +23,23 @@ struct AdjRK {
   int last;
 };
 
+// (loaded whether the zone is inside or not: no branch between a face's loads)
 __device__ __forceinline__ double adj_ld(const KParams& P, const double* ldU, int i, int j, int k) {
-  return (i >= 0 && i < P.n1 && j >= 0 && j < P.n2) ? ldU[(size_t)zidx(P, i, j) * 8 + k] : 0.;
+  const bool in = i >= 0 && i < P.n1 && j >= 0 && j < P.n2;
+  const double v = ldU[(size_t)(in ? zidx(P, i, j) : 0) * 8 + k];
+  return in ? v : 0.;
 }
 
 // The adjoint's steps are replayed as HIP graphs; the step index lives on
 // the device (ctr[0] = step n, ctr[1] = first step of the segment), so one
 // captured graph serves every step.
 
-// dt of step ctr[0]: record (before the step) or impose
-__global__ void k_adj_dt(DevScalars* ds, double* dts, const int* ctr, int impose) {
-  const int n = ctr[0];
+// (step of a graph: its place there, rel, beside ctr[0], which one launch
+// advances at the graph's end)
+
+// dt of step ctr[0] + rel: record (before the step) or impose
+__global__ void k_adj_dt(DevScalars* ds, double* dts, const int* ctr, int rel, int impose) {
+  const int n = ctr[0] + rel;
   if (impose) ds->dt = dts[n];
   else dts[n] = ds->dt;
 }
@@ -45,26 +51,57 @@ __global__ void k_adj_setctr(int* ctr, int n, int n0) {
 
 __global__ void k_adj_next(int* ctr, int delta) { ctr[0] += delta; }
 
-// substage state s of step ctr[0] within its segment's store
-__device__ __forceinline__ size_t adj_state(const int* ctr, int nto, int s, size_t nz8) {
-  return ((size_t)(ctr[0] - ctr[1]) * nto + s) * nz8;
-}
+// a substage's place in the segment's store: state s of step ctr[0] + rel
+struct AdjAt {
+  const double* seg;
+  const int* ctr;
+  int nto, s, rel;
+  size_t nz8;
+  __device__ __forceinline__ int step() const { return ctr[0] + rel; }
+  __device__ __forceinline__ size_t offset() const { return ((size_t)(step() - ctr[1]) * nto + s) * nz8; }
+  __device__ __forceinline__ const double* before() const { return seg + offset(); }        // the substage's pb
+  __device__ __forceinline__ const double* after() const { return seg + offset() + nz8; }   // its pf
+};
 
-// store the state after substage `to` (state to+1 of the step)
-__global__ void k_adj_store(const double* __restrict__ src, double* __restrict__ seg, const int* __restrict__ ctr,
-                            int nto, int to, size_t nz8) {
-  double* dst = seg + adj_state(ctr, nto, to + 1, nz8);
-  const size_t n2 = nz8 / 2;
+// store the state at `at`
+__global__ void k_adj_store(const double* __restrict__ src, double* __restrict__ seg, AdjAt at) {
+  double* dst = seg + at.offset();
+  const size_t n2 = at.nz8 / 2;
   const double2* s2 = reinterpret_cast<const double2*>(src);
   double2* d2 = reinterpret_cast<double2*>(dst);
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n2; t += (size_t)gridDim.x * blockDim.x)
     d2[t] = s2[t];
 }
 
-// slot[0] = pb of substage s (the state before it), slot[1] = its pf
-__global__ void k_adj_slot(const double* seg, const int* ctr, int nto, int s, size_t nz8, const double** slot) {
-  slot[0] = seg + adj_state(ctr, nto, s, nz8);
-  slot[1] = slot[0] + nz8;
+// periodic bound_prim transposed, at interior zone (i,j): what k_adj_bt_x2 and
+// k_adj_bt_x1 leave there, in their order (ghosts below, then above)
+__device__ __forceinline__ void adj_fold_x2(const KParams& P, const double* __restrict__ lp, int i, int j, double* v) {
+  load8(lp, zidx(P, i, j), v);
+  double g[NPR];
+  if (j >= P.n2 - NG) {
+    load8(lp, zidx(P, i, j - P.n2), g);
+#pragma unroll
+    for (int k = 0; k < NPR; k++) v[k] += g[k];
+  }
+  if (j < NG) {
+    load8(lp, zidx(P, i, j + P.n2), g);
+#pragma unroll
+    for (int k = 0; k < NPR; k++) v[k] += g[k];
+  }
+}
+__device__ __forceinline__ void adj_fold(const KParams& P, const double* __restrict__ lp, int i, int j, double* v) {
+  adj_fold_x2(P, lp, i, j, v);
+  double g[NPR];
+  if (i >= P.n1 - NG) {
+    adj_fold_x2(P, lp, i - P.n1, j, g);
+#pragma unroll
+    for (int k = 0; k < NPR; k++) v[k] += g[k];
+  }
+  if (i < NG) {
+    adj_fold_x2(P, lp, i + P.n1, j, g);
+#pragma unroll
+    for (int k = 0; k < NPR; k++) v[k] += g[k];
+  }
 }
 
 // periodic bound_prim transposed: x2 ghosts (all i) fold into their sources,
@@ -98,12 +135,15 @@ __global__ void k_adj_bt_x1(KParams P, double* lp) {
   }
 }
 
-// seed: lambda_N = d(sum 0.5 b^2 gdet dx1 dx2)/dp_N on the interior, and the
-// functional's row sums (summed on the host in a fixed order)
-__global__ void k_adj_seed_bsq(KParams P, const double* p, const double* gC, double* lp, double* rowsum) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y * blockDim.y + threadIdx.y;
-  if (i >= P.n1 + NG || j >= P.n2 + NG || i < -NG) return;
+// seed: lambda_N = d(sum 0.5 b^2 gdet dx1 dx2)/dp_N on the interior, zero in
+// the ghosts, and the functional's terms [n1][n2], whose row sums follow (the
+// host sums these in a fixed order)
+__global__ __launch_bounds__(256) void k_adj_seed_bsq(KParams P, const double* __restrict__ p,
+                                                      const double* __restrict__ gC, double* __restrict__ lp,
+                                                      double* __restrict__ term) {
+  const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x) - NG;
+  const int i = (int)(blockIdx.y * blockDim.y + threadIdx.y) - NG;
+  if (i >= P.n1 + NG || j >= P.n2 + NG) return;
   const int z = zidx(P, i, j);
   double l[NPR] = {0., 0., 0., 0., 0., 0., 0., 0.};
   if (i >= 0 && i < P.n1 && j >= 0 && j < P.n2) {
@@ -114,38 +154,38 @@ __global__ void k_adj_seed_bsq(KParams P, const double* p, const double* gC, dou
     double pr[NPR];
     load8(p, z, pr);
     bsq_rev(pr, g, g.gdet * P.dx1 * P.dx2, l);
+    State q;
+    get_state(pr, g, q);
+    term[(size_t)i * P.n2 + j] = 0.5 * dot4(q.bcon, q.bcov) * g.gdet * P.dx1 * P.dx2;
   }
   store8(lp, z, l);
-  if (j == 0 && i >= 0 && i < P.n1) {
-    double acc = 0.;
-    for (int jj = 0; jj < P.n2; jj++) {
-      const int zz = zidx(P, i, jj);
-      double gc[36];
-      load_cent(P, gC, zz, gc);
-      GeoU g;
-      geo_from_cent(gc, g);
-      double pr[NPR];
-      load8(p, zz, pr);
-      State q;
-      get_state(pr, g, q);
-      acc += 0.5 * dot4(q.bcon, q.bcov) * g.gdet * P.dx1 * P.dx2;
-    }
-    rowsum[i] = acc;
-  }
 }
+__global__ __launch_bounds__(64) void k_adj_rowsum(KParams P, const double* __restrict__ term,
+                                                   double* __restrict__ rowsum) {
+  const double s = row_sum(term + (size_t)blockIdx.x * P.n2, P.n2, 0.);
+  if (threadIdx.x == 0) rowsum[blockIdx.x] = s;
+}
+
+// The reverse substage: 128x128 zones are 256 wavefronts, one a compute unit, so
+// each kernel is a wavefront's chain (and 4 us of launch): workgroups of one or
+// two wavefronts over the zones as one line (64 x 4 blocks crowded a quarter of
+// the units' load paths and left lanes beyond the columns), and no launches of
+// their own for the transposed fills, the EMFs and the pointers.  us a substage
+// of a 128x128 Orszag-Tang gradient, before -> after: 62 -> 36.6 (zone 11.4 ->
+// 9.5, face 15.1 -> 15.7 with the EMFs, gather 17.3 -> 11.3 with two wavefronts).
 
 // inversion (implicit-function theorem) + RK combination, interior zones
 template <int LIMC, int FMC>
-__global__ __launch_bounds__(256) void k_adj_zone(KParams P0, AdjRK R, const double* const* __restrict__ slot, const double* __restrict__ dts,
-                           const int* __restrict__ ctr, const double* __restrict__ gC,
-                           const double* __restrict__ lp, double* __restrict__ lunew, double* __restrict__ lulast,
-                           double* __restrict__ lUi, double* __restrict__ ldU, int* __restrict__ nonsmooth) {
+__global__ __launch_bounds__(64) void k_adj_zone(KParams P0, AdjRK R, AdjAt at, const double* __restrict__ dts,
+                                                 const double* __restrict__ gC, const double* __restrict__ lp,
+                                                 double* __restrict__ lunew, double* __restrict__ lulast,
+                                                 double* __restrict__ lUi, double* __restrict__ ldU,
+                                                 int* __restrict__ nonsmooth) {
   const KParams P = specialize<LIMC, HARM_EOMGRMHD, FMC>(P0);
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y * blockDim.y + threadIdx.y;
-  if (i >= P.n1 || j >= P.n2) return;
-  const double* __restrict__ pf = slot[1];
-  R.dt = dts[ctr[0]];
+  const int id = blockIdx.x * 64 + threadIdx.x, i = id / P.n2, j = id % P.n2;
+  if (i >= P.n1) return;
+  const double* __restrict__ pf = at.after();
+  R.dt = dts[at.step()];
   const int z = zidx(P, i, j);
   double gc[36];
   load_cent(P, gC, z, gc);
@@ -153,7 +193,7 @@ __global__ __launch_bounds__(256) void k_adj_zone(KParams P0, AdjRK R, const dou
   geo_from_cent(gc, g);
   double p[NPR], lpf[NPR];
   load8(pf, z, p);
-  load8(lp, z, lpf);
+  adj_fold(P, lp, i, j, lpf);
   int ns = 0;
   if (P.eomtype == 0) {  // fixup1zone floors on their active branch
     double fr = gc[33], fu = gc[34];
@@ -188,15 +228,12 @@ __global__ __launch_bounds__(256) void k_adj_zone(KParams P0, AdjRK R, const dou
   if (ns) atomicAdd(nonsmooth, ns);
 }
 
-// corner EMF adjoints (flux-CT transposed), corners i in [0,N1], j in [0,N2]
-__global__ void k_adj_emf(KParams P, const double* __restrict__ ldU, double* __restrict__ lemf) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y * blockDim.y + threadIdx.y;
-  if (i > P.n1 || j > P.n2) return;
+// corner EMF adjoint (flux-CT transposed) at corner (i,j), i in [0,N1], j in [0,N2]
+__device__ __forceinline__ double adj_emf(const KParams& P, const double* __restrict__ ldU, int i, int j) {
   const double idx1 = 1.0 / P.dx1, idx2 = 1.0 / P.dx2;
   auto f1b = [&](int a, int b) { return (adj_ld(P, ldU, a, b, B2) - adj_ld(P, ldU, a - 1, b, B2)) * idx1; };
   auto f2b = [&](int a, int b) { return (adj_ld(P, ldU, a, b, B1) - adj_ld(P, ldU, a, b - 1, B1)) * idx2; };
-  lemf[zidx(P, i, j)] = 0.5 * (f1b(i, j) + f1b(i, j - 1)) - 0.5 * (f2b(i, j) + f2b(i - 1, j));
+  return 0.5 * (f1b(i, j) + f1b(i, j - 1)) - 0.5 * (f2b(i, j) + f2b(i - 1, j));
 }
 
 // face adjoints: flux adjoint from the divergence (and CT), then the face
@@ -205,8 +242,7 @@ __global__ void k_adj_emf(KParams P, const double* __restrict__ ldU, double* __r
 template <int DIR>
 __device__ __forceinline__ void adj_face(const KParams& P, const double* __restrict__ pb,
                                          const double* __restrict__ gF, const double* __restrict__ gC,
-                                         const double* __restrict__ ldU, const double* __restrict__ lemf,
-                                         double* __restrict__ lf, int i, int j, int& ns) {
+                                         const double* __restrict__ ldU, double* __restrict__ lf, int i, int j, int& ns) {
   const int zstride = (DIR == 1) ? P.N2M : 1;
   const int z0 = zidx(P, i, j);
   const double idx = 1.0 / ((DIR == 1) ? P.dx1 : P.dx2);
@@ -219,8 +255,8 @@ __device__ __forceinline__ void adj_face(const KParams& P, const double* __restr
   load_geo_face(P, gF, z0, g);
   if (P.fluxb == HARM_FLUXCTTOTH) {
     auto le = [&](int a, int b) {
-      return (a >= 0 && a <= P.n1 && b >= 0 && b <= P.n2) ? geo_entry(P, gC, GC_GDETC, zidx(P, a, b)) * lemf[zidx(P, a, b)]
-                                                           : 0.;
+      const double v = geo_entry(P, gC, GC_GDETC, zidx(P, a, b)) * adj_emf(P, ldU, a, b);
+      return (a >= 0 && a <= P.n1 && b >= 0 && b <= P.n2) ? v : 0.;
     };
     if (DIR == 1) {
       Fob[B1] = 0.;
@@ -248,24 +284,20 @@ __device__ __forceinline__ void adj_face(const KParams& P, const double* __restr
 }
 
 template <int LIMC, int FMC>
-__global__ __launch_bounds__(256) void k_adj_face(KParams P0, const double* const* __restrict__ slot,
-                                                  const double* __restrict__ gF, const double* __restrict__ gC,
-                                                  const double* __restrict__ ldU, const double* __restrict__ lemf,
-                                                  double* __restrict__ lf1, double* __restrict__ lf2,
-                                                  int* __restrict__ nonsmooth) {
+__global__ __launch_bounds__(64) void k_adj_face(KParams P0, AdjAt at, const double* __restrict__ gF,
+                                                 const double* __restrict__ gC, const double* __restrict__ ldU,
+                                                 double* __restrict__ lf1, double* __restrict__ lf2,
+                                                 int* __restrict__ nonsmooth) {
   const KParams P = specialize<LIMC, HARM_EOMGRMHD, FMC>(P0);
-  const double* __restrict__ pb = slot[0];
-  const int dir = 1 + blockIdx.z;
-  const int jf = blockIdx.x * blockDim.x + threadIdx.x;
-  const int ifc = blockIdx.y * blockDim.y + threadIdx.y;
-  const size_t nz = (size_t)(P.n1 + 2 * NG) * P.N2M;
+  const double* __restrict__ pb = at.before();
+  const int id = blockIdx.x * 64 + threadIdx.x;
   int ns = 0;
-  if (dir == 1) {
-    const int i = ifc, j = jf - 1;
-    if (i <= P.n1 && j <= P.n2) adj_face<1>(P, pb, gF, gC, ldU, lemf, lf1, i, j, ns);
+  if (blockIdx.y == 0) {
+    const int i = id / (P.n2 + 2), j = id % (P.n2 + 2) - 1;
+    if (i <= P.n1) adj_face<1>(P, pb, gF, gC, ldU, lf1, i, j, ns);
   } else {
-    const int i = ifc - 1, j = jf;
-    if (i <= P.n1 && j <= P.n2) adj_face<2>(P, pb, gF + nz * GF, gC, ldU, lemf, lf2, i, j, ns);
+    const int i = id / (P.n2 + 1) - 1, j = id % (P.n2 + 1);
+    if (i <= P.n1) adj_face<2>(P, pb, gF + (size_t)P.nz * GF, gC, ldU, lf2, i, j, ns);
   }
   if (ns) atomicAdd(nonsmooth, ns);
 }
@@ -273,49 +305,44 @@ __global__ __launch_bounds__(256) void k_adj_face(KParams P0, const double* cons
 // gather: adjoint of every zone of pb from the face-state adjoints of the
 // faces whose reconstruction stencil holds it (pl(f) = p(f-1) + dq(f-1)/2,
 // pr(f) = p(f) - dq(f)/2, dq on the limiter's branch), plus the source term
+// A wavefront a direction; the first takes the other's sum and the source term.
 template <int LIMC, int FMC>
-__global__ __launch_bounds__(256) void k_adj_gather(KParams P0, const double* const* __restrict__ slot,
-                                                    const double* __restrict__ gC, const double* __restrict__ gConn,
-                                                    const double* __restrict__ ldU, const double* __restrict__ lf1,
-                                                    const double* __restrict__ lf2, double* __restrict__ lp) {
+__global__ __launch_bounds__(128) void k_adj_gather(KParams P0, AdjAt at, const double* __restrict__ gC,
+                                                    const double* __restrict__ gConn, const double* __restrict__ ldU,
+                                                    const double* __restrict__ lf1, const double* __restrict__ lf2,
+                                                    double* __restrict__ lp) {
   const KParams P = specialize<LIMC, HARM_EOMGRMHD, FMC>(P0);
-  const double* __restrict__ pb = slot[0];
-  const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x) - NG;
-  const int i = (int)(blockIdx.y * blockDim.y + threadIdx.y) - NG;
-  if (i > P.n1 + NG - 1 || j > P.n2 + NG - 1) return;
-  const int z = zidx(P, i, j);
+  __shared__ double x2[NPR][64];
+  const double* __restrict__ pb = at.before();
+  const int tx = threadIdx.x, w2 = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int z = min((int)blockIdx.x * 64 + tx, P.nz - 1);  // lanes beyond the last zone repeat it
+  const int i = z / P.N2M - NG, j = z % P.N2M - NG;
   double l[NPR];
-#pragma unroll
-  for (int k = 0; k < NPR; k++) l[k] = 0.;
-#pragma unroll
-  for (int dir = 1; dir <= 2; dir++) {
-    const double* lf = (dir == 1) ? lf1 : lf2;
-    const int c = (dir == 1) ? i : j;                 // position along the line
-    const int nmax = ((dir == 1) ? P.n1 : P.n2) + NG;  // one past the last zone
-    const int stride = (dir == 1) ? P.N2M : 1;
+  {
+    const double* lf = w2 ? lf2 : lf1;
+    const int c = w2 ? j : i;                  // position along the line
+    const int nmax = (w2 ? P.n2 : P.n1) + NG;  // one past the last zone
+    const int stride = w2 ? 1 : P.N2M;
     // lpl(f) = lf[2 z(f)], lpr(f) = lf[2 z(f) + 1]; faces exist for f in
     // [-NG, nmax).  The line's zones c-2..c+2 and faces c-1..c+2 are loaded
-    // once, as whole records; out-of-range entries are never used.
+    // once, as whole records, all before any is used: beyond the line its end's
+    // (zones, never used) or zero (faces).
     double pz[5][NPR], fl[4][NPR], fr[4][NPR];
 #pragma unroll
-    for (int m = 0; m < 5; m++) {
-      const int w = c - 2 + m;
-      if (w >= -NG && w < nmax) {
-        load8(pb, z + (w - c) * stride, pz[m]);
-      } else {
+    for (int m = 0; m < 5; m++) load8(pb, z + (min(max(c - 2 + m, -NG), nmax - 1) - c) * stride, pz[m]);
 #pragma unroll
-        for (int k = 0; k < NPR; k++) pz[m][k] = 0.;
-      }
+    for (int m = 0; m < 4; m++) {
+      const int f = min(max(c - 1 + m, -NG), nmax - 1);
+      load8(lf, 2 * (z + (f - c) * stride), fl[m]);
+      load8(lf, 2 * (z + (f - c) * stride) + 1, fr[m]);
     }
 #pragma unroll
     for (int m = 0; m < 4; m++) {
-      const int f = c - 1 + m;
-      if (f >= -NG && f < nmax) {
-        load8(lf, 2 * (z + (f - c) * stride), fl[m]);
-        load8(lf, 2 * (z + (f - c) * stride) + 1, fr[m]);
-      } else {
+      const bool in = c - 1 + m >= -NG && c - 1 + m < nmax;
 #pragma unroll
-        for (int k = 0; k < NPR; k++) fl[m][k] = fr[m][k] = 0.;
+      for (int k = 0; k < NPR; k++) {
+        fl[m][k] = in ? fl[m][k] : 0.;
+        fr[m][k] = in ? fr[m][k] : 0.;
       }
     }
 #pragma unroll
@@ -324,24 +351,33 @@ __global__ __launch_bounds__(256) void k_adj_gather(KParams P0, const double* co
 #pragma unroll
       for (int dw = -1; dw <= 1; dw++) {
         const int w = c + dw;
-        if (w - 1 < -NG || w + 1 >= nmax) continue;
         const double ldq = 0.5 * fl[dw + 2][k] - 0.5 * fr[dw + 1][k];  // lpl(w+1), lpr(w)
-        if (ldq == 0.) continue;
         double cl, cc, cr;
         slope3_coef(P.lim, pz[dw + 1][k], pz[dw + 2][k], pz[dw + 3][k], cl, cc, cr);
-        acc += ((dw == -1) ? cr : ((dw == 0) ? cc : cl)) * ldq;
+        const double more = acc + ((dw == -1) ? cr : ((dw == 0) ? cc : cl)) * ldq;
+        acc = (w - 1 < -NG || w + 1 >= nmax || ldq == 0.) ? acc : more;
       }
-      l[k] += acc;
+      l[k] = 0. + acc;
     }
   }
-  if (i >= 0 && i < P.n1 && j >= 0 && j < P.n2) {
-    double gc[36];
+  if (w2) {
+#pragma unroll
+    for (int k = 0; k < NPR; k++) x2[k][tx] = l[k];
+  }
+  const bool zone = i >= 0 && i < P.n1 && j >= 0 && j < P.n2;
+  double gc[36], pr[NPR], ldu[NPR];
+  if (!w2) {
     load_cent(P, gC, z, gc);
-    GeoU g;
-    geo_from_cent(gc, g);
-    double pr[NPR], ldu[NPR];
     load8(pb, z, pr);
     load8(ldU, z, ldu);
+  }
+  __syncthreads();
+  if (w2 || (int)blockIdx.x * 64 + tx >= P.nz) return;
+#pragma unroll
+  for (int k = 0; k < NPR; k++) l[k] += x2[k][tx];
+  if (zone) {
+    GeoU g;
+    geo_from_cent(gc, g);
     source_rev_at(P, pr, g, [&](int e) { return conn_entry(P, gConn, conn_sym(e), z); }, ldu, l);
   }
   store8(lp, z, l);
@@ -349,13 +385,12 @@ __global__ __launch_bounds__(256) void k_adj_gather(KParams P0, const double* co
 
 // Ui = U(p_n) transposed into the adjoint of p_n; clears lUi, lunew, lulast
 // (the adjoints of the substage accumulators, which start each step at zero)
-__global__ __launch_bounds__(256) void k_adj_ui(KParams P, const double* const* __restrict__ slot, const double* __restrict__ gC,
+__global__ __launch_bounds__(64) void k_adj_ui(KParams P, AdjAt at, const double* __restrict__ gC,
                          double* __restrict__ lUi, double* __restrict__ lunew, double* __restrict__ lulast,
                          double* __restrict__ lp) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y * blockDim.y + threadIdx.y;
-  if (i >= P.n1 || j >= P.n2) return;
-  const double* __restrict__ pn = slot[0];
+  const int id = blockIdx.x * 64 + threadIdx.x, i = id / P.n2, j = id % P.n2;
+  if (i >= P.n1) return;
+  const double* __restrict__ pn = at.before();
   const int z = zidx(P, i, j);
   double gc[36];
   load_cent(P, gC, z, gc);
@@ -394,10 +429,9 @@ struct harm_adj {
   DevScalars* d_dsN;
   double* seg;                     // K*nto+1 states of one segment
   int nto;
-  double *lp, *lunew, *lulast, *lUi, *ldU, *lemf, *lf1, *lf2, *rowsum;
+  double *lp, *lunew, *lulast, *lUi, *ldU, *lterm, *lf1, *lf2, *rowsum;
   int* d_ns;
   int* d_ctr;                      // step index, first step of the segment
-  const double** d_slot;           // pb and pf of the substage being reversed
   hipGraphExec_t gx[5];            // steps: record dt, impose dt, impose + store, reverse, record + store
   bool gx_ok[5];
   hipGraphExec_t gx8[5];           // the same, ADJ_STEPS_PER_GRAPH steps per graph
@@ -427,10 +461,9 @@ extern "C" int harm_adj_destroy(harm_adj* a) {
     if (a->gx8_ok[k]) (void)hipGraphExecDestroy(a->gx8[k]);
   }
   if (a->d_ctr) (void)hipFree(a->d_ctr);
-  if (a->d_slot) (void)hipFree((void*)a->d_slot);
   if (a->ckpt)
     for (double* pp : *a->ckpt) (void)hipFree(pp);
-  double* bufs[] = {a->d_dts, a->pN, a->seg, a->lp, a->lunew, a->lulast, a->lUi, a->ldU, a->lemf, a->lf1, a->lf2,
+  double* bufs[] = {a->d_dts, a->pN, a->seg, a->lp, a->lunew, a->lulast, a->lUi, a->ldU, a->lterm, a->lf1, a->lf2,
                     a->rowsum};
   for (double* b : bufs) (void)hipFree(b);
   (void)hipFree(a->d_ckds);
@@ -470,16 +503,14 @@ extern "C" int harm_adj_create(harm_ctx* c, int nsteps, int checkpoint_every, ha
   double** lb[] = {&a->lp, &a->lunew, &a->lulast, &a->lUi, &a->ldU};
   for (double** b : lb)
     if (e == hipSuccess && (e = hipMalloc(b, sb)) == hipSuccess) e = hipMemset(*b, 0, sb);
-  if (e == hipSuccess && (e = hipMalloc(&a->lemf, (size_t)c->nz * sizeof(double))) == hipSuccess)
-    e = hipMemset(a->lemf, 0, (size_t)c->nz * sizeof(double));
+  if (e == hipSuccess && (e = hipMalloc(&a->lterm, (size_t)c->nz * sizeof(double))) == hipSuccess)
+    e = hipMemset(a->lterm, 0, (size_t)c->nz * sizeof(double));
   if (e == hipSuccess && (e = hipMalloc(&a->lf1, 2 * sb)) == hipSuccess) e = hipMemset(a->lf1, 0, 2 * sb);
   if (e == hipSuccess && (e = hipMalloc(&a->lf2, 2 * sb)) == hipSuccess) e = hipMemset(a->lf2, 0, 2 * sb);
   if (e == hipSuccess) e = hipMalloc(&a->rowsum, sizeof(double) * c->kp.n1);
   if (e == hipSuccess && (e = hipMalloc(&a->d_ns, sizeof(int))) == hipSuccess) e = hipMemset(a->d_ns, 0, sizeof(int));
   if (e == hipSuccess && (e = hipMalloc(&a->d_ctr, 2 * sizeof(int))) == hipSuccess)
     e = hipMemset(a->d_ctr, 0, 2 * sizeof(int));
-  if (e == hipSuccess && (e = hipMalloc((void**)&a->d_slot, 2 * sizeof(double*))) == hipSuccess)
-    e = hipMemset((void*)a->d_slot, 0, 2 * sizeof(double*));
   if (e != hipSuccess) {
     harm_adj_destroy(a);
     return seterr("harm_adj_create: %s", hipGetErrorString(e));
@@ -488,12 +519,11 @@ extern "C" int harm_adj_create(harm_ctx* c, int nsteps, int checkpoint_every, ha
   return 0;
 }
 
-// one step with the dt of step n imposed (or recorded), eager launches
-// one forward step of step ctr[0] (dt recorded or imposed); with store, the
-// state after every substage goes to the segment store; then ctr[0]++
-static int adj_step(harm_adj* a, int impose, bool store) {
+// forward step ctr[0] + rel (dt recorded or imposed); with store, the state after
+// every substage goes to the segment store
+static int adj_step(harm_adj* a, int rel, int impose, bool store) {
   harm_ctx* c = a->c;
-  hipLaunchKernelGGL(k_adj_dt, dim3(1), dim3(1), 0, c->stream, c->ds, a->d_dts, a->d_ctr, impose);
+  hipLaunchKernelGGL(k_adj_dt, dim3(1), dim3(1), 0, c->stream, c->ds, a->d_dts, a->d_ctr, rel, impose);
   double CUf[4][3], Cunew[4][3];
   int pii[4], pbb[4], pff[4], nto;
   rk_setup(c->prm.timeorder, &nto, CUf, Cunew, pii, pbb, pff);
@@ -506,43 +536,37 @@ static int adj_step(harm_adj* a, int impose, bool store) {
                             (one_launch(c, pbb[to], pff[to], bnd) ? KB_TAKE : 0)))
       return 1;
     if (store)
-      hipLaunchKernelGGL(k_adj_store, dim3(512), dim3(256), 0, c->stream, c->arr[pff[to]], a->seg, a->d_ctr, nto, to,
-                         nz8);
+      hipLaunchKernelGGL(k_adj_store, dim3(512), dim3(256), 0, c->stream, c->arr[pff[to]], a->seg,
+                         AdjAt{a->seg, a->d_ctr, nto, to + 1, rel, nz8});
   }
-  hipLaunchKernelGGL(k_adj_next, dim3(1), dim3(1), 0, c->stream, a->d_ctr, 1);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
 static int adj_boundT(harm_adj* a);
 
-// the reverse of step ctr[0] (its substage states in the segment store),
-// then ctr[0]--
 // the reverse kernels specialised for the Orszag-Tang scheme (MC with HLL or
 // LAXF), or the general ones
 template <int LIMC, int FMC>
-static void adj_launch_substage(harm_adj* a, const AdjRK& R, bool first) {
+static void adj_launch_substage(harm_adj* a, const AdjRK& R, const AdjAt& at) {
   harm_ctx* c = a->c;
-  const dim3 b(64, 4);
-  const dim3 gz = grid2(c->kp.n2, c->kp.n1, b);
-  const dim3 gc2 = grid2(c->kp.n2 + 1, c->kp.n1 + 1, b);
-  const dim3 gf((c->kp.n2 + 2 + 63) / 64, (c->kp.n1 + 2 + 3) / 4, 2);
-  const dim3 gall = grid2(c->kp.n2 + 2 * NG, c->kp.n1 + 2 * NG, b);
-  hipLaunchKernelGGL((k_adj_zone<LIMC, FMC>), gz, b, 0, c->stream, c->kp, R, a->d_slot, a->d_dts, a->d_ctr, c->gC,
-                     a->lp, a->lunew, a->lulast, a->lUi, a->ldU, a->d_ns);
-  if (c->prm.fluxb == HARM_FLUXCTTOTH)
-    hipLaunchKernelGGL(k_adj_emf, gc2, b, 0, c->stream, c->kp, a->ldU, a->lemf);
-  hipLaunchKernelGGL((k_adj_face<LIMC, FMC>), gf, b, 0, c->stream, c->kp, a->d_slot, c->gF, c->gC, a->ldU, a->lemf,
-                     a->lf1, a->lf2, a->d_ns);
-  hipLaunchKernelGGL((k_adj_gather<LIMC, FMC>), gall, b, 0, c->stream, c->kp, a->d_slot, c->gC, c->gConn, a->ldU,
-                     a->lf1, a->lf2, a->lp);
-  if (first)
-    hipLaunchKernelGGL(k_adj_ui, gz, b, 0, c->stream, c->kp, a->d_slot, c->gC, a->lUi, a->lunew, a->lulast, a->lp);
+  const int n1 = c->kp.n1, n2 = c->kp.n2;
+  auto line = [](int zones) { return (unsigned)((zones + 63) / 64); };
+  hipLaunchKernelGGL((k_adj_zone<LIMC, FMC>), dim3(line(n1 * n2)), dim3(64), 0, c->stream, c->kp, R, at, a->d_dts,
+                     c->gC, a->lp, a->lunew, a->lulast, a->lUi, a->ldU, a->d_ns);
+  const int faces = std::max((n1 + 1) * (n2 + 2), (n1 + 2) * (n2 + 1));
+  hipLaunchKernelGGL((k_adj_face<LIMC, FMC>), dim3(line(faces), 2), dim3(64), 0, c->stream, c->kp, at, c->gF, c->gC,
+                     a->ldU, a->lf1, a->lf2, a->d_ns);
+  hipLaunchKernelGGL((k_adj_gather<LIMC, FMC>), dim3(line(c->kp.nz)), dim3(64, 2), 0, c->stream, c->kp, at, c->gC,
+                     c->gConn, a->ldU, a->lf1, a->lf2, a->lp);
+  if (at.s == 0)
+    hipLaunchKernelGGL(k_adj_ui, dim3(line(n1 * n2)), dim3(64), 0, c->stream, c->kp, at, c->gC, a->lUi, a->lunew,
+                       a->lulast, a->lp);
 }
 
-static int adj_reverse_step(harm_adj* a) {
+// the reverse of step ctr[0] + rel (its substage states in the segment store)
+static int adj_reverse_step(harm_adj* a, int rel) {
   harm_ctx* c = a->c;
-  const size_t nz8 = (size_t)c->nz * 8;
   double CUf[4][3], Cunew[4][3];
   int pii[4], pbb[4], pff[4], nto;
   rk_setup(c->prm.timeorder, &nto, CUf, Cunew, pii, pbb, pff);
@@ -552,16 +576,14 @@ static int adj_reverse_step(harm_adj* a) {
     R.b0 = Cunew[s][0]; R.b1 = Cunew[s][1]; R.b2 = Cunew[s][2];
     R.dt = 0.;  // read from the dt sequence on the device
     R.last = (s == nto - 1);
-    if (adj_boundT(a)) return 1;
-    hipLaunchKernelGGL(k_adj_slot, dim3(1), dim3(1), 0, c->stream, a->seg, a->d_ctr, nto, s, nz8, a->d_slot);
+    const AdjAt at{a->seg, a->d_ctr, nto, s, rel, (size_t)c->nz * 8};
     if (c->kp.lim == HARM_MC && c->kp.fluxmethod == HARM_HLLFLUX)
-      adj_launch_substage<HARM_MC, HARM_HLLFLUX>(a, R, s == 0);
+      adj_launch_substage<HARM_MC, HARM_HLLFLUX>(a, R, at);
     else if (c->kp.lim == HARM_MC && c->kp.fluxmethod == HARM_LAXFFLUX)
-      adj_launch_substage<HARM_MC, HARM_LAXFFLUX>(a, R, s == 0);
+      adj_launch_substage<HARM_MC, HARM_LAXFFLUX>(a, R, at);
     else
-      adj_launch_substage<-1, -1>(a, R, s == 0);
+      adj_launch_substage<-1, -1>(a, R, at);
   }
-  hipLaunchKernelGGL(k_adj_next, dim3(1), dim3(1), 0, c->stream, a->d_ctr, -1);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -569,8 +591,7 @@ static int adj_reverse_step(harm_adj* a) {
 // graph k: 0 forward step recording dt, 1 forward step imposing dt,
 // 2 recompute step (imposed dt, states stored), 3 reverse step, 4 forward
 // step recording dt with its states stored
-// (each step advances the device step counter itself, so a graph of several
-// steps is that many steps)
+// (its last launch advances the device step counter by its steps)
 constexpr int ADJ_STEPS_PER_GRAPH = 8;
 static int adj_graph(harm_adj* a, int k, bool multi = false) {
   hipGraphExec_t* ex = multi ? &a->gx8[k] : &a->gx[k];
@@ -580,8 +601,10 @@ static int adj_graph(harm_adj* a, int k, bool multi = false) {
   hipGraph_t g;
   HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   int rc = 0;
-  for (int s = 0; s < (multi ? ADJ_STEPS_PER_GRAPH : 1) && !rc; s++)
-    rc = (k == 3) ? adj_reverse_step(a) : adj_step(a, (k == 0 || k == 4) ? 0 : 1, k == 2 || k == 4);
+  const int steps = multi ? ADJ_STEPS_PER_GRAPH : 1;
+  for (int s = 0; s < steps && !rc; s++)
+    rc = (k == 3) ? adj_reverse_step(a, -s) : adj_step(a, s, (k == 0 || k == 4) ? 0 : 1, k == 2 || k == 4);
+  if (!rc) hipLaunchKernelGGL(k_adj_next, dim3(1), dim3(1), 0, c->stream, a->d_ctr, (k == 3) ? -steps : steps);
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   if (rc) {
     if (e == hipSuccess) (void)hipGraphDestroy(g);
@@ -665,21 +688,11 @@ extern "C" int harm_adj_seed_magnetic_energy(harm_adj* a, double* J) {
   if (!a->forward_done) return seterr("adjoint: run harm_adj_forward first");
   harm_ctx* c = a->c;
   const dim3 b(64, 4);
-  hipLaunchKernelGGL(k_adj_seed_bsq, grid2(c->kp.n2 + NG, c->kp.n1 + NG, b), b, 0, c->stream, c->kp, a->pN, c->gC,
-                     a->lp, a->rowsum);
+  hipLaunchKernelGGL(k_adj_seed_bsq, grid2(c->N2M, c->N1M, b), b, 0, c->stream, c->kp, a->pN, c->gC, a->lp, a->lterm);
+  hipLaunchKernelGGL(k_adj_rowsum, dim3(c->kp.n1), dim3(64), 0, c->stream, c->kp, a->lterm, a->rowsum);
   HIPCHK(hipGetLastError());
-  // ghost rows/columns below 0 are not covered by that grid: clear them
   std::vector<double> rs(c->kp.n1);
   HIPCHK(hipStreamSynchronize(c->stream));
-  {
-    std::vector<double> h((size_t)c->nz * 8);
-    HIPCHK(hipMemcpy(h.data(), a->lp, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int i = 0; i < c->N1M; i++)
-      for (int j = 0; j < c->N2M; j++)
-        if (i < NG || j < NG)
-          for (int k = 0; k < 8; k++) h[((size_t)i * c->N2M + j) * 8 + k] = 0.;
-    HIPCHK(hipMemcpy(a->lp, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
-  }
   HIPCHK(hipMemcpy(rs.data(), a->rowsum, sizeof(double) * c->kp.n1, hipMemcpyDeviceToHost));
   double s = 0.;
   for (int i = 0; i < c->kp.n1; i++) s += rs[i];
