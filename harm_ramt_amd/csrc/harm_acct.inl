@@ -45,6 +45,7 @@ struct AcctState {
   double* lumvsr;   // [n1]
   double* scratch;  // per-term buffer of the first phase
   double* out;      // 4 doubles: dump-time results
+  double* host;     // pinned: acc, frdot and lumvsr on their way to the caller
   int* faces;       // (i, j) of each boundary face, boundaries in (region, dir) order
   size_t scratch_n;
   // fixup events of a substage (slots of acct_base) and their compaction
@@ -1053,6 +1054,7 @@ static int acct_alloc(harm_ctx* c) {
   if (e == hipSuccess) e = hipMalloc(&a->lumvsr, (size_t)n1 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&a->scratch, a->scratch_n * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&a->out, 8 * sizeof(double));
+  if (e == hipSuccess) e = hipHostMalloc((void**)&a->host, (ACC_D + (size_t)n1 * 9) * sizeof(double), hipHostMallocDefault);
   if (e == hipSuccess) e = hipMalloc(&a->faces, (size_t)ACC_NREG * 2 * (n1 + n2 + 2) * 2 * sizeof(int));
   a->nslots = acct_base(n1, n2, 4);
   a->nblocks = (a->nslots + 255) / 256;
@@ -1083,6 +1085,7 @@ static void acct_free(harm_ctx* c) {
                      a->flag, a->val,   a->list,   a->cval,    a->cnt, a->sterm, a->total, a->part};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  if (a->host) (void)hipHostFree(a->host);
   if (a->fork) (void)hipEventDestroy(a->fork);
   if (a->join) (void)hipEventDestroy(a->join);
   if (a->side) (void)hipStreamDestroy(a->side);
@@ -1263,15 +1266,17 @@ extern "C" int harm_acct_read(harm_ctx* c, harm_ener_region* regions, double* je
   if (!c) return seterr("null ctx");
   if (!c->acct) return seterr("accounting was never set up (harm_acct_setup)");
   AcctState* a = c->acct;
-  std::vector<double> h(ACC_D);
-  HIPCHK(hipMemcpyAsync(h.data(), a->acc, ACC_D * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (frdot)
-    HIPCHK(hipMemcpyAsync(frdot, a->frdot, (size_t)c->prm.n1 * 8 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (lumvsr)
-    HIPCHK(hipMemcpyAsync(lumvsr, a->lumvsr, (size_t)c->prm.n1 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  std::lock_guard<std::mutex> lk(c->stage->mu);
+  const size_t n1 = (size_t)c->prm.n1;
+  double *h = a->host, *hf = h + ACC_D, *hl = hf + n1 * 8;
+  HIPCHK(hipMemcpyAsync(h, a->acc, ACC_D * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if (frdot) HIPCHK(hipMemcpyAsync(hf, a->frdot, n1 * 8 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if (lumvsr) HIPCHK(hipMemcpyAsync(hl, a->lumvsr, n1 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
-  if (regions) memcpy(regions, h.data(), sizeof(harm_ener_region) * ACC_NREG);
-  if (jet2) memcpy(jet2, h.data() + OFF_JET2, 4 * ACC_NFL * 8 * sizeof(double));
+  if (regions) memcpy(regions, h, sizeof(harm_ener_region) * ACC_NREG);
+  if (jet2) memcpy(jet2, h + OFF_JET2, 4 * ACC_NFL * 8 * sizeof(double));
+  if (frdot) memcpy(frdot, hf, n1 * 8 * sizeof(double));
+  if (lumvsr) memcpy(lumvsr, hl, n1 * sizeof(double));
   return 0;
 }
 

@@ -33,6 +33,7 @@
 #include <stdlib.h>
 #include <vector>
 #include <mutex>
+#include <new>
 #include <algorithm>
 #include <stddef.h>
 #include <type_traits>
@@ -2924,8 +2925,45 @@ struct AcctState;  // conservation accounting (harm_acct.inl)
 struct CurState;   // the current J, F (harm_diag.inl)
 }
 
+// What a context's calls hand to the host and take from it, by way of pinned
+// memory: a copy to or from pageable memory waits for the stream, is staged by the
+// runtime and waits again (a step and its get_time() take 10 us longer in the
+// pageable form).  One call at a time uses it.
+constexpr int STAGE_ZONES = 1 << 16;  // zones of an inversion that are staged (9 MB); more take allocations of their own
+struct HostStage {
+  std::mutex mu;
+  double* few = nullptr;   // [8]: t, dt, tf
+  char* host = nullptr;    // zones * ZONE bytes, and the device's counterpart
+  char* dev = nullptr;
+  int zones = 0;
+  static constexpr size_t ZONE = 17 * sizeof(double) + sizeof(int);  // U, (i, j), primitives, flag
+  hipError_t init() { return hipHostMalloc((void**)&few, 8 * sizeof(double), hipHostMallocDefault); }
+  hipError_t room(int n) {  // n <= STAGE_ZONES
+    if (n <= zones) return hipSuccess;
+    int want = 256;
+    while (want < n) want *= 2;
+    drop();
+    hipError_t e = hipHostMalloc((void**)&host, want * ZONE, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc((void**)&dev, want * ZONE);
+    if (e == hipSuccess) zones = want;
+    else drop();
+    return e;
+  }
+  void drop() {
+    if (host) (void)hipHostFree(host);
+    if (dev) (void)hipFree(dev);
+    host = dev = nullptr;
+    zones = 0;
+  }
+  ~HostStage() {
+    drop();
+    if (few) (void)hipHostFree(few);
+  }
+};
+
 struct harm_ctx {
   harm_params prm;
+  HostStage* stage;
   KParams kp;
   int N1M, N2M, nz;
   double* arr[HARM_NARRAYS];
@@ -3092,6 +3130,7 @@ extern "C" int harm_create(const harm_params* prm, harm_ctx** out) {
   if (e == hipSuccess) e = hipMalloc(&c->gConn, nz * NCONN * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&c->ds, sizeof(DevScalars));
   if (e == hipSuccess) e = hipStreamCreate(&c->own_stream);
+  if (e == hipSuccess) e = (c->stage = new (std::nothrow) HostStage()) ? c->stage->init() : hipErrorOutOfMemory;
   if (e == hipSuccess) e = hipGetDevice(&c->device);
   if (e != hipSuccess) {
     seterr("harm_create: %s", hipGetErrorString(e));
@@ -3199,6 +3238,7 @@ extern "C" int harm_destroy(harm_ctx* c) {
   acct_free(c);
   cur_free(c);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
+  delete c->stage;
   free(c);
   return 0;
 }
@@ -3364,8 +3404,9 @@ extern "C" int harm_set_time(harm_ctx* c, double t, double dt, double tf) {
 
 extern "C" int harm_get_time(harm_ctx* c, double* t, double* dt) {
   if (!c) return seterr("null ctx");
-  double v[3];
-  HIPCHK(hipMemcpyAsync(v, &c->ds->t, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  std::lock_guard<std::mutex> lk(c->stage->mu);
+  const double* v = c->stage->few;
+  HIPCHK(hipMemcpyAsync(c->stage->few, &c->ds->t, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   if (t) *t = v[0];
   if (dt) *dt = v[1];
@@ -4001,6 +4042,38 @@ extern "C" int harm_step_n(harm_ctx* c, int nsteps) {
   return 0;
 }
 
+// up to STAGE_ZONES zones by way of the context's staging: two copies in (the
+// second half is laid out while the first is on its way), one out, one wait.
+// 4,096 zones: 82 us; with four allocations and five pageable copies 119.
+static int utoprimgen_staged(harm_ctx* c, int n, const int* zone, const double* U, double* pr, int* pflag) {
+  HostStage& st = *c->stage;
+  std::lock_guard<std::mutex> lk(st.mu);
+  hipError_t e = st.room(n);
+  const size_t m = (size_t)n, zo = m * 64, po = zo + m * 8, fo = po + m * 64;  // U, zones, primitives, flags
+  if (e == hipSuccess) {
+    memcpy(st.host, U, m * 64);
+    memcpy(st.host + zo, zone, m * 8);
+    e = hipMemcpyAsync(st.dev, st.host, po, hipMemcpyHostToDevice, c->stream);
+  }
+  if (e == hipSuccess) {
+    memcpy(st.host + po, pr, m * 64);
+    e = hipMemcpyAsync(st.dev + po, st.host + po, m * 64, hipMemcpyHostToDevice, c->stream);
+  }
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_utoprim_batch, dim3((n + 63) / 64), dim3(64), 0, c->stream, c->kp, n,
+                       (const int*)(st.dev + zo), (const double*)st.dev, (double*)(st.dev + po), (int*)(st.dev + fo),
+                       c->gC);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(st.host + po, st.dev + po, m * 68, hipMemcpyDeviceToHost, c->stream);
+  const hipError_t w = hipStreamSynchronize(c->stream);  // also where a step failed: the staging is free again
+  if (e == hipSuccess) e = w;
+  if (e != hipSuccess) return seterr("harm_utoprimgen: %s", hipGetErrorString(e));
+  memcpy(pr, st.host + po, m * 64);
+  memcpy(pflag, st.host + fo, m * 4);
+  return 0;
+}
+
 extern "C" int harm_utoprimgen(harm_ctx* c, int n, const int* zone, const double* U, double* pr, int* pflag) {
   if (need_geom(c)) return 1;
   if (n <= 0) return 0;
@@ -4010,6 +4083,7 @@ extern "C" int harm_utoprimgen(harm_ctx* c, int n, const int* zone, const double
     if (i < -NG || i >= c->prm.n1 + NG || j < -NG || j >= c->prm.n2 + NG)
       return seterr("zone %d (%d,%d) out of range", t, i, j);
   }
+  if (n <= STAGE_ZONES) return utoprimgen_staged(c, n, zone, U, pr, pflag);
   int* dz;
   double *dU, *dp;
   int* dfl;
