@@ -1184,49 +1184,22 @@ __device__ __forceinline__ void load_cent(const KParams& P, const double* __rest
       [&](int m) { return v[m]; }, gc);
 }
 
-// flux2dUavg (advance.c:204-265): each direction's flux difference from the
-// zone's lower (a) and upper (b) face fluxes, with the flux-CT B fluxes formed
-// from the corner EMFs e (step_ch.c:1223-1234, 1405-1412)
-__device__ __forceinline__ void flux_diff(const KParams& P, double* f1a, double* f1b, double* f2a, double* f2b,
-                                          bool ct, const double (&e)[4], double* d1, double* d2) {
-  if (ct) {  // e00, e01, e10, e11
-    f1a[B1] = 0.;
-    f1a[B2] = 0.5 * (e[0] + e[1]);
-    f1b[B1] = 0.;
-    f1b[B2] = 0.5 * (e[2] + e[3]);
-    f2a[B1] = -0.5 * (e[0] + e[2]);
-    f2a[B2] = 0.;
-    f2b[B1] = -0.5 * (e[1] + e[3]);
-    f2b[B2] = 0.;
-  }
-  const double idx1 = 1.0 / P.dx1, idx2 = 1.0 / P.dx2;
-#pragma unroll
-  for (int k = 0; k < NPR; k++) {
-    d1[k] = (-(f1b[k] - f1a[k]) * idx1);
-    d2[k] = (-(f2b[k] - f2a[k]) * idx2);
-  }
-}
-
-template <int GEO = GEO_ANY>
-__device__ __forceinline__ void flux_div(const KParams& P, const double* __restrict__ F1,
-                                         const double* __restrict__ F2, const double* __restrict__ q1,
-                                         const double* __restrict__ q2, const double* __restrict__ gC, int i, int j,
-                                         double* d1, double* d2) {
-  const int z = zidx(P, i, j);
-  double f1a[NPR], f1b[NPR], f2a[NPR], f2b[NPR];
-  load8(F1, z, f1a);
-  load8(F1, zidx(P, i + 1, j), f1b);
-  load8(F2, z, f2a);
-  load8(F2, zidx(P, i, j + 1), f2b);
-  double e[4] = {0., 0., 0., 0.};
-  const bool ct = P.fluxb == HARM_FLUXCTTOTH;
+// flux2dUavg (advance.c:204-265): a direction's flux difference from the zone's
+// lower (a) and upper (b) face fluxes, with the flux-CT B fluxes formed from the
+// corner EMFs e (step_ch.c:1223-1234, 1405-1412): e00, e01, e10, e11
+template <int DIR>
+__device__ __forceinline__ void flux_diff(const KParams& P, double* a, double* b, bool ct, const double (&e)[4],
+                                          double* d) {
   if (ct) {
-    e[0] = emf_at<GEO>(P, q1, q2, gC, i, j);
-    e[1] = emf_at<GEO>(P, q1, q2, gC, i, j + 1);
-    e[2] = emf_at<GEO>(P, q1, q2, gC, i + 1, j);
-    e[3] = emf_at<GEO>(P, q1, q2, gC, i + 1, j + 1);
+    constexpr int k = (DIR == 1) ? B2 : B1;
+    a[B1 + DIR - 1] = 0.;
+    b[B1 + DIR - 1] = 0.;
+    a[k] = (DIR == 1) ? 0.5 * (e[0] + e[1]) : -0.5 * (e[0] + e[2]);
+    b[k] = (DIR == 1) ? 0.5 * (e[2] + e[3]) : -0.5 * (e[1] + e[3]);
   }
-  flux_diff(P, f1a, f1b, f2a, f2b, ct, e, d1, d2);
+  const double idx = 1.0 / ((DIR == 1) ? P.dx1 : P.dx2);
+#pragma unroll
+  for (int k = 0; k < NPR; k++) d[k] = (-(b[k] - a[k]) * idx);
 }
 
 // Makes index j one that the compiler knows only once the values v are formed:
@@ -1235,6 +1208,43 @@ template <int N>
 __device__ __forceinline__ void after(int& j, double (&v)[N]) {
 #pragma unroll
   for (int k = 0; k < N; k++) asm volatile("" : "+v"(j), "+v"(v[k]));
+}
+
+// both directions' flux differences of zone (i, j).  SPLIT: the EMFs, then each
+// direction, are formed before the next is loaded (j: known after them)
+template <int GEO = GEO_ANY, bool SPLIT = false>
+__device__ __forceinline__ void flux_div(const KParams& P, const double* __restrict__ F1,
+                                         const double* __restrict__ F2, const double* __restrict__ q1,
+                                         const double* __restrict__ q2, const double* __restrict__ gC, int i, int& j,
+                                         double (&d1)[NPR], double (&d2)[NPR]) {
+  double f1a[NPR], f1b[NPR], f2a[NPR], f2b[NPR], e[4] = {0., 0., 0., 0.};
+  auto load = [&](const double* __restrict__ F, int up, double* a, double* b) {
+    const int z = zidx(P, i, j);
+    load8(F, z, a);
+    load8(F, z + up, b);
+  };
+  if (!SPLIT) {
+    load(F1, P.N2M, f1a, f1b);
+    load(F2, 1, f2a, f2b);
+  }
+  const bool ct = P.fluxb == HARM_FLUXCTTOTH;
+  if (ct) {
+    e[0] = emf_at<GEO>(P, q1, q2, gC, i, j);
+    e[1] = emf_at<GEO>(P, q1, q2, gC, i, j + 1);
+    e[2] = emf_at<GEO>(P, q1, q2, gC, i + 1, j);
+    e[3] = emf_at<GEO>(P, q1, q2, gC, i + 1, j + 1);
+  }
+  if (SPLIT) {
+    after(j, e);
+    load(F1, P.N2M, f1a, f1b);
+  }
+  flux_diff<1>(P, f1a, f1b, ct, e, d1);
+  if (SPLIT) {
+    after(j, d1);
+    load(F2, 1, f2a, f2b);
+  }
+  flux_diff<2>(P, f2a, f2b, ct, e, d2);
+  if (SPLIT) after(j, d2);
 }
 
 // RK combination of one zone (dUtoU, advance.c:273-286)
@@ -1403,18 +1413,23 @@ static_assert(NG == 3, "an edge block has NG rows besides the edge row");
 // operations in 40,000 cycles): the compiler, left alone, loads all of a zone's
 // values at the top and holds 298 to 326 registers, which leaves one.  So what
 // the flux difference and the RK combination read is loaded once U(pi) and the
-// source term are formed (after()): 174 to 239 registers, nothing spilled.  us a
+// source term are formed (after()): 174 to 247 registers, nothing spilled.  us a
 // launch, before -> after: torus 512x512 79.4 -> 63.6, monopole 512x512 60.1 ->
-// 50.4, twelve tori of 88 to 256 zones a side 154.8 -> 111.9, Orszag-Tang 256x256
-// 22.5 -> 21.3; torus 256x256, one wavefront a SIMD in all, 23.2 -> 23.5 (without
-// the fill 20.2 -> 18.8).  Three wavefronts (loads in four groups, 168 registers)
-// cost the twelve tori 146.8 and gain nothing elsewhere.
+// 50.4, twelve tori of 88 to 256 zones a side 154.8 -> 114, Orszag-Tang 256x256
+// 22.5 -> 21.3; torus 256x256, one wavefront a SIMD in all, 23.2 -> 23.4.  Three
+// wavefronts (168 registers) cost the twelve tori 147 and gain nothing elsewhere.
+// SPLIT: these loads in four groups, where the geometry is read from memory and
+// the fill is done here: torus 256x256 23.4 -> 22.2, 512x512 63.6 -> 61.7, monopole
+// 50.6 -> 50.0 (a uniform geometry 21.2 -> 22.5, without the fill 56.7 -> 57.5, the
+// batch's launch 112 -> 129: not there).  What is left of a 256x256 launch is
+// every wavefront's first loads at once (24,000 of 42,000 cycles until the source
+// term is formed), then the Newton iterations (10,000).
 //
 // BND: the first bound_prim() of the substage done here (ENO 0 only): each
 // zone near an edge writes its ghost images after its inversion; an outflow
 // edge row hands its values to the other rows of its workgroup (LDS, one
 // barrier), which write the NG x1 ghost columns, one column per row
-template <int ENO, int BND = 0, int GEO = GEO_ANY>
+template <int ENO, int BND = 0, int GEO = GEO_ANY, bool SPLIT = false>
 __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* __restrict__ pi,
                                                 const double* __restrict__ pb, double* __restrict__ pf,
                                                 double* __restrict__ ulast, double* __restrict__ unew,
@@ -1456,19 +1471,19 @@ __device__ __forceinline__ void update_body(KParams P, RKCoef C, const double* _
       after(jf, dUg);
       after(jf, Ui);
     }
-    const int zf = zidx(P, i, jf);
     double d1[NPR], d2[NPR];
     if constexpr (ENO == 2) {
       eno_cvt_zone<ENO_A2C, 1>(P, eA, i, j, d1);
       eno_cvt_zone<ENO_A2C, 2>(P, eB, i, j, d2);
     } else {
-      flux_div<GEO>(P, F1, F2, q1, q2, gC, i, jf, d1, d2);
+      flux_div<GEO, SPLIT>(P, F1, F2, q1, q2, gC, i, jf, d1, d2);
     }
     double ul[NPR], un[NPR], Uf[NPR];
     if (C.timeorder == 0) {
 #pragma unroll
       for (int k = 0; k < NPR; k++) ul[k] = un[k] = 0.0;
     } else {
+      const int zf = zidx(P, i, jf);
       load8(ulast, zf, ul);
       load8(unew, zf, un);
     }
@@ -1549,7 +1564,7 @@ __global__ __launch_bounds__(256, ENO == 0 ? 2 : 1) void k_update(KParams P, RKC
                                                 const double* __restrict__ gC, const double* __restrict__ gConn,
                                                 int* __restrict__ pflag, int* __restrict__ faillist,
                                                 DevScalars* __restrict__ ds, double* eA, const double* eB) {
-  update_body<ENO, BND, GEO>(specialize<-1, EOMC, -1>(P), C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gC, gConn, pflag,
+  update_body<ENO, BND, GEO, BND && GEO != GEO_UNIFORM>(specialize<-1, EOMC, -1>(P), C, pi, pb, pf, ulast, unew, F1, F2, q1, q2, gC, gConn, pflag,
                    faillist, ds, eA, eB, dim3(blockIdx.x, blockIdx.y, blockIdx.z),
                    dim3(gridDim.x, gridDim.y, gridDim.z));
 }
@@ -1596,7 +1611,8 @@ __global__ __launch_bounds__(256) void k_eno_fluxdiv(KParams P, const double* __
   const int i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i >= P.n1 || j >= P.n2) return;
   double d1[NPR], d2[NPR];
-  flux_div(P, F1, F2, q1, q2, gC, i, j, d1, d2);
+  int jf = j;
+  flux_div(P, F1, F2, q1, q2, gC, i, jf, d1, d2);
   const int z = zidx(P, i, j);
   store8(d1out, z, d1);
   store8(d2out, z, d2);

@@ -239,7 +239,8 @@ __device__ __forceinline__ void substage_body(
       e[2] = emf(1, 0);
       e[3] = emf(1, 1);
     }
-    flux_diff(P, f1a, f1b, f2a, f2b, ct, e, d1, d2);
+    flux_diff<1>(P, f1a, f1b, ct, e, d1);
+    flux_diff<2>(P, f2a, f2b, ct, e, d2);
   }
   __syncthreads();
   if (upd) {
