@@ -38,7 +38,9 @@ HBM_PEAK_GBS = 8000.0
 #              240) + connection (Gamma^k_{lj}, l <= j: 40 doubles, 320)
 #              + F1, F2 (128) + q1, q2 (16) + ulast, unew read (128)
 #              + pf, ulast, unew written (192) + pflag (4)          = 1156 B
-BYTES_PER_UNIT = {"flux": 264, "update": 1156}
+# On a Kerr-Schild metric 5 of a face's 16 geometry numbers and 13 of a zone's
+# 70 hold one value over all zones and are read once a wavefront: 224, 1052.
+BYTES_PER_UNIT = {"flux": 224, "update": 1052}
 
 
 def units_per_launch(stage, n1, n2):

@@ -5,15 +5,17 @@
 //   flux       fluxcalc() for both directions in one launch: reconstruction,
 //              limit_gamma, states, fluxes, vchar, HLL/LAXF, fix_flux edge
 //              rules, wavefront-reduced Courant minimum      (step_ch.c:741)
-//              k_flux_single (thread per face) or k_flux (lane pair per face)
+//              k_flux_shared (thread per zone and direction), k_flux_single
+//              (thread per face) or k_flux (lane pair per face)
 //   k_update   advance() per zone: U(pi), source(pb), flux divergence with
 //              the flux-CT fluxes formed from the corner EMFs (step_ch.c:1159)
 //              inline, RK combination, Newton con-to-prim, fixup1zone, and
 //              the list of zones whose inversion failed      (advance.c:46)
 //   boundary   bound_prim(), post_fixup() on the failed list, bound_prim(),
 //              and after the last substage the t,dt update (step_ch.c:85-183):
-//              k_boundary (one workgroup) or k_bx1/k_bx2/k_fixlist/k_fixapply
-// All variants of a stage give bit-identical results; the first step times
+//              in the update and k_fixbound, k_boundary (one workgroup) or
+//              k_bx1/k_bx2/k_fixlist/k_fixapply
+// On small grids the flux and the update are one launch (k_substage).  All variants of a stage give bit-identical results; the first step times
 // them and keeps the fastest.  A step never synchronises with the host, and
 // a whole step is captured once into a HIP graph and replayed.
 //
