@@ -4066,13 +4066,14 @@ extern "C" int harm_step_n(harm_ctx* c, int nsteps) {
 static int utoprimgen_staged(harm_ctx* c, int n, const int* zone, const double* U, double* pr, int* pflag) {
   HostStage& st = *c->stage;
   std::lock_guard<std::mutex> lk(st.mu);
-  hipError_t e = st.room(n);
-  const size_t m = (size_t)n, zo = m * 64, po = zo + m * 8, fo = po + m * 64;  // U, zones, primitives, flags
-  if (e == hipSuccess) {
-    memcpy(st.host, U, m * 64);
-    memcpy(st.host + zo, zone, m * 8);
-    e = hipMemcpyAsync(st.dev, st.host, po, hipMemcpyHostToDevice, c->stream);
+  if (st.room(n) != hipSuccess) {  // no room for it: the call allocates for itself
+    (void)hipGetLastError();
+    return -1;
   }
+  const size_t m = (size_t)n, zo = m * 64, po = zo + m * 8, fo = po + m * 64;  // U, zones, primitives, flags
+  memcpy(st.host, U, m * 64);
+  memcpy(st.host + zo, zone, m * 8);
+  hipError_t e = hipMemcpyAsync(st.dev, st.host, po, hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) {
     memcpy(st.host + po, pr, m * 64);
     e = hipMemcpyAsync(st.dev + po, st.host + po, m * 64, hipMemcpyHostToDevice, c->stream);
@@ -4101,7 +4102,10 @@ extern "C" int harm_utoprimgen(harm_ctx* c, int n, const int* zone, const double
     if (i < -NG || i >= c->prm.n1 + NG || j < -NG || j >= c->prm.n2 + NG)
       return seterr("zone %d (%d,%d) out of range", t, i, j);
   }
-  if (n <= STAGE_ZONES) return utoprimgen_staged(c, n, zone, U, pr, pflag);
+  if (n <= STAGE_ZONES) {
+    const int rc = utoprimgen_staged(c, n, zone, U, pr, pflag);
+    if (rc >= 0) return rc;
+  }
   int* dz;
   double *dU, *dp;
   int* dfl;
